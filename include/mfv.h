@@ -730,6 +730,9 @@ typedef struct mfv_ell_batch {
 #define MFV_KS_IT 14
 #define MFV_KS_OUTER 15
 #define MFV_KS_ITTOT 16
+#define MFV_KS_RHO_OLD 17 /* this and the next two: mfv_krylov_fused_tick only */
+#define MFV_KS_STOP_V 18
+#define MFV_KS_STOP_T 19
 #define MFV_KS_NSCAL 24
 
 typedef struct mfv_krylov_work {
@@ -754,6 +757,37 @@ int mfv_krylov_tick(const mfv_ell_batch *e, const mfv_krylov_work *w, int n_iter
  * reference: it lets a serving loop advance all solves with one launch. */
 int mfv_krylov_graph(const mfv_ell_batch *e, const mfv_krylov_work *w, int n_iter, int grid_slices,
                      int grid_inst, void **graph_out);
+
+/* Work arrays of the two-launch BiCGStab iteration (mfv_krylov_fused_tick). u holds
+ * (s, t, p, v) and w (r, v) of a row as one record each, so that a matrix slot costs one record
+ * gather. Partial sums are kept per chunk: pa[S], pb[5][S], pr[3][S], the
+ * chunk c of an instance at its first slice + c. chunks[k] = (instance, the instance's first
+ * slice, c | chunk count << 16, the instance's slices): chunk c covers the slices
+ * [c span, (c + 1) span) of its instance, span = MFV_KRYLOV_SPAN(slices); n_chunks[0] entries,
+ * every live instance's chunks once. */
+typedef struct mfv_krylov_fused {
+    double *x, *b;           /* [64 S] FP64 solution and right-hand side */
+    float *d, *rh, *dinv, *p; /* [64 S] FP32 inner-solve vectors */
+    float *u, *w;            /* [64 S][4] and [64 S][2], 16-byte aligned */
+    double *pa, *pb, *pr;    /* [S], [5][S], [3][S] */
+    double *scal;            /* [I][MFV_KS_NSCAL] */
+    int32_t *status;         /* [I] */
+    const int32_t *chunks;   /* [S][4], 16-byte aligned */
+    const int32_t *n_chunks; /* device scalar */
+} mfv_krylov_fused;
+
+/* Slices per chunk of an instance of ns slices: four (one per wave of a block), more where an
+ * instance would have over MFV_KRYLOV_MAX_CHUNKS chunks. */
+#define MFV_KRYLOV_MAX_CHUNKS 512
+#define MFV_KRYLOV_SPAN(ns) (4 * (((ns) + 4 * MFV_KRYLOV_MAX_CHUNKS - 1) / (4 * MFV_KRYLOV_MAX_CHUNKS)))
+
+/* mfv_krylov_tick and mfv_krylov_graph with two launches per BiCGStab iteration instead of
+ * eight; the same states, scalars and stopping tests. grid_chunks: blocks of the per-chunk
+ * kernels, grid_inst: of the per-instance kernel. */
+int mfv_krylov_fused_tick(const mfv_ell_batch *e, const mfv_krylov_fused *w, int n_iter, int grid_chunks,
+                          int grid_inst, void *stream);
+int mfv_krylov_fused_graph(const mfv_ell_batch *e, const mfv_krylov_fused *w, int n_iter, int grid_chunks,
+                           int grid_inst, void **graph_out);
 
 /* 16-bit columns for the slices [slice0, slice0 + nslices) of an assembled ELL batch (no
  * counterpart in the reference: a storage form of the matrix of solvers/ls/system.py:154-171).

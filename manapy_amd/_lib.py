@@ -159,6 +159,12 @@ class MfvKrylovWork(ctypes.Structure):
                 ('dinv', P), ('partial', P), ('scal', P), ('status', P)]
 
 
+class MfvKrylovFused(ctypes.Structure):
+    """Mirror of ``struct mfv_krylov_fused`` (include/mfv.h)."""
+    _fields_ = [(k, P) for k in ('x', 'b', 'd', 'rh', 'dinv', 'p', 'u', 'w', 'pa', 'pb', 'pr', 'scal', 'status', 'chunks',
+                                 'n_chunks')]
+
+
 class MfvSwBatch(ctypes.Structure):
     """Mirror of ``struct mfv_sw_batch`` (include/mfv.h)."""
     _fields_ = [('nb_inst', ctypes.c_int32), ('nb_waves', ctypes.c_int32), ('wave_inst', P), ('inst_cell0', P),
@@ -170,11 +176,13 @@ KS_IDLE, KS_START, KS_INNER, KS_CORRECT, KS_DONE, KS_FAILED = 0, 1, 2, 3, 4, 5
 KS_SIGMA, KS_TAU, KS_TOL_OUT, KS_TOL_IN, KS_MAXIT_IN, KS_MAXIT_OUT = 0, 1, 2, 3, 4, 5
 KS_RHO, KS_ALPHA, KS_OMEGA, KS_BETA, KS_R0N2, KS_RN2, KS_BN2, KS_RESN2 = 6, 7, 8, 9, 10, 11, 12, 13
 KS_IT, KS_OUTER, KS_ITTOT, KS_NSCAL = 14, 15, 16, 24
+KRYLOV_MAX_CHUNKS = 512
 
 MESH_P = ctypes.POINTER(MfvMesh)
 DIA_P = ctypes.POINTER(MfvDiamond)
 ELL_P = ctypes.POINTER(MfvEllBatch)
 KW_P = ctypes.POINTER(MfvKrylovWork)
+KF_P = ctypes.POINTER(MfvKrylovFused)
 SWB_P = ctypes.POINTER(MfvSwBatch)
 SWP_P = ctypes.POINTER(MfvSwPacked)
 SWM_P = ctypes.POINTER(MfvSwMixed)
@@ -278,6 +286,8 @@ _SIGNATURES = {
     'mfv_domain_geometry_3d_free': [ctypes.POINTER(MfvDomainGeometry3d)],
     'mfv_krylov_tick': [ELL_P, KW_P, c_int, c_int, c_int, P],
     'mfv_krylov_graph': [ELL_P, KW_P, c_int, c_int, c_int, ctypes.POINTER(c_void_p)],
+    'mfv_krylov_fused_tick': [ELL_P, KF_P, c_int, c_int, c_int, P],
+    'mfv_krylov_fused_graph': [ELL_P, KF_P, c_int, c_int, c_int, ctypes.POINTER(c_void_p)],
     'mfv_ell_spmv': [ELL_P, P, P, c_int, P],
     'mfv_ell_narrow_columns': [ELL_P, c_int, c_int, P, P, P],
 }

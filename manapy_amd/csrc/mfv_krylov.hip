@@ -453,6 +453,531 @@ __global__ void __launch_bounds__(256) k_ell_spmv(Ell e, const double *__restric
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// The same solve with two launches per iteration (mfv_krylov_fused_tick).
+//
+// The eight-launch iteration above is bound by launches and memory latency, not by bytes: at
+// 13k rows each of its kernels takes 3 to 4.6 us for under 1 us of traffic (32.8 us an
+// iteration). Here an iteration is two matrix products with everything else folded into them:
+//
+//   v:  omega, rho, beta from the sums of t;  d += alpha p + omega s;  r = s - omega t;
+//       p = r + beta (p - omega v);  v = M op(p);                            sum rh.v
+//   t:  alpha from the sum of v;  s = r - alpha v;  t = M op(s);
+//                                           sums t.s, t.t, s.s, rh.s, rh.t
+//
+// * M = 1 / diag scales the rows of the product (the system M op(d) = M r), so a slot needs
+//   nothing of its column but p (s), which is computed again from the column's record for each
+//   slot: three multiply-adds (one) and one gather of 16 bytes (8) instead of a launch and a
+//   trip of the vector through memory. The v product reads u = (s, t, p, v) and writes
+//   w = (r, v) and p; the t product reads those and writes u, so no row writes what another one
+//   reads. With M on the right the v product gathered 20 bytes and held 195 registers, two waves
+//   a SIMD: 12.0 us at 193k rows in eight systems, 8.5 us so.
+// * Measured, v and t product: 6.3 + 5.3 us at 12 800 rows and 8.5 + 7.2 us at 193k rows, against
+//   28 us and 29 us for the eight kernels. What is left is the chain chunk -> columns -> records
+//   with a trip to memory each, and the fixed cost of adding up.
+// * |r|^2 and rh.r of the new residual follow from the t product's sums (r = s - omega t), so
+//   omega, rho and beta need no third pass; the refinement's own residual stays FP64 and is
+//   formed from x itself.
+// * The sums have no launch of their own: every block of the next product adds up its
+//   instance's chunk sums, in the same fixed order, so all blocks hold the same bits. A chunk is
+//   four slices (one a wave) and an instance has at most 512, so that this costs two loads a
+//   thread; larger instances take more slices a chunk.
+// * A scalar is never read in the launch that writes it: the v product reads ALPHA, RHO_OLD, IT
+//   and STOP_T and writes OMEGA, BETA, RHO, RN2 and STOP_V; the t product reads RHO and STOP_V
+//   and writes ALPHA, RHO_OLD, IT, ITTOT and STOP_T. A launch for a stopped instance finds the
+//   sums unchanged and comes to the same verdict again. Only the instance's first block writes.
+struct Fused {
+    double *__restrict__ x;
+    double *__restrict__ b;
+    float *__restrict__ d;
+    float *__restrict__ rh;
+    float *__restrict__ dinv;
+    float4 *__restrict__ u;
+    float2 *__restrict__ w;
+    float *__restrict__ p;
+    double *__restrict__ pa;
+    double *__restrict__ pb;
+    double *__restrict__ pr;
+    double *__restrict__ scal;
+    int32_t *__restrict__ status;
+    const int4 *__restrict__ chunks;
+    const int32_t *__restrict__ n_chunks;
+};
+
+static Fused to_kernel(const mfv_krylov_fused *w)
+{
+    return Fused{w->x,  w->b,  w->d,  w->rh,   w->dinv,   reinterpret_cast<float4 *>(w->u),
+                 reinterpret_cast<float2 *>(w->w), w->p, w->pa, w->pb, w->pr, w->scal, w->status,
+                 reinterpret_cast<const int4 *>(w->chunks), w->n_chunks};
+}
+
+constexpr int kChunkBlock = 256;
+constexpr int kChunkWaves = kChunkBlock / 64;
+static_assert(MFV_KRYLOV_SPAN(1) == kChunkWaves, "a chunk's first slices are one a wave");
+
+// The wave's number in its block, known to be the same for all lanes (scalar slice tables).
+__device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
+
+struct Chunk {
+    int inst, s0, c, nch, ns, begin, end;
+};
+__device__ __forceinline__ Chunk chunk_at(const Fused &w, int k)
+{
+    const int4 q = w.chunks[k];
+    Chunk h;
+    h.inst = q.x;
+    h.s0 = q.y;
+    h.c = q.z & 0xffff;
+    h.nch = q.z >> 16;
+    h.ns = q.w;
+    const int span = MFV_KRYLOV_SPAN(q.w);
+    h.begin = h.s0 + h.c * span;
+    h.end = min(h.begin + span, h.s0 + h.ns);
+    return h;
+}
+
+// Sum over the wave, in every lane: moves inside the register file (row shifts, then the two row
+// broadcasts) instead of wave_sum's twelve trips through the LDS crossbar, which cost more than
+// the loads of a small instance's sums (v product of a stopped instance: 4.8 us against 3.0 us
+// for the t product, which adds one sum instead of five).
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double wave_total(double v)
+{
+    v += dpp_move<0x111>(v);  // row_shr:1
+    v += dpp_move<0x112>(v);  // row_shr:2
+    v += dpp_move<0x114>(v);  // row_shr:4
+    v += dpp_move<0x118>(v);  // row_shr:8: lane 15 of each row of 16 holds the row's sum
+    const long long b = __double_as_longlong(v);
+    double t = 0.;
+#pragma unroll
+    for (int r = 15; r < 64; r += 16) {
+        const int lo = __builtin_amdgcn_readlane((int)b, r), hi = __builtin_amdgcn_readlane((int)(b >> 32), r);
+        t += __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+    }
+    return t;
+}
+
+// The chunk sums part[k][s0 .. s0 + nch) of an instance, in an order that depends on nch alone;
+// every thread gets the totals. Up to 128 chunks (32 768 rows) each wave adds them up for itself,
+// two loads a lane and no barrier; above, the block shares them. Block-uniform calls only.
+template <int N>
+__device__ __forceinline__ void chunk_totals(const double *__restrict__ part, size_t S, int s0, int nch,
+                                             double (&out)[N])
+{
+    __shared__ double red[N][kChunkWaves];
+    double acc[N];
+    if (nch <= 128) {
+        const int i = threadIdx.x & 63;
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+            const double a = part[k * S + s0 + min(i, nch - 1)], b = part[k * S + s0 + min(i + 64, nch - 1)];
+            acc[k] = (i < nch ? a : 0.) + (i + 64 < nch ? b : 0.);
+        }
+#pragma unroll
+        for (int k = 0; k < N; k++) out[k] = wave_total(acc[k]);
+        return;
+    }
+#pragma unroll
+    for (int k = 0; k < N; k++) acc[k] = 0.;
+    for (int i = threadIdx.x; i < nch; i += kChunkBlock) {
+#pragma unroll
+        for (int k = 0; k < N; k++) acc[k] += part[k * S + s0 + i];
+    }
+    __syncthreads();  // the totals of the block's previous chunk have been read
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        const double a = wave_total(acc[k]);
+        if ((threadIdx.x & 63) == 0) red[k][threadIdx.x >> 6] = a;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        double a = red[k][0];
+#pragma unroll
+        for (int q = 1; q < kChunkWaves; q++) a += red[k][q];
+        out[k] = a;
+    }
+}
+
+// The block's sums of one chunk, from each lane's: stored at part[k][at] by one thread.
+template <int N>
+__device__ __forceinline__ void chunk_store(double *__restrict__ part, size_t S, int at, const double (&lane)[N])
+{
+    __shared__ double red[N][kChunkWaves];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        const double a = wave_total(lane[k]);
+        if ((threadIdx.x & 63) == 0) red[k][threadIdx.x >> 6] = a;
+    }
+    __syncthreads();
+    if (threadIdx.x < N) {
+        double a = red[threadIdx.x][0];
+#pragma unroll
+        for (int q = 1; q < kChunkWaves; q++) a += red[threadIdx.x][q];
+        part[threadIdx.x * S + at] = a;
+    }
+}
+
+// Slots of a row: values, and the records that load(column) returns, all requested before any is
+// used; add() then sums the slots below the slice's width in slot order. first() takes the slots
+// from 0 on without waiting for the width: the 16-bit columns, the values and the slice's width
+// are requested together (the arrays hold e.W slots whatever the width), and a slot past the
+// width takes the row itself. A triangle's row has at most 16 slots, so one first() is the row.
+template <class Rec, int N>
+struct SlotGroup {
+    float v[N];
+    Rec r[N];
+    template <class Load>
+    __device__ __forceinline__ int first(const Ell &e, int s, int lane, Load load)
+    {
+        const int row = s * 64 + lane;
+        const size_t base = (size_t)s * e.W * 64 + lane;
+        int c[N];
+        if (e.cols16) {
+#pragma unroll
+            for (int k = 0; k < N; k++) c[k] = e.cols16[base + (size_t)min(k, e.W - 1) * 64];
+        }
+#pragma unroll
+        for (int k = 0; k < N; k++) v[k] = e.vals32[base + (size_t)min(k, e.W - 1) * 64];
+        const int wdt = e.slice_w[s];
+        if (!slice_is_narrow(e, s)) {  // the same branch for the whole wave
+#pragma unroll
+            for (int k = 0; k < N; k++) c[k] = e.cols[base + (size_t)min(k, e.W - 1) * 64] - row;
+        }
+#pragma unroll
+        for (int k = 0; k < N; k++) r[k] = load(row + (k < wdt ? c[k] : 0));
+        return wdt;
+    }
+    template <class Load>
+    __device__ __forceinline__ void next(const Ell &e, int s, int lane, int j, int wdt, Load load)
+    {
+        const int row = s * 64 + lane;
+        const size_t base = (size_t)s * e.W * 64 + lane;
+        int c[N];
+        if (slice_is_narrow(e, s)) {
+#pragma unroll
+            for (int k = 0; k < N; k++) c[k] = row + e.cols16[base + (size_t)min(j + k, wdt - 1) * 64];
+        } else {
+#pragma unroll
+            for (int k = 0; k < N; k++) c[k] = e.cols[base + (size_t)min(j + k, wdt - 1) * 64];
+        }
+#pragma unroll
+        for (int k = 0; k < N; k++) v[k] = e.vals32[base + (size_t)min(j + k, wdt - 1) * 64];
+#pragma unroll
+        for (int k = 0; k < N; k++) r[k] = load(c[k]);
+    }
+    template <class Eval>
+    __device__ __forceinline__ float add(float acc, int j, int wdt, Eval eval) const
+    {
+#pragma unroll
+        for (int k = 0; k < N; k++)
+            if (j + k < wdt) acc = fmaf(v[k], eval(r[k]), acc);
+        return acc;
+    }
+};
+constexpr int kFirst = 16, kNext = 8;
+
+// x += d with the last iteration's alpha p + omega s (a stop before its t product has none).
+__global__ void __launch_bounds__(kChunkBlock) k_fused_correct(Fused w)
+{
+    const int n = *w.n_chunks;
+    for (int k = blockIdx.x; k < n; k += gridDim.x) {
+        const Chunk h = chunk_at(w, k);
+        if (w.status[h.inst] != MFV_KS_CORRECT) continue;
+        const double *sc = w.scal + (size_t)h.inst * MFV_KS_NSCAL;
+        const bool pending = sc[MFV_KS_STOP_T] == 0.;
+        const float alpha = (float)sc[MFV_KS_ALPHA], omega = (float)sc[MFV_KS_OMEGA];
+        for (int row = h.begin * 64 + threadIdx.x; row < h.end * 64; row += kChunkBlock) {
+            float d = w.d[row];
+            if (pending) {
+                const float4 u = w.u[row];
+                d = fmaf(omega, u.x, fmaf(alpha, u.z, d));
+            }
+            w.x[row] += (double)d;
+        }
+    }
+}
+
+// r = b - op(x) in FP64 (states START and CORRECT) and the start of the inner solve.
+__global__ void __launch_bounds__(kChunkBlock) k_fused_residual(Ell e, Fused w)
+{
+    const int lane = threadIdx.x & 63;
+    const int n = *w.n_chunks;
+    for (int k = blockIdx.x; k < n; k += gridDim.x) {
+        const Chunk h = chunk_at(w, k);
+        const int st = w.status[h.inst];
+        if (st != MFV_KS_START && st != MFV_KS_CORRECT) continue;
+        const double *sc = w.scal + (size_t)h.inst * MFV_KS_NSCAL;
+        const double sigma = sc[MFV_KS_SIGMA], tau = sc[MFV_KS_TAU];
+        double sum[3] = {0., 0., 0.};
+        for (int s = h.begin + wave_index(); s < h.end; s += kChunkWaves) {
+            const int row = s * 64 + lane;
+            float di;
+            if (st == MFV_KS_START) {
+                const double dg = sigma + tau * e.diag[row];
+                w.dinv[row] = di = (dg != 0.) ? (float)(1. / dg) : 0.f;
+            } else {
+                di = w.dinv[row];
+            }
+            const double ax = ell_row64(e, s, lane, w.x);
+            const double bb = w.b[row];
+            const double res = bb - (sigma * w.x[row] + tau * ax);
+            const float r32 = (float)((double)di * res);
+            w.rh[row] = r32;
+            w.d[row] = 0.f;
+            w.u[row] = make_float4(r32, 0.f, 0.f, 0.f);
+            sum[0] += res * res;
+            sum[1] += bb * bb;
+            sum[2] += (double)r32 * (double)r32;
+        }
+        chunk_store<3>(w.pr, e.S, h.s0 + h.c, sum);
+    }
+}
+
+__device__ __forceinline__ int chunks_of(int ns) { return (ns + MFV_KRYLOV_SPAN(ns) - 1) / MFV_KRYLOV_SPAN(ns); }
+
+__global__ void __launch_bounds__(kChunkBlock) k_fused_check(Ell e, Fused w)
+{
+    const int n = *e.n_live_inst;
+    for (int i = blockIdx.x; i < n; i += gridDim.x) {
+        const int inst = e.live_inst[i];
+        const int was = w.status[inst];
+        __syncthreads();  // read by every thread before thread 0 changes it
+        if (was != MFV_KS_START && was != MFV_KS_CORRECT) continue;
+        double sum[3];
+        chunk_totals<3>(w.pr, e.S, e.inst_slice0[inst], chunks_of(e.inst_nslices[inst]), sum);
+        if (threadIdx.x == 0) {
+            double *sc = w.scal + (size_t)inst * MFV_KS_NSCAL;
+            const double resn2 = sum[0], bn2 = sum[1];
+            sc[MFV_KS_RESN2] = resn2;
+            sc[MFV_KS_BN2] = bn2;
+            if (was == MFV_KS_START) sc[MFV_KS_OUTER] = 0.;
+            sc[MFV_KS_OUTER] += 1.;
+            const double tol = sc[MFV_KS_TOL_OUT];
+            int st;
+            if (!isfinite(resn2) || !isfinite(bn2)) st = MFV_KS_FAILED;  // NaN/inf data: refinement cannot help
+            else if (resn2 <= tol * tol * bn2) st = MFV_KS_DONE;
+            else if (sc[MFV_KS_OUTER] > sc[MFV_KS_MAXIT_OUT]) st = MFV_KS_FAILED;
+            else {
+                sc[MFV_KS_RHO] = sum[2];
+                sc[MFV_KS_RHO_OLD] = sum[2];
+                sc[MFV_KS_R0N2] = sum[2];
+                sc[MFV_KS_RN2] = sum[2];
+                sc[MFV_KS_ALPHA] = 0.;
+                sc[MFV_KS_OMEGA] = 0.;
+                sc[MFV_KS_BETA] = 0.;
+                sc[MFV_KS_IT] = 0.;
+                sc[MFV_KS_STOP_V] = 0.;
+                sc[MFV_KS_STOP_T] = 0.;
+                st = MFV_KS_INNER;
+            }
+            w.status[inst] = st;
+        }
+    }
+}
+
+// omega, the new residual's norm and rho, and whether the inner solve ends, from the t product's
+// sums (t.s, t.t, s.s, rh.s, rh.t).
+struct Step {
+    double omega, rn2, rho;
+    bool done;
+};
+struct Stop {
+    double tol, r0n2, it, maxit;
+};
+__device__ __forceinline__ Stop stop_of(const double *sc)
+{
+    return Stop{sc[MFV_KS_TOL_IN], sc[MFV_KS_R0N2], sc[MFV_KS_IT], sc[MFV_KS_MAXIT_IN]};
+}
+__device__ __forceinline__ Step close_step(const double (&q)[5], const Stop &s)
+{
+    Step r;
+    const double om = (q[1] != 0.) ? q[0] / q[1] : 0.;
+    r.omega = isfinite(om) ? om : 0.;
+    r.rn2 = q[2] - 2. * r.omega * q[0] + r.omega * r.omega * q[1];
+    r.rho = q[3] - r.omega * q[4];
+    r.done = r.rn2 <= s.tol * s.tol * s.r0n2 || s.it >= s.maxit || r.rho == 0. || r.omega == 0.;
+    return r;
+}
+
+__global__ void __launch_bounds__(kChunkBlock, 3) k_fused_v(Ell e, Fused w)
+{
+    const int lane = threadIdx.x & 63;
+    Chunk h = chunk_at(w, min((int)blockIdx.x, e.S - 1));  // with the count, not after it
+    const int n = *w.n_chunks;
+    for (int k = blockIdx.x; k < n; k += gridDim.x) {
+        if (k != (int)blockIdx.x) h = chunk_at(w, k);
+        double *sc = w.scal + (size_t)h.inst * MFV_KS_NSCAL;
+        const int status = w.status[h.inst];  // the scalars too, before anything is waited for
+        const double stopped = sc[MFV_KS_STOP_T], rho_old = sc[MFV_KS_RHO_OLD], alpha_old = sc[MFV_KS_ALPHA];
+        const float sigma = (float)sc[MFV_KS_SIGMA], tau = (float)sc[MFV_KS_TAU];
+        const Stop lim = stop_of(sc);
+        auto load = [&](int c) { return w.u[c]; };
+        // the first slots' records are on their way while the sums are added up, also for an
+        // instance that turns out to be idle
+        int s = h.begin + wave_index();
+        SlotGroup<float4, kFirst> g;
+        float4 own;
+        float rh = 0.f, d = 0.f, di = 0.f;
+        int wdt = 0;
+        auto take = [&]() {
+            const int row = s * 64 + lane;
+            own = load(row);
+            rh = w.rh[row];
+            d = w.d[row];
+            di = w.dinv[row];
+            wdt = g.first(e, s, lane, load);
+        };
+        if (s < h.end) take();
+        double q[5];
+        chunk_totals<5>(w.pb, e.S, h.s0, h.nch, q);
+        if (status != MFV_KS_INNER || stopped != 0.) continue;
+        float alpha = 0.f, om = 0.f, be = 0.f;
+        if (lim.it != 0.) {
+            const Step st = close_step(q, lim);
+            const double beta = (st.rho / rho_old) * (alpha_old / st.omega);
+            if (h.c == 0 && threadIdx.x == 0) {
+                sc[MFV_KS_OMEGA] = st.omega;
+                sc[MFV_KS_RN2] = st.rn2;
+                if (st.done) {
+                    sc[MFV_KS_STOP_V] = 1.;
+                } else {
+                    sc[MFV_KS_BETA] = beta;
+                    sc[MFV_KS_RHO] = st.rho;
+                }
+            }
+            if (st.done) continue;
+            alpha = (float)alpha_old;
+            om = (float)st.omega;
+            be = (float)beta;
+        }
+        auto p_of = [&](const float4 &u) { return fmaf(be, fmaf(-om, u.w, u.z), fmaf(-om, u.y, u.x)); };
+        double sum[1] = {0.};
+        while (s < h.end) {
+            const int row = s * 64 + lane;
+            float acc = g.add(0.f, 0, wdt, p_of);
+            for (int j = kFirst; j < wdt; j += kNext) {
+                SlotGroup<float4, kNext> m;
+                m.next(e, s, lane, j, wdt, load);
+                acc = m.add(acc, j, wdt, p_of);
+            }
+            const float p = p_of(own);
+            const float v = di * fmaf(sigma, p, tau * acc);
+            w.d[row] = fmaf(om, own.x, fmaf(alpha, own.z, d));
+            w.w[row] = make_float2(fmaf(-om, own.y, own.x), v);
+            w.p[row] = p;
+            sum[0] += (double)rh * (double)v;
+            s += kChunkWaves;
+            if (s < h.end) take();
+        }
+        chunk_store<1>(w.pa, e.S, h.s0 + h.c, sum);
+    }
+}
+
+__global__ void __launch_bounds__(kChunkBlock) k_fused_t(Ell e, Fused w)
+{
+    const int lane = threadIdx.x & 63;
+    Chunk h = chunk_at(w, min((int)blockIdx.x, e.S - 1));
+    const int n = *w.n_chunks;
+    for (int k = blockIdx.x; k < n; k += gridDim.x) {
+        if (k != (int)blockIdx.x) h = chunk_at(w, k);
+        double *sc = w.scal + (size_t)h.inst * MFV_KS_NSCAL;
+        const int status = w.status[h.inst];
+        const double stopped = sc[MFV_KS_STOP_V], rho = sc[MFV_KS_RHO];
+        const float sigma = (float)sc[MFV_KS_SIGMA], tau = (float)sc[MFV_KS_TAU];
+        auto load = [&](int c) { return w.w[c]; };
+        int s = h.begin + wave_index();
+        SlotGroup<float2, kFirst> g;
+        float2 own;
+        float rh = 0.f, di = 0.f, p = 0.f;
+        int wdt = 0;
+        auto take = [&]() {
+            const int row = s * 64 + lane;
+            own = load(row);
+            rh = w.rh[row];
+            di = w.dinv[row];
+            p = w.p[row];
+            wdt = g.first(e, s, lane, load);
+        };
+        if (s < h.end) take();
+        double rv[1];
+        chunk_totals<1>(w.pa, e.S, h.s0, h.nch, rv);
+        if (status != MFV_KS_INNER || stopped != 0.) continue;
+        const double a = rho / rv[0];
+        const bool broken = rv[0] == 0. || !isfinite(a);  // breakdown: refine with what d holds
+        if (h.c == 0 && threadIdx.x == 0) {
+            if (broken) {
+                sc[MFV_KS_STOP_T] = 1.;
+            } else {
+                sc[MFV_KS_ALPHA] = a;
+                sc[MFV_KS_RHO_OLD] = rho;
+                sc[MFV_KS_IT] += 1.;
+                sc[MFV_KS_ITTOT] += 1.;
+            }
+        }
+        if (broken) continue;
+        const float al = (float)a;
+        auto s_of = [&](const float2 &r) { return fmaf(-al, r.y, r.x); };
+        double sum[5] = {0., 0., 0., 0., 0.};
+        while (s < h.end) {
+            const int row = s * 64 + lane;
+            float acc = g.add(0.f, 0, wdt, s_of);
+            for (int j = kFirst; j < wdt; j += kNext) {
+                SlotGroup<float2, kNext> m;
+                m.next(e, s, lane, j, wdt, load);
+                acc = m.add(acc, j, wdt, s_of);
+            }
+            const float ss = s_of(own);
+            const float t = di * fmaf(sigma, ss, tau * acc);
+            w.u[row] = make_float4(ss, t, p, own.y);
+            sum[0] += (double)t * (double)ss;
+            sum[1] += (double)t * (double)t;
+            sum[2] += (double)ss * (double)ss;
+            sum[3] += (double)rh * (double)ss;
+            sum[4] += (double)rh * (double)t;
+            s += kChunkWaves;
+            if (s < h.end) take();
+        }
+        chunk_store<5>(w.pb, e.S, h.s0 + h.c, sum);
+    }
+}
+
+// The end of a tick: an inner solve that has ended moves to CORRECT, so that the next tick starts
+// with its refinement (its last sums would otherwise be looked at one tick later).
+__global__ void __launch_bounds__(kChunkBlock) k_fused_close(Ell e, Fused w)
+{
+    const int n = *e.n_live_inst;
+    for (int i = blockIdx.x; i < n; i += gridDim.x) {
+        const int inst = e.live_inst[i];
+        double *sc = w.scal + (size_t)inst * MFV_KS_NSCAL;
+        const int was = w.status[inst];
+        const bool stopped = sc[MFV_KS_STOP_V] != 0. || sc[MFV_KS_STOP_T] != 0.;
+        const bool fresh = sc[MFV_KS_IT] == 0.;
+        __syncthreads();  // read by every thread before thread 0 changes them
+        if (was != MFV_KS_INNER || (fresh && !stopped)) continue;
+        if (stopped) {
+            if (threadIdx.x == 0) w.status[inst] = MFV_KS_CORRECT;
+            continue;
+        }
+        double q[5];
+        chunk_totals<5>(w.pb, e.S, e.inst_slice0[inst], chunks_of(e.inst_nslices[inst]), q);
+        const Step st = close_step(q, stop_of(sc));
+        if (st.done && threadIdx.x == 0) {
+            sc[MFV_KS_OMEGA] = st.omega;
+            sc[MFV_KS_RN2] = st.rn2;
+            w.status[inst] = MFV_KS_CORRECT;
+        }
+    }
+}
+
 static int validate_ell(const mfv_ell_batch *e)
 {
     MFV_REQUIRE(e != nullptr, "ELL batch descriptor is NULL");
@@ -526,6 +1051,64 @@ extern "C" int mfv_krylov_graph(const mfv_ell_batch *e, const mfv_krylov_work *w
     MfvGraph *g = new MfvGraph();
     int rc = graph_begin(g);
     if (rc == MFV_OK) rc = graph_finish(g, tick_launches(e, w, n_iter, grid_slices, grid_inst, g->stream));
+    if (rc != MFV_OK) {
+        graph_free(g);
+        return rc;
+    }
+    *graph_out = g;
+    return MFV_OK;
+}
+
+static int check_fused(const mfv_ell_batch *e, const mfv_krylov_fused *w, int n_iter, int grid_chunks, int grid_inst)
+{
+    if (int rc = validate_ell(e)) return rc;
+    MFV_REQUIRE(w != nullptr, "Krylov work descriptor is NULL");
+    MFV_REQUIRE(w->x && w->b && w->d && w->rh && w->dinv && w->u && w->w && w->p && w->pa && w->pb && w->pr && w->scal &&
+                    w->status && w->chunks && w->n_chunks,
+                "Krylov work descriptor has NULL pointers");
+    MFV_REQUIRE(((reinterpret_cast<uintptr_t>(w->u) | reinterpret_cast<uintptr_t>(w->w) |
+                  reinterpret_cast<uintptr_t>(w->chunks)) &
+                 15) == 0,
+                "u, w and chunks must be 16-byte aligned");
+    MFV_REQUIRE(n_iter >= 0 && n_iter <= 4096, "n_iter %d out of [0, 4096]", n_iter);
+    MFV_REQUIRE(grid_chunks >= 1 && grid_chunks <= 65536, "grid_chunks %d out of [1, 65536]", grid_chunks);
+    MFV_REQUIRE(grid_inst >= 1 && grid_inst <= 65536, "grid_inst %d out of [1, 65536]", grid_inst);
+    return MFV_OK;
+}
+
+static int fused_launches(const mfv_ell_batch *e, const mfv_krylov_fused *w, int n_iter, int grid_chunks,
+                          int grid_inst, hipStream_t st)
+{
+    const Ell ek = to_kernel(e);
+    const Fused wk = to_kernel(w);
+    const dim3 gc(grid_chunks), gi(grid_inst), b(kChunkBlock);
+    hipLaunchKernelGGL(k_fused_correct, gc, b, 0, st, wk);
+    hipLaunchKernelGGL(k_fused_residual, gc, b, 0, st, ek, wk);
+    hipLaunchKernelGGL(k_fused_check, gi, b, 0, st, ek, wk);
+    for (int it = 0; it < n_iter; it++) {
+        hipLaunchKernelGGL(k_fused_v, gc, b, 0, st, ek, wk);
+        hipLaunchKernelGGL(k_fused_t, gc, b, 0, st, ek, wk);
+    }
+    hipLaunchKernelGGL(k_fused_close, gi, b, 0, st, ek, wk);
+    return check_launch("krylov tick");
+}
+
+extern "C" int mfv_krylov_fused_tick(const mfv_ell_batch *e, const mfv_krylov_fused *w, int n_iter, int grid_chunks,
+                                     int grid_inst, void *stream)
+{
+    if (int rc = check_fused(e, w, n_iter, grid_chunks, grid_inst)) return rc;
+    return fused_launches(e, w, n_iter, grid_chunks, grid_inst, as_stream(stream));
+}
+
+extern "C" int mfv_krylov_fused_graph(const mfv_ell_batch *e, const mfv_krylov_fused *w, int n_iter, int grid_chunks,
+                                      int grid_inst, void **graph_out)
+{
+    if (int rc = check_fused(e, w, n_iter, grid_chunks, grid_inst)) return rc;
+    MFV_REQUIRE(graph_out, "graph_out is NULL");
+    *graph_out = nullptr;
+    MfvGraph *g = new MfvGraph();
+    int rc = graph_begin(g);
+    if (rc == MFV_OK) rc = graph_finish(g, fused_launches(e, w, n_iter, grid_chunks, grid_inst, g->stream));
     if (rc != MFV_OK) {
         graph_free(g);
         return rc;

@@ -59,6 +59,20 @@ class RangeAllocator(object):
         return max((m for _, m in self.free), default=0)
 
 
+def chunk_list(ranges):
+    """Chunks [n][4] int32 (mfv_krylov_fused in include/mfv.h) of live instances given as
+    (instance, first slice, slices), in the order given."""
+    out = []
+    for inst, s0, ns in ranges:
+        span = 4 * ((ns + 4 * _lib.KRYLOV_MAX_CHUNKS - 1) // (4 * _lib.KRYLOV_MAX_CHUNKS))
+        n = (ns + span - 1) // span
+        c = np.empty((n, 4), dtype=np.int32)
+        c[:, 0], c[:, 1], c[:, 3] = inst, s0, ns
+        c[:, 2] = np.arange(n) | (n << 16)
+        out.append(c)
+    return np.concatenate(out) if out else np.zeros((0, 4), np.int32)
+
+
 class EllBatch(object):
     def __init__(self, max_slices, max_inst=64, width=32, device=None):
         torch = require_gpu()
@@ -86,8 +100,11 @@ class EllBatch(object):
         R = S * 64
         self.x = torch.zeros(R, dtype=f64, device=dev)
         self.b = torch.zeros(R, dtype=f64, device=dev)
-        self.f32 = {k: torch.zeros(R, dtype=f32, device=dev) for k in ('d', 'r', 'rh', 'p', 'v', 'yz', 't', 'dinv')}
-        self.partial = torch.zeros(S * 4, dtype=f64, device=dev)
+        self.f32 = {k: torch.zeros(R, dtype=f32, device=dev) for k in ('d', 'rh', 'dinv', 'p')}
+        self.f32.update({k: torch.zeros((R, n), dtype=f32, device=dev) for k, n in (('u', 4), ('w', 2))})
+        self.partial = {k: torch.zeros(S * n, dtype=f64, device=dev) for k, n in (('pa', 1), ('pb', 5), ('pr', 3))}
+        self.chunks = torch.zeros((S, 4), dtype=i32, device=dev)
+        self.n_chunks = torch.zeros(1, dtype=i32, device=dev)
         self.scal = torch.zeros(I * _lib.KS_NSCAL, dtype=f64, device=dev)
         self.status = torch.zeros(I, dtype=i32, device=dev)
 
@@ -96,11 +113,11 @@ class EllBatch(object):
         for k in ('slice_inst', 'slice_w', 'cols', 'vals', 'vals32', 'diag', 'inst_slice0', 'inst_nslices',
                   'live_slices', 'n_live_slices', 'live_inst', 'n_live_inst', 'cols16', 'slice_narrow'):
             setattr(e, k, getattr(self, k).data_ptr())
-        w = _lib.MfvKrylovWork()
-        w.x, w.b = self.x.data_ptr(), self.b.data_ptr()
-        for k, t in self.f32.items():
+        w = _lib.MfvKrylovFused()
+        for k, t in dict(self.f32, **self.partial).items():
             setattr(w, k, t.data_ptr())
-        w.partial, w.scal, w.status = self.partial.data_ptr(), self.scal.data_ptr(), self.status.data_ptr()
+        for k in ('x', 'b', 'scal', 'status', 'chunks', 'n_chunks'):
+            setattr(w, k, getattr(self, k).data_ptr())
         self._e, self._w = e, w
         self._ranges = RangeAllocator(S)
         self._inst = {}                # inst -> (slice0, nslices, nrows)
@@ -167,7 +184,11 @@ class EllBatch(object):
             self.inst_slice0[idx] = s0
             self.inst_nslices[idx] = ns
         self.n_live_inst.fill_(len(insts))
-        self._n_live = (len(sl), len(insts))
+        ch = chunk_list([(i,) + self._inst[i][:2] for i in insts])
+        if len(ch):
+            self.chunks[:len(ch)] = torch.from_numpy(ch).to(self.device)
+        self.n_chunks.fill_(len(ch))
+        self._n_live = (len(sl), len(insts), len(ch))
 
     # -- matrix and system ------------------------------------------------------------------------
     def assemble_diamond(self, inst, ddia, node_dir, face_dir_rank):
@@ -237,7 +258,8 @@ class EllBatch(object):
 
     # -- execution ----------------------------------------------------------------------------
     def grids(self):
-        nsl, ni = getattr(self, '_n_live', (0, 0))
+        """Blocks of the per-slice (spmv) and per-instance kernels."""
+        nsl, ni, _ = getattr(self, '_n_live', (0, 0, 0))
         return max(1, min(4096, (nsl + 3) // 4)), max(1, ni)
 
     def tick(self, n_iter=8, grid_slices=None, grid_inst=None, stream=None, graph=False):
@@ -245,17 +267,18 @@ class EllBatch(object):
         replayed from a HIP graph captured once per (n_iter, grid sizes rounded up to powers of
         two): the kernels read the live lists from device memory, so a graph stays valid as
         instances come and go, and the result is the same bits as the eager tick."""
-        gs, gi = self.grids()
-        gs, gi = int(grid_slices or gs), int(grid_inst or gi)
+        _, gi = self.grids()
+        nch = max(1, min(16384, getattr(self, '_n_live', (0, 0, 0))[2]))
+        gs, gi = int(grid_slices or nch), int(grid_inst or gi)
         if not graph:
-            _lib.call('mfv_krylov_tick', self.eptr, self.wptr, int(n_iter), gs, gi, stream_ptr(stream))
+            _lib.call('mfv_krylov_fused_tick', self.eptr, self.wptr, int(n_iter), gs, gi, stream_ptr(stream))
             return
-        key = (int(n_iter), min(4096, _pow2(gs)), min(65536, _pow2(gi)))
+        key = (int(n_iter), min(16384, _pow2(gs)), min(65536, _pow2(gi)))
         graphs = self.__dict__.setdefault('_graphs', {})
         g = graphs.get(key)
         if g is None:
             out = ctypes.c_void_p()
-            _lib.call('mfv_krylov_graph', self.eptr, self.wptr, key[0], key[1], key[2], ctypes.byref(out))
+            _lib.call('mfv_krylov_fused_graph', self.eptr, self.wptr, key[0], key[1], key[2], ctypes.byref(out))
             g = graphs[key] = out.value
         _lib.call('mfv_graph_launch', g, stream_ptr(stream))
 
