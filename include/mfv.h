@@ -78,6 +78,18 @@ int mfv_device_count(int *count_host);
 int mfv_ghost_value(const mfv_mesh *m, int kind, const double *src, double *w_ghost,
                     const int32_t *faces, int nfaces, void *stream);
 
+/* The ghost fills of several boundary locations and fields in one launch: for each of the nseg
+ * segments (a host array), over its n faces f: ghost[f] = w[face_cells[f][0]] (kind 0), minus
+ * that (1), w[f] (2, w = the boundary values) or w[face_cells[f][0]] + cst[f] * dist[f] (3). */
+typedef struct mfv_ghost_seg {
+    const int32_t *faces;
+    const double *w;
+    double *ghost;
+    const double *cst, *dist; /* kind 3 only */
+    int32_t n, kind;
+} mfv_ghost_seg;
+int mfv_ghost_values(const mfv_mesh *m, const mfv_ghost_seg *segs, int nseg, void *stream);
+
 /* facetocell (ast/ast_utils.py:8-18). */
 int mfv_facetocell(const mfv_mesh *m, const double *u_face, double *u_c, void *stream);
 

@@ -159,6 +159,12 @@ class MfvKrylovWork(ctypes.Structure):
                 ('dinv', P), ('partial', P), ('scal', P), ('status', P)]
 
 
+class MfvGhostSeg(ctypes.Structure):
+    """Mirror of ``struct mfv_ghost_seg`` (include/mfv.h)."""
+    _fields_ = [(k, P) for k in ('faces', 'w', 'ghost', 'cst', 'dist')] + \
+        [('n', ctypes.c_int32), ('kind', ctypes.c_int32)]
+
+
 class MfvKrylovFused(ctypes.Structure):
     """Mirror of ``struct mfv_krylov_fused`` (include/mfv.h)."""
     _fields_ = [(k, P) for k in ('x', 'b', 'd', 'rh', 'dinv', 'p', 'u', 'w', 'pa', 'pb', 'pr', 'scal', 'status', 'chunks',
@@ -198,6 +204,7 @@ _SIGNATURES = {
     'mfv_last_error': [],
     'mfv_device_count': [ctypes.POINTER(c_int)],
     'mfv_ghost_value': [MESH_P, c_int, P, P, P, c_int, P],
+    'mfv_ghost_values': [MESH_P, ctypes.POINTER(MfvGhostSeg), c_int, P],
     'mfv_facetocell': [MESH_P, P, P, P],
     'mfv_cell_gradient': [MESH_P, P, P, P, P, P, P],
     'mfv_barthlimiter': [MESH_P, P, P, P, P, P, P, P],

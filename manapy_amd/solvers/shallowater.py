@@ -21,7 +21,7 @@ import numpy as np
 from .. import _lib
 from ..base import Struct, make_get_conf, process_conf
 from ..device import stream_ptr, SwPacked
-from ..variable import Variable
+from ..variable import Variable, fill_ghosts
 from ._common import DeviceClock
 
 
@@ -63,6 +63,7 @@ class ShallowWaterSolver(object):
             raise ValueError("hC must be a Variable type")
         self.Z = Z if Z is not None else Variable(domain=self.domain)
         self.hc = hc if hc is not None else Variable(domain=self.domain)
+        self._ghost_cache = []
         self.varbs = {'h': self.h, 'hu': self.hu, 'hv': self.hv, 'hc': self.hc, 'Z': self.Z}
         self.Dxx, self.Dyy, self.Dzz = get("Dxx"), get("Dyy"), 0.
         self.dt = get("dt")
@@ -191,8 +192,7 @@ class ShallowWaterSolver(object):
         return self.dt
 
     def update_ghost_values(self):
-        for var in self.varbs.values():
-            var.update_ghost_value()
+        fill_ghosts(self.domain, [(bc, v) for v in self.varbs.values() for bc in v.BCs.values()], self._ghost_cache)
 
     def explicit_convective(self):
         """``system.py:162-178``. Rusanov: gradients of eta, hu, hv, then residuals."""

@@ -9,7 +9,8 @@ with ``var.cell[:] = ...`` (tensor or numpy) and read back with ``var.cell.cpu()
 Boundary conditions follow ``ast/core.py:105-335`` and ``boundary/bc.py``: a dict
 ``{"in": "neumann" | "dirichlet" | "nonslip" | "neumannNH" | "slip", ...}`` and, for
 Dirichlet / non-homogeneous Neumann, ``values={"in": float | lambda x, y, z: ...}``.
-The ghost fill of every BC kind runs in ``mfv_ghost_value`` on the device.
+The ghost fill of every BC kind runs in ``mfv_ghost_values`` on the device, one launch for all
+locations.
 """
 import types
 
@@ -18,7 +19,22 @@ import numpy as np
 from . import _lib
 from .device import stream_ptr
 
-_KIND = {"neumann": 0, "periodic": 0, "slip": 0, "nonslip": 1, "dirichlet": 2}
+_KIND = {"neumann": 0, "periodic": 0, "slip": 0, "nonslip": 1, "dirichlet": 2, "neumannNH": 3}
+
+
+def fill_ghosts(domain, pairs, cache=None):
+    """Ghost values of (boundary location, Variable) pairs in one launch (mfv_ghost_values).
+    ``cache``: a list that keeps the segments between calls; they are built again whenever an
+    array they point to is another one."""
+    pairs = [(b, v) for b, v in pairs if len(b.BCfaces)]
+    key = [b.ghost_key(v) for b, v in pairs]
+    if cache and cache[0] == key:
+        segs = cache[1]
+    else:
+        segs = (_lib.MfvGhostSeg * len(pairs))(*[b.ghost_segment(v) for b, v in pairs])
+        if cache is not None:
+            cache[:] = [key, segs]
+    _lib.call('mfv_ghost_values', domain.device_mesh.ptr, segs, len(pairs), stream_ptr())
 
 
 class Boundary(object):
@@ -74,22 +90,26 @@ class Boundary(object):
 
     def fill_ghost(self, var):
         """ghost_value_* of ``boundary/bc_utils.py:45-68`` for this location."""
-        n = len(self._BCfaces)
-        if n == 0:
-            return
-        dm = self._domain.device_mesh
-        if self._BCtype == "neumannNH":
-            # w_ghost[f] = w_c[cellid[f][0]] + cst[f] * dist[f]
-            _lib.call('mfv_ghost_value', dm.ptr, 0, var.cell.data_ptr(), var.ghost.data_ptr(),
-                      self._faces_dev.data_ptr(), n, stream_ptr())
-            import torch
-            f = self._faces_dev.long()
-            var.ghost[f] = var.ghost[f] + self.constNH[f] * dm.dist_ortho[f]
-            return
-        kind = _KIND[self._BCtype]
-        src = self.BCvalueface if kind == 2 else var.cell
-        _lib.call('mfv_ghost_value', dm.ptr, kind, src.data_ptr(), var.ghost.data_ptr(), self._faces_dev.data_ptr(),
-                  n, stream_ptr())
+        fill_ghosts(self._domain, [(self, var)])
+
+    def ghost_key(self, var):
+        """The device addresses that a ghost segment of this location holds."""
+        kind, more = self._BCtype, ()
+        if kind == "dirichlet":
+            more = (self.BCvalueface.data_ptr(),)
+        elif kind == "neumannNH":
+            more = (self.constNH.data_ptr(), self._domain.device_mesh.dist_ortho.data_ptr())
+        return (var.cell.data_ptr(), var.ghost.data_ptr(), self._faces_dev.data_ptr(), kind) + more
+
+    def ghost_segment(self, var):
+        """``mfv_ghost_seg`` of this location and field."""
+        s = _lib.MfvGhostSeg()
+        s.faces, s.ghost, s.n = self._faces_dev.data_ptr(), var.ghost.data_ptr(), len(self._BCfaces)
+        s.kind = _KIND[self._BCtype]
+        s.w = (self.BCvalueface if s.kind == 2 else var.cell).data_ptr()
+        if s.kind == 3:  # w_ghost[f] = w_c[cellid[f][0]] + cst[f] * dist[f]
+            s.cst, s.dist = self.constNH.data_ptr(), self._domain.device_mesh.dist_ortho.data_ptr()
+        return s
 
     domain = property(lambda self: self._domain)
     BCfaces = property(lambda self: self._BCfaces)
@@ -166,6 +186,7 @@ class Variable(object):
         self.BCneumann = np.asarray(self.BCneumann, dtype=np.int32)
         self.BCneumannNH = np.asarray(self.BCneumannNH, dtype=np.int32)
         self._diamond_bc = None
+        self._ghost_cache = []
 
     def diamond_bc(self):
         """Device tables (node_dir, face_dir_rank, face_bc) of the diamond kernels."""
@@ -183,8 +204,7 @@ class Variable(object):
 
     def update_ghost_value(self):
         """``ast/core.py:492-497``."""
-        for bc in self._BCs.values():
-            bc.fill_ghost(self)
+        fill_ghosts(self._domain, [(bc, self) for bc in self._BCs.values()], self._ghost_cache)
 
     def interpolate_facetocell(self):
         """``ast/core.py:422-423`` -> ``ast_utils.facetocell``."""
