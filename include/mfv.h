@@ -102,6 +102,14 @@ int mfv_cell_gradient(const mfv_mesh *m, const double *w_c, const double *w_ghos
 int mfv_barthlimiter(const mfv_mesh *m, const double *w_c, const double *w_ghost,
                      const double *w_x, const double *w_y, const double *w_z, double *psi, void *stream);
 
+/* mfv_cell_gradient then mfv_barthlimiter of one or two fields in one launch (the same bits;
+ * the geometry is read once for both). */
+typedef struct mfv_gradient_fields {
+    const double *w, *ghost;
+    double *gx, *gy, *gz, *psi;
+} mfv_gradient_fields;
+int mfv_cell_gradient_limited(const mfv_mesh *m, int nfields, const mfv_gradient_fields *f, void *stream);
+
 /* ---------------- advection (solvers/advec) --------------------------------------- */
 
 /* time_step (solvers/advec/fvm_utils.py:293-309): dt = min_K cfl |K| / sum_f |u_K.n_f|.

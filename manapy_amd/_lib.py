@@ -165,6 +165,11 @@ class MfvGhostSeg(ctypes.Structure):
         [('n', ctypes.c_int32), ('kind', ctypes.c_int32)]
 
 
+class MfvGradientFields(ctypes.Structure):
+    """Mirror of ``struct mfv_gradient_fields`` (include/mfv.h)."""
+    _fields_ = [(k, P) for k in ('w', 'ghost', 'gx', 'gy', 'gz', 'psi')]
+
+
 class MfvKrylovFused(ctypes.Structure):
     """Mirror of ``struct mfv_krylov_fused`` (include/mfv.h)."""
     _fields_ = [(k, P) for k in ('x', 'b', 'd', 'rh', 'dinv', 'p', 'u', 'w', 'pa', 'pb', 'pr', 'scal', 'status', 'chunks',
@@ -208,6 +213,7 @@ _SIGNATURES = {
     'mfv_facetocell': [MESH_P, P, P, P],
     'mfv_cell_gradient': [MESH_P, P, P, P, P, P, P],
     'mfv_barthlimiter': [MESH_P, P, P, P, P, P, P, P],
+    'mfv_cell_gradient_limited': [MESH_P, c_int, ctypes.POINTER(MfvGradientFields), P],
     'mfv_time_step': [MESH_P, P, P, P, c_double, P, DP, P],
     'mfv_explicitscheme_convective': [MESH_P, P, P, P, P, P, P, P, P, P, P, c_int, P],
     'mfv_update_new_value': [MESH_P, P, P, P, P, c_double, P, P],

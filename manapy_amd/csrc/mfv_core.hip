@@ -317,6 +317,182 @@ extern "C" int mfv_barthlimiter(const mfv_mesh *m, const double *w_c, const doub
 }
 
 // ---------------------------------------------------------------------------------------------
+// gradient and limiter of NF fields in one pass (cell_gradient then barthlimiter, bit for bit)
+
+template <int NF>
+struct GradArgs {
+    const double *__restrict__ w[NF];
+    const double *__restrict__ ghost[NF];
+    double *__restrict__ gx[NF];
+    double *__restrict__ gy[NF];
+    double *__restrict__ gz[NF];
+    double *__restrict__ psi[NF];
+};
+
+template <int DIM, int NF>
+__device__ __forceinline__ void stencil_sums(const Mesh &m, const GradArgs<NF> &a, int i, double cx, double cy,
+                                             double cz, const double (&wi)[NF], double (&I)[6], double (&J)[NF][3])
+{
+    constexpr int G = 8;
+    const int nn = m.lsq_ncells[i], ng = m.lsq_nghosts[i];
+    const int nmax = wave_max_int(nn), gmax = wave_max_int(ng);
+    int c[G];
+#pragma unroll
+    for (int k = 0; k < G; k++) c[k] = (k < m.K) ? m.lsq_cells[(size_t)k * m.C + i] : 0;
+    for (int j = 0; j < nmax; j += G) {
+        double p[G][3], v[G][NF];
+#pragma unroll
+        for (int k = 0; k < G; k++) {
+            const int q = (j + k < nn) ? c[k] : i;
+            p[k][0] = m.cell_center[3 * (size_t)q];
+            p[k][1] = m.cell_center[3 * (size_t)q + 1];
+            if (DIM == 3) p[k][2] = m.cell_center[3 * (size_t)q + 2];
+#pragma unroll
+            for (int f = 0; f < NF; f++) v[k][f] = a.w[f][q];
+        }
+#pragma unroll
+        for (int k = 0; k < G; k++) c[k] = (j + G + k < m.K) ? m.lsq_cells[(size_t)(j + G + k) * m.C + i] : 0;
+#pragma unroll
+        for (int k = 0; k < G; k++) {
+            if (j + k >= nn) continue;
+            const double jx = p[k][0] - cx, jy = p[k][1] - cy, jz = DIM == 3 ? p[k][2] - cz : 0.;
+            lsq_accumulate<DIM>(I, J[0], jx, jy, jz, v[k][0] - wi[0]);
+#pragma unroll
+            for (int f = 1; f < NF; f++) {
+                const double dw = v[k][f] - wi[f];
+                J[f][0] += (jx * dw);
+                J[f][1] += (jy * dw);
+                if (DIM == 3) J[f][2] += (jz * dw);
+            }
+        }
+    }
+    for (int j = 0; j < gmax; j++) {
+        if (j >= ng) continue;
+        const int q = m.lsq_ghosts[(size_t)j * m.C + i];
+        const double *g = m.face_ghost + 3 * (size_t)q;
+        const double jx = g[0] - cx, jy = g[1] - cy, jz = DIM == 3 ? g[2] - cz : 0.;
+        lsq_accumulate<DIM>(I, J[0], jx, jy, jz, a.ghost[0][q] - wi[0]);
+#pragma unroll
+        for (int f = 1; f < NF; f++) {
+            const double dw = a.ghost[f][q] - wi[f];
+            J[f][0] += (jx * dw);
+            J[f][1] += (jy * dw);
+            if (DIM == 3) J[f][2] += (jz * dw);
+        }
+    }
+}
+
+template <int DIM, int NF, int MF>
+__global__ void __launch_bounds__(kBlock) k_gradient_limited(Mesh m, GradArgs<NF> a)
+{
+    const int i = xcd_block() * blockDim.x + threadIdx.x;
+    if (i >= m.C) return;
+    const double cx = m.cell_center[3 * (size_t)i], cy = m.cell_center[3 * (size_t)i + 1],
+                 cz = m.cell_center[3 * (size_t)i + 2];
+    const int nf = m.cell_nfaces[i];
+    int fid[MF];
+#pragma unroll
+    for (int s = 0; s < MF; s++) {
+        const int f = m.cell_faces[(size_t)s * m.C + i];
+        fid[s] = (s < nf) ? f : -1;
+    }
+    double wi[NF], I[6] = {0., 0., 0., 0., 0., 0.}, J[NF][3];
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+        wi[f] = a.w[f][i];
+        J[f][0] = J[f][1] = J[f][2] = 0.;
+    }
+    stencil_sums<DIM, NF>(m, a, i, cx, cy, cz, wi, I, J);
+    // the faces: what lies on both sides, and the face's centre
+    int2 ab[MF];
+    int nm[MF];
+    double r[MF][3];
+#pragma unroll
+    for (int s = 0; s < MF; s++) {
+        const size_t f = fid[s] >= 0 ? fid[s] : 0;
+        ab[s] = reinterpret_cast<const int2 *>(m.face_cells)[f];
+        nm[s] = m.face_name[f];
+        r[s][0] = m.face_center[3 * f] - cx;
+        r[s][1] = m.face_center[3 * f + 1] - cy;
+        if (DIM == 3) r[s][2] = m.face_center[3 * f + 2] - cz;
+    }
+    const double eps = (DIM == 2) ? 1e-8 : 1e-10;
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+        double wl[MF], wr[MF];
+#pragma unroll
+        for (int s = 0; s < MF; s++) {
+            const bool has = fid[s] >= 0, inner = nm[s] == 0 || nm[s] > 10;
+            wl[s] = a.w[f][has ? ab[s].x : i];
+            const double *src = (has && !inner) ? a.ghost[f] : a.w[f];
+            wr[s] = src[!has ? i : inner ? ab[s].y : fid[s]];
+        }
+        double gx, gy, gz;
+        lsq_solve<DIM>(I, J[f], gx, gy, gz);
+        double hi = wi[f], lo = wi[f];
+#pragma unroll
+        for (int s = 0; s < MF; s++)
+            if (fid[s] >= 0) {
+                hi = pmax(pmax(hi, wl[s]), wr[s]);
+                lo = pmin(pmin(lo, wl[s]), wr[s]);
+            }
+        double psi = 1., psi_ij = 1.;
+#pragma unroll
+        for (int s = 0; s < MF; s++)
+            if (fid[s] >= 0) {
+                const double delta2 =
+                    (DIM == 2) ? (gx * r[s][0] + gy * r[s][1]) : (gx * r[s][0] + gy * r[s][1] + gz * r[s][2]);
+                if (fabs(delta2) < eps) {
+                    psi_ij = 1.;
+                } else {
+                    if (delta2 > 0.) psi_ij = pmin(1., (hi - wi[f]) / delta2);
+                    if (delta2 < 0.) psi_ij = pmin(1., (lo - wi[f]) / delta2);
+                }
+                psi = pmin(psi, psi_ij);
+            }
+        a.gx[f][i] = gx;
+        a.gy[f][i] = gy;
+        a.gz[f][i] = gz;
+        a.psi[f][i] = psi;
+    }
+}
+
+template <int NF>
+static int gradient_limited(const mfv_mesh *m, const GradArgs<NF> &a, hipStream_t st)
+{
+    const Mesh k = to_kernel(m);
+    const dim3 g(grid_for(m->nb_cells)), b(kBlock);
+#define LAUNCH(D, M) hipLaunchKernelGGL((k_gradient_limited<D, NF, M>), g, b, 0, st, k, a)
+    if (m->dim == 2) {
+        if (m->max_cell_faces <= 3) LAUNCH(2, 3);
+        else if (m->max_cell_faces == 4) LAUNCH(2, 4);
+        else LAUNCH(2, 8);
+    } else {
+        if (m->max_cell_faces <= 4) LAUNCH(3, 4);
+        else LAUNCH(3, 8);
+    }
+#undef LAUNCH
+    return check_launch("k_gradient_limited");
+}
+
+extern "C" int mfv_cell_gradient_limited(const mfv_mesh *m, int nfields, const mfv_gradient_fields *f, void *stream)
+{
+    if (int rc = validate_mesh(m, 1, 0, 0)) return rc;
+    MFV_REQUIRE(nfields == 1 || nfields == 2, "nfields must be 1 or 2, got %d", nfields);
+    MFV_REQUIRE(f, "fields missing");
+    for (int k = 0; k < nfields; k++)
+        MFV_REQUIRE(f[k].w && f[k].ghost && f[k].gx && f[k].gy && f[k].gz && f[k].psi, "NULL array");
+    if (m->nb_cells == 0) return MFV_OK;
+    if (nfields == 1)
+        return gradient_limited<1>(m, GradArgs<1>{{f->w}, {f->ghost}, {f->gx}, {f->gy}, {f->gz}, {f->psi}},
+                                   as_stream(stream));
+    return gradient_limited<2>(m,
+                               GradArgs<2>{{f[0].w, f[1].w}, {f[0].ghost, f[1].ghost}, {f[0].gx, f[1].gx},
+                                           {f[0].gy, f[1].gy}, {f[0].gz, f[1].gz}, {f[0].psi, f[1].psi}},
+                               as_stream(stream));
+}
+
+// ---------------------------------------------------------------------------------------------
 // dt reduction helpers
 
 __global__ void k_dt_reset(double *dt) { dt[0] = 1e6; }

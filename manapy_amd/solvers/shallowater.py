@@ -21,7 +21,7 @@ import numpy as np
 from .. import _lib
 from ..base import Struct, make_get_conf, process_conf
 from ..device import stream_ptr, SwPacked
-from ..variable import Variable, fill_ghosts
+from ..variable import Variable, cell_gradients, fill_ghosts
 from ._common import DeviceClock
 
 
@@ -143,8 +143,7 @@ class ShallowWaterSolver(object):
         """``system.py:162-178``: gradients (+ limiter) of h and hc at order 2, then
         explicitscheme_convective_SW."""
         if self.order == 2:
-            self.h.compute_cell_gradient()
-            self.hc.compute_cell_gradient()
+            cell_gradients(self.domain, (self.h, self.hc))
         v = (self.h, self.hu, self.hv, self.hc, self.Z)
         _lib.call('mfv_explicitscheme_convective_sw', self._m.ptr, *[x.convective.data_ptr() for x in v],
                   *[x.cell.data_ptr() for x in v], *[x.ghost.data_ptr() for x in v], self.h.gradcellx.data_ptr(),

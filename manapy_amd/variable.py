@@ -37,6 +37,16 @@ def fill_ghosts(domain, pairs, cache=None):
     _lib.call('mfv_ghost_values', domain.device_mesh.ptr, segs, len(pairs), stream_ptr())
 
 
+def cell_gradients(domain, variables):
+    """Least-squares gradient then Barth-Jespersen limiter of one or two Variables in one launch."""
+    dm = domain.device_mesh
+    dm.ensure_lsq()
+    f = (_lib.MfvGradientFields * len(variables))(*[
+        (v.cell.data_ptr(), v.ghost.data_ptr(), v.gradcellx.data_ptr(), v.gradcelly.data_ptr(),
+         v.gradcellz.data_ptr(), v.psi.data_ptr()) for v in variables])
+    _lib.call('mfv_cell_gradient_limited', dm.ptr, len(variables), f, stream_ptr())
+
+
 class Boundary(object):
     """One boundary location of a Variable (``boundary/bc.py:8-103``)."""
 
@@ -233,13 +243,7 @@ class Variable(object):
 
     def compute_cell_gradient(self):
         """``ast/core.py:442-478``: least-squares gradient then Barth-Jespersen limiter."""
-        dm = self._domain.device_mesh
-        dm.ensure_lsq()
-        s = stream_ptr()
-        _lib.call('mfv_cell_gradient', dm.ptr, self.cell.data_ptr(), self.ghost.data_ptr(), self.gradcellx.data_ptr(),
-                  self.gradcelly.data_ptr(), self.gradcellz.data_ptr(), s)
-        _lib.call('mfv_barthlimiter', dm.ptr, self.cell.data_ptr(), self.ghost.data_ptr(), self.gradcellx.data_ptr(),
-                  self.gradcelly.data_ptr(), self.gradcellz.data_ptr(), self.psi.data_ptr(), s)
+        cell_gradients(self._domain, (self,))
 
     def norml2(self, exact, order=None):
         """``ast/core.py:500-515``: ||(w - exact) vol||_p / ||exact vol||_p (on the device)."""
