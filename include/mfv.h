@@ -234,6 +234,16 @@ typedef struct mfv_sw_packed {
 int mfv_sw_pack(const mfv_mesh *m, const mfv_sw_packed *p, const double *h, const double *hu,
                 const double *hv, const double *Z, const double *zgrad, int order, void *stream);
 
+/* mfv_sw_pack from fields in another cell order (cell i of this mesh is perm[i] of theirs), into
+ * p->cellrec and a second record buffer cellrec_b alike. Reads Z and zgrad [3][C] there too. */
+int mfv_sw_load(const mfv_mesh *m, const mfv_sw_packed *p, double *cellrec_b, const int64_t *perm,
+                const double *h, const double *hu, const double *hv, const double *Z, const double *zgrad,
+                int order, void *stream);
+
+/* h, hu, hv [perm[i]] = the fields of record i. */
+int mfv_sw_store(const mfv_mesh *m, const double *cellrec, const int64_t *perm, double *h, double *hu,
+                 double *hv, void *stream);
+
 /* Copies h, hu, hv out of cellrec. */
 int mfv_sw_unpack(const mfv_mesh *m, const mfv_sw_packed *p, double *h, double *hu, double *hv,
                   void *stream);
@@ -345,6 +355,13 @@ void mfv_sw_tiles_host_free(mfv_sw_tiles_host *t);
 int mfv_sw_step_packed_tiled(const mfv_mesh *m, const mfv_sw_packed *p, const mfv_sw_tiles *t,
                              double *cellrec_out, double grav, double cfl, int order, double *dt_ring,
                              int step, void *stream);
+
+/* nsteps of mfv_sw_step_packed_tiled (ring steps 0 .. nsteps - 1), alternating between p->cellrec
+ * and cellrec_b (the same static fields); the result is in p->cellrec for even nsteps, else in
+ * cellrec_b. Same bits. */
+int mfv_sw_run_packed_tiled(const mfv_mesh *m, const mfv_sw_packed *p, const mfv_sw_tiles *t,
+                            double *cellrec_b, double grav, double cfl, int order, double *dt_ring,
+                            int nsteps, void *stream);
 
 /* mfv_sw_step_packed_tiled with no device allocation of its own. No counterpart in the
  * reference: it is for callers that cannot allocate (code under HIP graph capture, tight

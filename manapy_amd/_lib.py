@@ -233,6 +233,9 @@ _SIGNATURES = {
     'mfv_term_wind_sw': [c_int, P, P, P, P, P],
     'mfv_sw_pack': [MESH_P, SWP_P, P, P, P, P, P, c_int, P],
     'mfv_sw_unpack': [MESH_P, SWP_P, P, P, P, P],
+    'mfv_sw_load': [MESH_P, SWP_P, P, P, P, P, P, P, P, c_int, P],
+    'mfv_sw_store': [MESH_P, P, P, P, P, P, P],
+    'mfv_sw_run_packed_tiled': [MESH_P, SWP_P, SWT_P, P, c_double, c_double, c_int, P, c_int, P],
     'mfv_sw_recon': [MESH_P, SWP_P, c_int, P],
     'mfv_sw_flux_packed': [MESH_P, SWP_P, c_double, c_double, P, c_int, P],
     'mfv_sw_pack_mixed': [MESH_P, SWM_P, P, P, P, P, P, c_int, P],

@@ -172,6 +172,39 @@ __device__ __forceinline__ void ring_advance(const DtRing &r)
     }
 }
 
+// The dt of a fused step. n == 0: the ring's current slot. n > 0: min(1e6, part[0..n)) over the
+// partials that the previous step's waves left, folded by every wave for itself (the minimum of
+// a set does not depend on the order), so that step needs no k_dt_finish launch before it; the
+// first wave of the grid then writes the slot and the ring's other entries. A wave reads n / 64
+// values a lane: against the 5 us of a launch of its own this pays up to kFoldMax partials.
+constexpr int kFoldMax = 1024;
+__device__ __forceinline__ double step_dt(const DtRing &r, const double *__restrict__ part, int n)
+{
+    if (n == 0) {
+        ring_advance(r);
+        return r.cur[0];
+    }
+    double m = 1e6;
+    for (int j = threadIdx.x & 63; j < n; j += 256) {
+        double v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = part[min(j + 64 * k, n - 1)];
+#pragma unroll
+        for (int k = 0; k < 4; k++) m = (v[k] < m) ? v[k] : m;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const double o = __shfl_xor(m, off, 64);
+        m = (o < m) ? o : m;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        const_cast<double *>(r.cur)[0] = m;
+        r.spare[0] = 1e6;
+        r.time[0] += m;
+    }
+    return m;
+}
+
 // Mesh descriptor passed by value to kernels.
 struct Mesh {
     int C, F, MF, K, G;

@@ -484,6 +484,73 @@ __global__ void __launch_bounds__(kBlock) k_sw_pack_zf_across(Mesh m, mfv_sw_pac
     }
 }
 
+// The records of both buffers and both bathymetry values of every face slot from fields in
+// another cell order (cell i of this mesh is perm[i] of theirs). One pass: the neighbour's z_f is
+// formed again from its own Z, gradient and offset (the same expression) instead of being read
+// back after a second launch (with the fused step that it feeds, 10 steps at 1M cells take 1302 us,
+// 2512 us before; the two launches alone were 182 us, the gathers into this order 45 us).
+template <int MF>
+__global__ void __launch_bounds__(kBlock) k_sw_load(Mesh m, mfv_sw_packed p, double *__restrict__ rec_b,
+                                                    const int64_t *__restrict__ perm, const double *__restrict__ h,
+                                                    const double *__restrict__ hu, const double *__restrict__ hv,
+                                                    const double *__restrict__ Z, const double *__restrict__ zgrad,
+                                                    double om)
+{
+    const int i = xcd_block() * blockDim.x + threadIdx.x;
+    if (i >= m.C) return;
+    const size_t C = m.C;
+    const size_t q = (size_t)perm[i];
+    const int nf = m.cell_nfaces[i];
+    const double zi = Z[q], hi = h[q], zx = zgrad[q], zy = zgrad[C + q];
+    const double2 r0 = make_double2(m.cell_center[3 * (size_t)i], m.cell_center[3 * (size_t)i + 1]),
+                  r1 = make_double2(hi + zi, hu[q]), r2 = make_double2(hv[q], hi),
+                  r3 = make_double2(zi, m.cell_volume[i]);
+    double2 *a = reinterpret_cast<double2 *>(p.cellrec + 8 * (size_t)i),
+            *b = reinterpret_cast<double2 *>(rec_b + 8 * (size_t)i);
+    a[0] = b[0] = r0;
+    a[1] = b[1] = r1;
+    a[2] = b[2] = r2;
+    a[3] = b[3] = r3;
+    int code[MF];
+    double2 own[MF], nb[MF];
+#pragma unroll
+    for (int s = 0; s < MF; s++) {
+        const int c = p.nbr[(size_t)s * C + i];
+        code[s] = (s < nf) ? c : -1;
+    }
+#pragma unroll
+    for (int s = 0; s < MF; s++) {
+        own[s] = *reinterpret_cast<const double2 *>(p.cfrec + 4 * (MF * (size_t)i + s));
+        const int j = code[s] >= 0 ? code[s] >> 3 : i, k = code[s] >= 0 ? (code[s] >> 1) & 3 : s;
+        nb[s] = *reinterpret_cast<const double2 *>(p.cfrec + 4 * (MF * (size_t)j + k));
+    }
+#pragma unroll
+    for (int s = 0; s < MF; s++) {
+        if (s >= nf) continue;
+        const double zo = zi + om * (zx * own[s].x + zy * own[s].y);
+        double zn = zo;
+        if (code[s] >= 0) {
+            const size_t j = (size_t)perm[code[s] >> 3];
+            zn = Z[j] + om * (zgrad[j] * nb[s].x + zgrad[C + j] * nb[s].y);
+        }
+        reinterpret_cast<double2 *>(p.cfrec + 4 * (MF * (size_t)i + s))[1] = make_double2(zo, zn);
+    }
+}
+
+__global__ void __launch_bounds__(kBlock) k_sw_store(int C, const double *__restrict__ cellrec,
+                                                     const int64_t *__restrict__ perm, double *__restrict__ h,
+                                                     double *__restrict__ hu, double *__restrict__ hv)
+{
+    const int i = xcd_block() * blockDim.x + threadIdx.x;
+    if (i >= C) return;
+    const double2 *r = reinterpret_cast<const double2 *>(cellrec + 8 * (size_t)i);
+    const double2 b = r[1], c = r[2];
+    const size_t q = (size_t)perm[i];
+    hu[q] = b.y;
+    hv[q] = c.x;
+    h[q] = c.y;
+}
+
 template <int MF>
 __global__ void __launch_bounds__(kBlock) k_sw_unpack(int C, const double *__restrict__ cellrec,
                                                        double *__restrict__ h, double *__restrict__ hu,
@@ -984,7 +1051,8 @@ inline size_t packed_tiled_lds(int max_ext, int max_items, int MF)
 template <int MF, int T, int KMAX>
 __global__ void __launch_bounds__(T) k_sw_step_packed_tiled(Mesh m, mfv_sw_packed p, TilesP t,
                                                             double *__restrict__ rec_out, double om, double g,
-                                                            double cfl, DtRing ring, double *__restrict__ dtpart)
+                                                            double cfl, DtRing ring, const double *__restrict__ fold,
+                                                            int nfold, double *__restrict__ dtpart)
 {
     extern __shared__ double2 lds2[];
     const int E = (t.E + 1) & ~1;
@@ -997,7 +1065,7 @@ __global__ void __launch_bounds__(T) k_sw_step_packed_tiled(Mesh m, mfv_sw_packe
     const int e0 = t.eptr[tile], ne = t.eptr[tile + 1] - e0;
     double *f_v = reinterpret_cast<double *>(f_eu + MF * (nc + nh));  // [items][MF]
     const size_t r0 = t.iptr[tile];
-    ring_advance(ring);
+    const double dt = step_dt(ring, fold, nfold);
     for (int e = threadIdx.x; e < nc + ne; e += 2 * T) {  // two cells per pass: one latency for both
         const int2 c = tile_ext_pair(t.ext, c0, nc, e0, ne, e, T);
         const int eb = (e + T < nc + ne) ? e + T : e;
@@ -1059,8 +1127,7 @@ __global__ void __launch_bounds__(T) k_sw_step_packed_tiled(Mesh m, mfv_sw_packe
             fv.zn[s] = zp[s].y;
         }
         const CellVals cv{s_eu[q].y, s_v[q], hZv[0], hZv[1], hZv[2]};
-        dloc = sw_flux_packed_core<MF>(p, i, cv, rec_out + 8 * (size_t)i, fv, code_of, nf_q, ord_q, g, cfl,
-                                       ring.cur[0]);
+        dloc = sw_flux_packed_core<MF>(p, i, cv, rec_out + 8 * (size_t)i, fv, code_of, nf_q, ord_q, g, cfl, dt);
     }
     wave_min_part(dtpart, (size_t)c0 + q, dloc);
 }
@@ -1094,6 +1161,33 @@ extern "C" int mfv_sw_pack(const mfv_mesh *m, const mfv_sw_packed *p, const doub
     hipLaunchKernelGGL(tri ? k_sw_pack_zf_across<3> : k_sw_pack_zf_across<4>, dim3(grid_for(m->nb_cells)),
                        dim3(kBlock), 0, as_stream(stream), to_kernel(m), *p);
     return check_launch("k_sw_pack_zf_across");
+}
+
+extern "C" int mfv_sw_load(const mfv_mesh *m, const mfv_sw_packed *p, double *cellrec_b, const int64_t *perm,
+                           const double *h, const double *hu, const double *hv, const double *Z, const double *zgrad,
+                           int order, void *stream)
+{
+    if (int rc = validate_mesh(m, 0, 0, 0)) return rc;
+    if (int rc = check_packed(m, p)) return rc;
+    MFV_REQUIRE(m->dim == 2, "shallow water needs a 2D mesh");
+    MFV_REQUIRE(order == 1 || order == 2, "order must be 1 or 2");
+    MFV_REQUIRE(cellrec_b && cellrec_b != p->cellrec && perm && h && hu && hv && Z && zgrad, "NULL or aliased array");
+    if (m->nb_cells == 0) return MFV_OK;
+    auto k = m->max_cell_faces == 3 ? k_sw_load<3> : k_sw_load<4>;
+    hipLaunchKernelGGL(k, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream), to_kernel(m), *p, cellrec_b,
+                       perm, h, hu, hv, Z, zgrad, (double)(order - 1));
+    return check_launch("k_sw_load");
+}
+
+extern "C" int mfv_sw_store(const mfv_mesh *m, const double *cellrec, const int64_t *perm, double *h, double *hu,
+                            double *hv, void *stream)
+{
+    if (int rc = validate_mesh(m, 0, 0, 0)) return rc;
+    MFV_REQUIRE(cellrec && perm && h && hu && hv, "NULL array");
+    if (m->nb_cells == 0) return MFV_OK;
+    hipLaunchKernelGGL(k_sw_store, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream), m->nb_cells,
+                       cellrec, perm, h, hu, hv);
+    return check_launch("k_sw_store");
 }
 
 extern "C" int mfv_sw_unpack(const mfv_mesh *m, const mfv_sw_packed *p, double *h, double *hu, double *hv,
@@ -1142,23 +1236,32 @@ static int check_tiles_packed(const mfv_mesh *m, const mfv_sw_tiles *t)
 }
 
 template <int MF, int T>
-static void launch_packed_tiled(const mfv_mesh *m, const mfv_sw_packed *p, const mfv_sw_tiles *t, double *out,
-                                double om, double g, double cfl, DtRing r, double *part, hipStream_t st)
+static void launch_packed_tiled(const mfv_mesh *m, const mfv_sw_packed &p, const mfv_sw_tiles *t, double *out,
+                                double om, double g, double cfl, DtRing r, const double *fold, int nfold, double *part,
+                                hipStream_t st)
 {
     const TilesP tp{t->max_ext, t->tile_cell0, t->tile_ncells, t->tile_nhalo, t->ext_ptr, t->ext_cells,
                     t->item_ptr, t->lnbr, t->lst, t->lgh, t->lfn, t->nb_items};
     const size_t lds = packed_tiled_lds(t->max_ext, t->max_items, MF);
-    if (m->lsq_width <= 16)
-        hipLaunchKernelGGL((k_sw_step_packed_tiled<MF, T, 16>), dim3(t->nb_tiles), dim3(T), lds, st, to_kernel(m),
-                           *p, tp, out, om, g, cfl, r, part);
-    else
-        hipLaunchKernelGGL((k_sw_step_packed_tiled<MF, T, 0>), dim3(t->nb_tiles), dim3(T), lds, st, to_kernel(m),
-                           *p, tp, out, om, g, cfl, r, part);
+    auto k = m->lsq_width <= 16 ? k_sw_step_packed_tiled<MF, T, 16> : k_sw_step_packed_tiled<MF, T, 0>;
+    hipLaunchKernelGGL(k, dim3(t->nb_tiles), dim3(T), lds, st, to_kernel(m), p, tp, out, om, g, cfl, r, fold, nfold,
+                       part);
 }
 
-extern "C" int mfv_sw_step_packed_tiled(const mfv_mesh *m, const mfv_sw_packed *p, const mfv_sw_tiles *t,
-                                        double *cellrec_out, double grav, double cfl, int order, double *dt_ring_p,
-                                        int step, void *stream)
+// One step's launch (checked operands); fold, nfold: see step_dt.
+static int packed_tiled(const mfv_mesh *m, const mfv_sw_packed &p, const mfv_sw_tiles *t, double *out, double om,
+                        double g, double cfl, DtRing r, const double *fold, int nfold, double *part, hipStream_t st)
+{
+    const bool tri = m->max_cell_faces == 3;
+    auto k = t->tile_size == 128   ? (tri ? launch_packed_tiled<3, 128> : launch_packed_tiled<4, 128>)
+             : t->tile_size == 256 ? (tri ? launch_packed_tiled<3, 256> : launch_packed_tiled<4, 256>)
+                                   : (tri ? launch_packed_tiled<3, 512> : launch_packed_tiled<4, 512>);
+    k(m, p, t, out, om, g, cfl, r, fold, nfold, part, st);
+    return check_launch("k_sw_step_packed_tiled");
+}
+
+static int check_step_packed_tiled(const mfv_mesh *m, const mfv_sw_packed *p, const mfv_sw_tiles *t,
+                                   const double *cellrec_out, int order, const double *dt_ring_p)
 {
     if (int rc = validate_mesh(m, 1, 0, 0)) return rc;
     if (int rc = check_packed(m, p)) return rc;
@@ -1166,30 +1269,54 @@ extern "C" int mfv_sw_step_packed_tiled(const mfv_mesh *m, const mfv_sw_packed *
     MFV_REQUIRE(m->dim == 2, "shallow water needs a 2D mesh");
     MFV_REQUIRE(order == 1 || order == 2, "order must be 1 or 2");
     MFV_REQUIRE(dt_ring_p && cellrec_out && cellrec_out != p->cellrec, "cellrec_out must be a second record buffer");
+    return MFV_OK;
+}
+
+extern "C" int mfv_sw_step_packed_tiled(const mfv_mesh *m, const mfv_sw_packed *p, const mfv_sw_tiles *t,
+                                        double *cellrec_out, double grav, double cfl, int order, double *dt_ring_p,
+                                        int step, void *stream)
+{
+    if (int rc = check_step_packed_tiled(m, p, t, cellrec_out, order, dt_ring_p)) return rc;
     if (m->nb_cells == 0) return MFV_OK;
     DtRing r = dt_ring(dt_ring_p, step);
     const size_t nw = ((size_t)m->nb_cells + 63) / 64;
-    double *part = dt_scratch(nw, as_stream(stream));
-    if (!part) return MFV_ENOMEM;
-    const double om = (double)(order - 1);
     hipStream_t st = as_stream(stream);
-    const bool tri = m->max_cell_faces == 3;
-    switch (t->tile_size) {
-    case 128:
-        if (tri) launch_packed_tiled<3, 128>(m, p, t, cellrec_out, om, grav, cfl, r, part, st);
-        else launch_packed_tiled<4, 128>(m, p, t, cellrec_out, om, grav, cfl, r, part, st);
-        break;
-    case 256:
-        if (tri) launch_packed_tiled<3, 256>(m, p, t, cellrec_out, om, grav, cfl, r, part, st);
-        else launch_packed_tiled<4, 256>(m, p, t, cellrec_out, om, grav, cfl, r, part, st);
-        break;
-    default:
-        if (tri) launch_packed_tiled<3, 512>(m, p, t, cellrec_out, om, grav, cfl, r, part, st);
-        else launch_packed_tiled<4, 512>(m, p, t, cellrec_out, om, grav, cfl, r, part, st);
-        break;
-    }
-    if (int rc = check_launch("k_sw_step_packed_tiled")) return rc;
+    double *part = dt_scratch(nw, st);
+    if (!part) return MFV_ENOMEM;
+    if (int rc = packed_tiled(m, *p, t, cellrec_out, (double)(order - 1), grav, cfl, r, nullptr, 0, part, st)) return rc;
     return dt_finish(part, nw, r.next, st);
+}
+
+// nsteps steps from p->cellrec, alternating with cellrec_b. Up to kFoldMax partials every step
+// folds its predecessor's for itself (step_dt), so a step is one launch: 30 steps at 5k cells 668 ->
+// 401 us, with k_sw_recon, k_sw_flux_packed and k_dt_finish replaced by it.
+extern "C" int mfv_sw_run_packed_tiled(const mfv_mesh *m, const mfv_sw_packed *p, const mfv_sw_tiles *t,
+                                       double *cellrec_b, double grav, double cfl, int order, double *dt_ring_p,
+                                       int nsteps, void *stream)
+{
+    if (int rc = check_step_packed_tiled(m, p, t, cellrec_b, order, dt_ring_p)) return rc;
+    MFV_REQUIRE(nsteps >= 0, "nsteps < 0");
+    if (m->nb_cells == 0 || nsteps == 0) return MFV_OK;
+    const size_t nw = ((size_t)m->nb_cells + 63) / 64;
+    const bool fold = nw <= (size_t)kFoldMax;
+    hipStream_t st = as_stream(stream);
+    double *part = dt_scratch(fold ? 2 * nw : nw, st);
+    if (!part) return MFV_ENOMEM;
+    mfv_sw_packed q = *p;
+    double *out = cellrec_b;
+    for (int k = 0; k < nsteps; k++) {
+        const DtRing r = dt_ring(dt_ring_p, k);
+        double *mine = part + (fold && (k & 1) ? nw : 0), *last = part + (fold && !(k & 1) ? nw : 0);
+        if (int rc = packed_tiled(m, q, t, out, (double)(order - 1), grav, cfl, r, last, fold && k > 0 ? (int)nw : 0,
+                                  mine, st))
+            return rc;
+        if (!fold || k == nsteps - 1)
+            if (int rc = dt_finish(mine, nw, r.next, st)) return rc;
+        double *in = q.cellrec;
+        q.cellrec = out;
+        out = in;
+    }
+    return MFV_OK;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1239,35 +1366,14 @@ extern "C" int mfv_sw_step_packed_tiled_noalloc(const mfv_mesh *m, const mfv_sw_
                 "%d cells need %zu dt partials: the allocation-free step holds at most %d (%d cells); use "
                 "mfv_sw_step_packed_tiled",
                 m->nb_cells, ((size_t)m->nb_cells + 63) / 64, MFV_NOALLOC_MAX_WAVES, 64 * MFV_NOALLOC_MAX_WAVES);
-    if (int rc = validate_mesh(m, 1, 0, 0)) return rc;
-    if (int rc = check_packed(m, p)) return rc;
-    if (int rc = check_tiles_packed(m, t)) return rc;
-    MFV_REQUIRE(m->dim == 2, "shallow water needs a 2D mesh");
-    MFV_REQUIRE(order == 1 || order == 2, "order must be 1 or 2");
-    MFV_REQUIRE(dt_ring_p && cellrec_out && cellrec_out != p->cellrec, "cellrec_out must be a second record buffer");
+    if (int rc = check_step_packed_tiled(m, p, t, cellrec_out, order, dt_ring_p)) return rc;
     if (m->nb_cells == 0) return MFV_OK;
     double *part = noalloc_partials();
     if (!part) return MFV_EHIP;
     DtRing r = dt_ring(dt_ring_p, step);
     const size_t nw = ((size_t)m->nb_cells + 63) / 64;
-    const double om = (double)(order - 1);
     hipStream_t st = as_stream(stream);
-    const bool tri = m->max_cell_faces == 3;
-    switch (t->tile_size) {
-    case 128:
-        if (tri) launch_packed_tiled<3, 128>(m, p, t, cellrec_out, om, grav, cfl, r, part, st);
-        else launch_packed_tiled<4, 128>(m, p, t, cellrec_out, om, grav, cfl, r, part, st);
-        break;
-    case 256:
-        if (tri) launch_packed_tiled<3, 256>(m, p, t, cellrec_out, om, grav, cfl, r, part, st);
-        else launch_packed_tiled<4, 256>(m, p, t, cellrec_out, om, grav, cfl, r, part, st);
-        break;
-    default:
-        if (tri) launch_packed_tiled<3, 512>(m, p, t, cellrec_out, om, grav, cfl, r, part, st);
-        else launch_packed_tiled<4, 512>(m, p, t, cellrec_out, om, grav, cfl, r, part, st);
-        break;
-    }
-    if (int rc = check_launch("k_sw_step_packed_tiled")) return rc;
+    if (int rc = packed_tiled(m, *p, t, cellrec_out, (double)(order - 1), grav, cfl, r, nullptr, 0, part, st)) return rc;
     return dt_finish(part, nw, r.next, st);
 }
 

@@ -214,26 +214,57 @@ def sw_packed_layout(domain):
     return {'nbr': nbr, 'cfrec': cfrec, 'cfgeo': cfgeo, 'order': order.astype(np.uint8), 'MF': MF}
 
 
-class SwPacked(object):
-    """Device tables and records of the packed shallow-water path for a DeviceMesh."""
+# Cells below which ShallowWaterSolver.run takes blocks of 128 threads (tiles of one wave's cells:
+# more blocks on a mesh that leaves the chip idle): 30 steps take 417 us against 424 us with 256
+# threads at 1k cells, 414 against 425 us at 5k, 471 against 440 us at 26k, and 256 threads lead from
+# there on (3.94 against 3.42 ms at 1M).
+SW_RUN_SMALL = 16384
+
+
+def sw_packed_lds(host):
+    """LDS bytes a block of the fused float64 step takes on a tiles layout."""
+    return ((host['max_ext'] + 1) // 2 * 2) * 40 + host['max_items'] * host['MF'] * 24
+
+
+class SwPackedTables(object):
+    """What the packed shallow-water path needs of a mesh alone: geometry, neighbour codes,
+    residual orders, and the tiles per block size (built on first use)."""
 
     def __init__(self, dmesh):
         import torch
         host = sw_packed_layout(dmesh.domain)
-        C = dmesh.C
-        MF = host['MF']
-        dev = dmesh.device
+        self.device = dmesh.device
+        self.MF = host['MF']
+        self.C = dmesh.C
         self.nbr_host = host['nbr']
         self._lsq = dmesh.host
         self._tiles = {}
+        for k in ('cfrec', 'cfgeo', 'nbr', 'order'):
+            setattr(self, k, torch.as_tensor(host[k], device=dmesh.device))
+
+    def tiles(self, T):
+        if T not in self._tiles:
+            self._tiles[T] = SwTiles(sw_tiles_native(self.nbr_host, self.C, T, T, self._lsq), self.device, stage=True)
+        return self._tiles[T]
+
+
+class SwPacked(object):
+    """Device tables and records of the packed shallow-water path for a DeviceMesh. ``tables``: a
+    SwPackedTables of the same mesh to share (its cfrec, which also takes the bathymetry, is
+    copied)."""
+
+    def __init__(self, dmesh, tables=None):
+        import torch
+        shared = tables is not None
+        self.tables = tables if shared else SwPackedTables(dmesh)
+        C, MF = dmesh.C, self.tables.MF
+        dev = dmesh.device
         self.cellrec2 = None  # second record buffer of the fused tiled step (on first use)
         self._rec_synced = None
         self.cellrec = torch.zeros((C, 8), dtype=torch.float64, device=dev)
         self.facerec = torch.zeros((C, MF, 4), dtype=torch.float64, device=dev)
-        self.cfrec = torch.as_tensor(host['cfrec'], device=dev)
-        self.cfgeo = torch.as_tensor(host['cfgeo'], device=dev)
-        self.nbr = torch.as_tensor(host['nbr'], device=dev)
-        self.order = torch.as_tensor(host['order'], device=dev)
+        self.cfrec = self.tables.cfrec.clone() if shared else self.tables.cfrec
+        self.cfgeo, self.nbr, self.order = self.tables.cfgeo, self.tables.nbr, self.tables.order
         d = _lib.MfvSwPacked()
         d.nb_cells = C
         d.max_cell_faces = MF
@@ -257,14 +288,37 @@ class SwPacked(object):
 
     def tiles(self, T=128):
         """Tiles of the fused float64 step for blocks of T threads (built on first use)."""
-        if T not in self._tiles:
-            self._tiles[T] = SwTiles(sw_tiles_native(self.nbr_host, self.desc.nb_cells, T, T, self._lsq),
-                                     self.cellrec.device, stage=True)
-        return self._tiles[T]
+        return self.tables.tiles(T)
+
+    def second_buffer(self):
+        if self.cellrec2 is None:
+            import torch
+            self.cellrec2 = torch.empty_like(self.cellrec)
+        return self.cellrec2
+
+    def load(self, dmesh, perm, h, hu, hv, Z, zgrad, order, stream=None):
+        """mfv_sw_load: both record buffers from fields in the order ``perm`` indexes."""
+        _lib.call('mfv_sw_load', dmesh.ptr, self.ptr, self.second_buffer().data_ptr(), perm.data_ptr(), h.data_ptr(),
+                  hu.data_ptr(), hv.data_ptr(), Z.data_ptr(), zgrad.data_ptr(), int(order),
+                  stream if stream is not None else stream_ptr())
+        self._rec_synced = self.cellrec
+
+    def run_tiled(self, dmesh, grav, cfl, order, ring, nsteps, T, stream=None):
+        """nsteps fused float64 steps after load() (mfv_sw_run_packed_tiled); the result is the
+        current record buffer."""
+        _lib.call('mfv_sw_run_packed_tiled', dmesh.ptr, self.ptr, self.tiles(T).ptr, self.cellrec2.data_ptr(),
+                  float(grav), float(cfl), int(order), ring.data_ptr(), int(nsteps),
+                  stream if stream is not None else stream_ptr())
+        if nsteps % 2 == 1:
+            self._swap()
+
+    def _swap(self):
+        self.cellrec, self.cellrec2 = self.cellrec2, self.cellrec
+        self.desc.cellrec = self.cellrec.data_ptr()
+        self._rec_synced = self.cellrec
 
     def lds_bytes(self, T=128):
-        h = self.tiles(T).host
-        return ((h['max_ext'] + 1) // 2 * 2) * 40 + h['max_items'] * h['MF'] * 24
+        return sw_packed_lds(self.tiles(T).host)
 
     def step_tiled(self, dmesh, grav, cfl, order, ring, step, T=128, stream=None, noalloc=False):
         """One fused float64 step: reads the current record buffer, writes the other, swaps
@@ -272,17 +326,12 @@ class SwPacked(object):
         pack(); the static fields change only there. noalloc: the entry point that allocates
         nothing (mfv_sw_step_packed_tiled_noalloc; same bits)."""
         if self.cellrec2 is None or self._rec_synced is not self.cellrec:
-            if self.cellrec2 is None:
-                import torch
-                self.cellrec2 = torch.empty_like(self.cellrec)
-            self.cellrec2.copy_(self.cellrec)
+            self.second_buffer().copy_(self.cellrec)
         _lib.call('mfv_sw_step_packed_tiled_noalloc' if noalloc else 'mfv_sw_step_packed_tiled', dmesh.ptr, self.ptr,
                   self.tiles(T).ptr, self.cellrec2.data_ptr(),
                   float(grav), float(cfl), int(order), ring.data_ptr(), int(step),
                   stream if stream is not None else stream_ptr())
-        self.cellrec, self.cellrec2 = self.cellrec2, self.cellrec
-        self.desc.cellrec = self.cellrec.data_ptr()
-        self._rec_synced = self.cellrec
+        self._swap()
 
 
 def sw_tiles_native(nbr, C, T, N, lsq, ranges=None):
@@ -707,6 +756,37 @@ class Euler32(object):
                   a.data_ptr(), b.data_ptr(), float(gamma), float(cfl), int(quirk), ring.data_ptr(), int(step),
                   self.cons.data_ptr() if sums else None, stream if stream is not None else stream_ptr())
         self.k += 1
+
+
+class SwRunMesh(object):
+    """A 2D mesh as ShallowWaterSolver.run takes it: in Hilbert-curve cell order (a relabelling:
+    same bits), with the packed tables, and the block size of the fused step."""
+
+    def __init__(self, dmesh):
+        import torch
+        from .renumber import renumbered
+        r = renumbered(dmesh.domain)
+        self.mesh = DeviceMesh(r, lsq=True, device=dmesh.device)
+        self.perm = torch.as_tensor(r.perm, device=dmesh.device)
+        assert self.perm.dtype == torch.int64
+        self.tables = SwPackedTables(self.mesh)
+        self._block = None
+
+    def block(self):
+        """Threads a block of the fused step, or 0 where the stencils do not fit a tile (the tables'
+        8-bit counts, the block's LDS): then the step takes its two kernels."""
+        if self._block is None:
+            T = 0
+            for cand in ((128, 256) if self.mesh.C < SW_RUN_SMALL else (256, 128)):
+                try:
+                    h = self.tables.tiles(cand).host
+                except _lib.MfvError:
+                    continue
+                if sw_packed_lds(h) <= 64 * 1024:
+                    T = cand
+                    break
+            self._block = T
+        return self._block
 
 
 class SwTiles(object):

@@ -11,8 +11,8 @@ Two numerical fluxes behind the reference's class, options and call sequence
   ``cells.cellfid`` in the source term; ``quirk=False`` uses the true face neighbours.
 * ``flux='rusanov'``: second-order MUSCL with least-squares gradients of eta, hu, hv, the
   Barth-Jespersen limiter, hydrostatic reconstruction (Audusse et al. 2004) and the
-  Rusanov flux, with walls (h Neumann, hu/hv nonslip). ``run`` fuses it into two kernels
-  per step on the packed layout.
+  Rusanov flux, with walls (h Neumann, hu/hv nonslip). ``run`` fuses it into one tiled kernel
+  per step on the packed layout (two where the stencils do not fit a tile).
 """
 import ctypes
 
@@ -248,31 +248,30 @@ class ShallowWaterSolver(object):
             return self._srnh_run(nsteps)
         if not self._zgrad_ready:
             self._bathymetry_gradient()
-        import torch
-        from ..device import DeviceMesh
-        from ..renumber import renumbered
+        from ..device import SwRunMesh
         m = self._m
         s = stream_ptr()
+        rm = m.__dict__.get('_sw_run')  # tables of the mesh alone, shared by its solvers
+        if rm is None:
+            rm = m._sw_run = SwRunMesh(m)
         if self._packed is None:
-            # the packed records live in Hilbert-curve cell order (a relabelling: same bits)
-            r = renumbered(self.domain)
-            self._rmesh = DeviceMesh(r, lsq=True, device=m.device)
-            self._perm = torch.as_tensor(r.perm, device=m.device)
-            self._packed = SwPacked(self._rmesh)
-        rm, p, perm = self._rmesh, self._packed, self._perm
-        ins = [x.index_select(0, perm) for x in (self.h.cell, self.hu.cell, self.hv.cell, self.Z.cell)]
-        zg = self._zgrad.index_select(1, perm).contiguous()
-        _lib.call('mfv_sw_pack', rm.ptr, p.ptr, *[x.data_ptr() for x in ins], zg.data_ptr(), self.order, s)
-        _lib.call('mfv_time_step_sw', m.ptr, self.h.cell.data_ptr(), self.hu.cell.data_ptr(), self.hv.cell.data_ptr(),
-                  self.cfl, self.grav, 0., 0., self._clock.dt0.data_ptr(), None, s)
+            self._packed = SwPacked(rm.mesh, rm.tables)
+        p, T = self._packed, rm.block()
+        fields = (self.h.cell, self.hu.cell, self.hv.cell)
+        p.load(rm.mesh, rm.perm, *fields, self.Z.cell, self._zgrad, self.order, s)
+        _lib.call('mfv_time_step_sw', m.ptr, *[x.data_ptr() for x in fields], self.cfl, self.grav, 0., 0.,
+                  self._clock.dt0.data_ptr(), None, s)
         self._clock.start()
-        for k in range(nsteps):
-            _lib.call('mfv_sw_recon', rm.ptr, p.ptr, self.order, s)
-            _lib.call('mfv_sw_flux_packed', rm.ptr, p.ptr, self.grav, self.cfl, self._clock.ring.data_ptr(), k, s)
-        _lib.call('mfv_sw_unpack', rm.ptr, p.ptr, ins[0].data_ptr(), ins[1].data_ptr(), ins[2].data_ptr(), s)
-        for var, x in zip((self.h, self.hu, self.hv), ins[:3]):
-            var.cell.index_copy_(0, perm, x)
-        del zg
+        nsteps = len(range(nsteps))
+        if T:
+            p.run_tiled(rm.mesh, self.grav, self.cfl, self.order, self._clock.ring, nsteps, T, s)
+        else:
+            for k in range(nsteps):
+                _lib.call('mfv_sw_recon', rm.mesh.ptr, p.ptr, self.order, s)
+                _lib.call('mfv_sw_flux_packed', rm.mesh.ptr, p.ptr, self.grav, self.cfl, self._clock.ring.data_ptr(),
+                          k, s)
+        _lib.call('mfv_sw_store', rm.mesh.ptr, p.cellrec.data_ptr(), rm.perm.data_ptr(),
+                  *[x.data_ptr() for x in fields], s)
         self._clock.step = nsteps
         if nsteps:
             self.dt = float(self._clock.ring[(nsteps - 1) % 3])
