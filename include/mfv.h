@@ -145,6 +145,15 @@ int mfv_advection_step(const mfv_mesh *m, const double *w_in, double *w_out, con
                        const double *v_face, const double *w_face, double cfl, int order,
                        double *dt_ring, int step, double *scratch, void *stream);
 
+/* nsteps of mfv_advection_step with the velocity and dt of the ring's current slot kept: the face
+ * velocities and the upwind cells are laid out once in workspace (mfv_advection_run_size doubles).
+ * Alternates between w_a (the start) and w_b; the result is in w_a for even nsteps, else in w_b.
+ * The ring is left as by those steps. Same bits. */
+int mfv_advection_run_size(const mfv_mesh *m, int order, size_t *doubles);
+int mfv_advection_run(const mfv_mesh *m, double *w_a, double *w_b, const double *u_face,
+                      const double *v_face, const double *w_face, int order, double *dt_ring,
+                      int nsteps, double *workspace, void *stream);
+
 /* ---------------- shallow water (solvers/shallowater) ----------------------------- */
 
 /* time_step_SW (solvers/shallowater/fvm_utils.py:16-42). Output as mfv_time_step. */

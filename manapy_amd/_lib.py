@@ -219,6 +219,8 @@ _SIGNATURES = {
     'mfv_update_new_value': [MESH_P, P, P, P, P, c_double, P, P],
     'mfv_dt_ring_init': [P, P, P],
     'mfv_advection_step': [MESH_P, P, P, P, P, P, P, P, P, c_double, c_int, P, c_int, P, P],
+    'mfv_advection_run_size': [MESH_P, c_int, ctypes.POINTER(ctypes.c_size_t)],
+    'mfv_advection_run': [MESH_P, P, P, P, P, P, c_int, P, c_int, P, P],
     'mfv_time_step_sw': [MESH_P, P, P, P, c_double, c_double, c_double, c_double, P, DP, P],
     'mfv_sw_gradients': [MESH_P, P, P, P, P, P, P],
     'mfv_sw_residuals': [MESH_P, P, P, P, P, P, P, c_double, c_int, P, P, P],

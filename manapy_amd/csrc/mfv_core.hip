@@ -318,6 +318,10 @@ extern "C" int mfv_barthlimiter(const mfv_mesh *m, const double *w_c, const doub
 
 // ---------------------------------------------------------------------------------------------
 // gradient and limiter of NF fields in one pass (cell_gradient then barthlimiter, bit for bit)
+//
+// OWNER: a ghost takes its owner's value (Neumann everywhere), as the fused advection steps read
+// it; RECORD > 0 then writes w, gx, gy, (gz,) psi as one record of that many doubles to gx[0], so
+// that a step gathers a neighbour's from one line.
 
 template <int NF>
 struct GradArgs {
@@ -329,7 +333,7 @@ struct GradArgs {
     double *__restrict__ psi[NF];
 };
 
-template <int DIM, int NF>
+template <int DIM, int NF, bool OWNER>
 __device__ __forceinline__ void stencil_sums(const Mesh &m, const GradArgs<NF> &a, int i, double cx, double cy,
                                              double cz, const double (&wi)[NF], double (&I)[6], double (&J)[NF][3])
 {
@@ -371,10 +375,11 @@ __device__ __forceinline__ void stencil_sums(const Mesh &m, const GradArgs<NF> &
         const int q = m.lsq_ghosts[(size_t)j * m.C + i];
         const double *g = m.face_ghost + 3 * (size_t)q;
         const double jx = g[0] - cx, jy = g[1] - cy, jz = DIM == 3 ? g[2] - cz : 0.;
-        lsq_accumulate<DIM>(I, J[0], jx, jy, jz, a.ghost[0][q] - wi[0]);
+        const int o = OWNER ? m.face_cells[2 * (size_t)q] : q;
+        lsq_accumulate<DIM>(I, J[0], jx, jy, jz, (OWNER ? a.w[0] : a.ghost[0])[o] - wi[0]);
 #pragma unroll
         for (int f = 1; f < NF; f++) {
-            const double dw = a.ghost[f][q] - wi[f];
+            const double dw = (OWNER ? a.w[f] : a.ghost[f])[o] - wi[f];
             J[f][0] += (jx * dw);
             J[f][1] += (jy * dw);
             if (DIM == 3) J[f][2] += (jz * dw);
@@ -382,7 +387,7 @@ __device__ __forceinline__ void stencil_sums(const Mesh &m, const GradArgs<NF> &
     }
 }
 
-template <int DIM, int NF, int MF>
+template <int DIM, int NF, int MF, bool OWNER, int RECORD>
 __global__ void __launch_bounds__(kBlock) k_gradient_limited(Mesh m, GradArgs<NF> a)
 {
     const int i = xcd_block() * blockDim.x + threadIdx.x;
@@ -393,7 +398,7 @@ __global__ void __launch_bounds__(kBlock) k_gradient_limited(Mesh m, GradArgs<NF
     int fid[MF];
 #pragma unroll
     for (int s = 0; s < MF; s++) {
-        const int f = m.cell_faces[(size_t)s * m.C + i];
+        const int f = m.cell_faces[(size_t)min(s, m.MF - 1) * m.C + i];
         fid[s] = (s < nf) ? f : -1;
     }
     double wi[NF], I[6] = {0., 0., 0., 0., 0., 0.}, J[NF][3];
@@ -402,7 +407,7 @@ __global__ void __launch_bounds__(kBlock) k_gradient_limited(Mesh m, GradArgs<NF
         wi[f] = a.w[f][i];
         J[f][0] = J[f][1] = J[f][2] = 0.;
     }
-    stencil_sums<DIM, NF>(m, a, i, cx, cy, cz, wi, I, J);
+    stencil_sums<DIM, NF, OWNER>(m, a, i, cx, cy, cz, wi, I, J);
     // the faces: what lies on both sides, and the face's centre
     int2 ab[MF];
     int nm[MF];
@@ -424,8 +429,8 @@ __global__ void __launch_bounds__(kBlock) k_gradient_limited(Mesh m, GradArgs<NF
         for (int s = 0; s < MF; s++) {
             const bool has = fid[s] >= 0, inner = nm[s] == 0 || nm[s] > 10;
             wl[s] = a.w[f][has ? ab[s].x : i];
-            const double *src = (has && !inner) ? a.ghost[f] : a.w[f];
-            wr[s] = src[!has ? i : inner ? ab[s].y : fid[s]];
+            const double *src = (has && !inner && !OWNER) ? a.ghost[f] : a.w[f];
+            wr[s] = src[!has ? i : inner ? ab[s].y : OWNER ? ab[s].x : fid[s]];
         }
         double gx, gy, gz;
         lsq_solve<DIM>(I, J[f], gx, gy, gz);
@@ -450,19 +455,30 @@ __global__ void __launch_bounds__(kBlock) k_gradient_limited(Mesh m, GradArgs<NF
                 }
                 psi = pmin(psi, psi_ij);
             }
+        if (RECORD) {
+            double2 *q = reinterpret_cast<double2 *>(a.gx[f] + RECORD * (size_t)i);
+            q[0] = make_double2(wi[f], gx);
+            q[1] = DIM == 3 ? make_double2(gy, gz) : make_double2(gy, psi);
+            if (DIM == 3) q[2] = make_double2(psi, 0.);
+            continue;
+        }
         a.gx[f][i] = gx;
         a.gy[f][i] = gy;
-        a.gz[f][i] = gz;
+        if (DIM == 3 || !OWNER) a.gz[f][i] = gz;
         a.psi[f][i] = psi;
     }
 }
 
-template <int NF>
+// Doubles of a cell's record (w, gradient, psi) in the fused advection steps.
+constexpr int adv_record(int dim) { return dim == 2 ? 4 : 8; }
+
+template <int NF, bool OWNER = false, bool RECORD = false>
 static int gradient_limited(const mfv_mesh *m, const GradArgs<NF> &a, hipStream_t st)
 {
     const Mesh k = to_kernel(m);
     const dim3 g(grid_for(m->nb_cells)), b(kBlock);
-#define LAUNCH(D, M) hipLaunchKernelGGL((k_gradient_limited<D, NF, M>), g, b, 0, st, k, a)
+#define LAUNCH(D, M) \
+    hipLaunchKernelGGL((k_gradient_limited<D, NF, M, OWNER, RECORD ? adv_record(D) : 0>), g, b, 0, st, k, a)
     if (m->dim == 2) {
         if (m->max_cell_faces <= 3) LAUNCH(2, 3);
         else if (m->max_cell_faces == 4) LAUNCH(2, 4);
@@ -842,45 +858,6 @@ extern "C" int mfv_update_new_value(const mfv_mesh *m, double *ne_c, const doubl
 // ----- fused advection step ------------------------------------------------------------------
 // Neumann ghosts (w_ghost[f] = w[c0]) are read straight from the owner cell.
 
-template <int DIM>
-__global__ void __launch_bounds__(kBlock) k_adv_grad_limit(Mesh m, const double *__restrict__ w,
-                                                            double *__restrict__ scratch)
-{
-    int i = xcd_block() * blockDim.x + threadIdx.x;
-    if (i >= m.C) return;
-    const double cx = m.cell_center[3 * i], cy = m.cell_center[3 * i + 1], cz = m.cell_center[3 * i + 2];
-    const double wi = w[i];
-    double I[6] = {0., 0., 0., 0., 0., 0.}, J[3] = {0., 0., 0.};
-    const int nn = m.lsq_ncells[i];
-    for (int j = 0; j < nn; j++) {
-        int c = m.lsq_cells[(size_t)j * m.C + i];
-        const double *p = m.cell_center + 3 * (size_t)c;
-        lsq_accumulate<DIM>(I, J, p[0] - cx, p[1] - cy, DIM == 3 ? p[2] - cz : 0., w[c] - wi);
-    }
-    const int ng = m.lsq_nghosts[i];
-    for (int j = 0; j < ng; j++) {
-        int f = m.lsq_ghosts[(size_t)j * m.C + i];
-        const double *p = m.face_ghost + 3 * (size_t)f;
-        lsq_accumulate<DIM>(I, J, p[0] - cx, p[1] - cy, DIM == 3 ? p[2] - cz : 0., w[m.face_cells[2 * f]] - wi);
-    }
-    double gx, gy, gz;
-    lsq_solve<DIM>(I, J, gx, gy, gz);
-    double w_max = wi, w_min = wi;
-    const int nf = m.cell_nfaces[i];
-    for (int j = 0; j < nf; j++) {
-        int f = m.cell_faces[(size_t)j * m.C + i];
-        int nm = m.face_name[f];
-        double a = w[m.face_cells[2 * f]];
-        double b = (nm == 0 || nm > 10) ? w[m.face_cells[2 * f + 1]] : w[m.face_cells[2 * f]];
-        w_max = pmax(pmax(w_max, a), b);
-        w_min = pmin(pmin(w_min, a), b);
-    }
-    scratch[i] = gx;
-    scratch[(size_t)m.C + i] = gy;
-    if (DIM == 3) scratch[2 * (size_t)m.C + i] = gz;
-    scratch[(size_t)DIM * m.C + i] = barth_psi<DIM>(m, i, wi, gx, gy, gz, w_max, w_min);
-}
-
 template <int DIM, int ORDER>
 __global__ void __launch_bounds__(kBlock) k_adv_step(Mesh m, const double *__restrict__ w_in,
                                                       double *__restrict__ w_out, const double *__restrict__ uc,
@@ -923,9 +900,9 @@ extern "C" int mfv_advection_step(const mfv_mesh *m, const double *w_in, double 
     Mesh k = to_kernel(m);
     hipStream_t st = as_stream(stream);
     if (order == 2) {
-        auto kg = (m->dim == 2) ? k_adv_grad_limit<2> : k_adv_grad_limit<3>;
-        hipLaunchKernelGGL(kg, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, st, k, w_in, scratch);
-        if (int rc = check_launch("k_adv_grad_limit")) return rc;
+        const size_t C = m->nb_cells;
+        const GradArgs<1> a{{w_in}, {nullptr}, {scratch}, {scratch + C}, {scratch + 2 * C}, {scratch + m->dim * C}};
+        if (int rc = gradient_limited<1, true>(m, a, st)) return rc;
     }
     const size_t nw = waves_for(m->nb_cells);
     double *part = dt_scratch(nw, as_stream(stream));
@@ -936,4 +913,177 @@ extern "C" int mfv_advection_step(const mfv_mesh *m, const double *w_in, double 
                        u_face, v_face, w_face, cfl, (double)(order - 1), scratch, r, part);
     if (int rc = check_launch("k_adv_step")) return rc;
     return dt_finish(part, nw, r.next, st);
+}
+
+// ----- nsteps advection steps ------------------------------------------------------------------
+// The velocity does not change within a run, so what a face contributes of it is laid out once: for
+// the r-th contribution of a cell's residual the cell whose value is carried (the upwind side), the
+// flux velocity out of the cell, and at order 2 the face's centre as seen from the upwind cell. dt
+// is one number for all steps. A step is then one launch (two at order 2) that reads 12 (28, 36)
+// coalesced bytes a slot and gathers one value (record) a slot, where the general step gathers both
+// sides of each face, its normal and velocities, and forms and reduces the same dt again. 100 steps
+// at 80k triangles, order 1: 1022 -> 326 us, about what 100 launches in a row take. The sums are the general step's term for term: the
+// outward velocity is the face's with its sign turned for the right-hand cell, which is exact.
+namespace {
+
+constexpr int kAdvNone = (int)0x80000000;  // no face in this position
+
+struct AdvTable {
+    int32_t *__restrict__ up;   // [MF][C] upwind cell; ~cell: its value without reconstruction (a ghost's)
+    double *__restrict__ coef;  // [MF][C] velocity through the face, out of the cell
+    double *__restrict__ r;     // [MF][DIM][C] face centre - upwind cell's centre (order 2)
+    double *__restrict__ rec;   // [C][adv_record] w, gradient, psi (order 2)
+};
+
+size_t adv_table(const mfv_mesh *m, int order, double *ws, AdvTable *t)
+{
+    const size_t C = ((size_t)m->nb_cells + 1) & ~(size_t)1, MF = m->max_cell_faces;
+    size_t n = 0;
+    auto take = [&](size_t k) {
+        n += k;
+        return ws ? ws + n - k : nullptr;
+    };
+    t->rec = order == 2 ? take(C * adv_record(m->dim)) : nullptr;
+    t->coef = take(MF * C);
+    t->r = order == 2 ? take(MF * C * m->dim) : nullptr;
+    t->up = reinterpret_cast<int32_t *>(take((MF * C + 1) / 2));
+    return n;
+}
+
+template <int DIM, int ORDER>
+__global__ void __launch_bounds__(kBlock) k_adv_table(Mesh m, AdvTable t, const double *__restrict__ uf,
+                                                      const double *__restrict__ vf, const double *__restrict__ wf)
+{
+    const int i = xcd_block() * blockDim.x + threadIdx.x;
+    if (i >= m.C) return;
+    const int nf = m.cell_nfaces[i];
+    for (int r = 0; r < m.MF; r++) {
+        const size_t q = (size_t)r * m.C + i;
+        if (r >= nf) {
+            t.up[q] = kAdvNone;
+            t.coef[q] = 0.;
+            if (ORDER == 2)
+                for (int d = 0; d < DIM; d++) t.r[((size_t)r * DIM + d) * m.C + i] = 0.;
+            continue;
+        }
+        const int f = m.cell_faces[(size_t)m.order_split[q] * m.C + i];
+        const int a = m.face_cells[2 * (size_t)f], b = m.face_cells[2 * (size_t)f + 1];
+        const double *n = m.face_normal + 3 * (size_t)f;
+        const double sign = uf[f] * n[0] + vf[f] * n[1] + wf[f] * n[2];
+        const bool left = sign >= 0;
+        const int up = (left || b < 0) ? a : b;
+        t.up[q] = (left || b >= 0) ? up : ~up;
+        t.coef[q] = (a == i) ? sign : -sign;
+        if (ORDER == 2) {
+            for (int d = 0; d < DIM; d++)
+                t.r[((size_t)r * DIM + d) * m.C + i] = m.face_center[3 * (size_t)f + d] - m.cell_center[3 * (size_t)up + d];
+        }
+    }
+}
+
+template <int DIM, int ORDER, int MF>
+__global__ void __launch_bounds__(kBlock) k_adv_run(Mesh m, AdvTable t, const double *__restrict__ w_in,
+                                                    double *__restrict__ w_out, DtRing ring, double om)
+{
+    const int i = xcd_block() * blockDim.x + threadIdx.x;
+    const double dt = ring.cur[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {  // the ring as a step that forms the same dt leaves it
+        ring.spare[0] = 1e6;
+        ring.time[0] += dt;
+        ring.next[0] = dt;
+    }
+    if (i >= m.C) return;
+    int up[MF];
+    double c[MF], r[MF][DIM], w[MF];
+#pragma unroll
+    for (int s = 0; s < MF; s++) {
+        const size_t row = min(s, m.MF - 1);
+        const int u = t.up[row * m.C + i];
+        up[s] = (s < m.MF) ? u : kAdvNone;
+        c[s] = t.coef[row * m.C + i];
+        if (ORDER == 2) {
+#pragma unroll
+            for (int d = 0; d < DIM; d++) r[s][d] = t.r[(row * DIM + d) * m.C + i];
+        }
+    }
+    const double wi = w_in[i], vol = m.cell_volume[i];
+#pragma unroll
+    for (int s = 0; s < MF; s++) {
+        const int q = up[s] == kAdvNone ? i : up[s] < 0 ? ~up[s] : up[s];
+        if (ORDER == 1) {
+            w[s] = w_in[q] + 0.;
+            continue;
+        }
+        const double2 *p = reinterpret_cast<const double2 *>(t.rec + adv_record(DIM) * (size_t)q);
+        const double2 a = p[0], b = p[1];
+        double full;
+        if (DIM == 2)
+            full = a.x + om * b.y * (a.y * r[s][0] + b.x * r[s][1]);
+        else
+            full = a.x + om * p[2].x * (a.y * r[s][0] + b.x * r[s][1] + b.y * r[s][DIM - 1]);
+        w[s] = up[s] < 0 ? a.x : full;
+    }
+    double rez = 0.;
+#pragma unroll
+    for (int s = 0; s < MF; s++)
+        if (up[s] != kAdvNone) rez -= c[s] * w[s];
+    w_out[i] = wi + dt * ((rez + 0.) / vol + 0.);
+}
+
+}  // namespace
+
+static int check_advection_run(const mfv_mesh *m, int order)
+{
+    MFV_REQUIRE(order == 1 || order == 2, "order must be 1 or 2");
+    if (int rc = validate_mesh(m, order == 2, 1, 0)) return rc;
+    MFV_REQUIRE(!(m->dim == 2 && m->max_cell_faces > 4), "2D cells have at most 4 faces");
+    return MFV_OK;
+}
+
+extern "C" int mfv_advection_run_size(const mfv_mesh *m, int order, size_t *doubles)
+{
+    if (int rc = check_advection_run(m, order)) return rc;
+    MFV_REQUIRE(doubles, "NULL pointer");
+    AdvTable t;
+    *doubles = adv_table(m, order, nullptr, &t);
+    return MFV_OK;
+}
+
+extern "C" int mfv_advection_run(const mfv_mesh *m, double *w_a, double *w_b, const double *u_face,
+                                 const double *v_face, const double *w_face, int order, double *dt_ring_p, int nsteps,
+                                 double *workspace, void *stream)
+{
+    if (int rc = check_advection_run(m, order)) return rc;
+    MFV_REQUIRE(nsteps >= 0, "nsteps < 0");
+    MFV_REQUIRE(w_a && w_b && w_a != w_b && u_face && v_face && w_face && dt_ring_p && workspace,
+                "NULL or aliased array");
+    MFV_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0, "workspace must be 16-byte aligned");
+    if (m->nb_cells == 0 || nsteps == 0) return MFV_OK;
+    const Mesh k = to_kernel(m);
+    const hipStream_t st = as_stream(stream);
+    const dim3 g(grid_for(m->nb_cells)), b(kBlock);
+    AdvTable t;
+    adv_table(m, order, workspace, &t);
+    auto kt = m->dim == 2 ? (order == 2 ? k_adv_table<2, 2> : k_adv_table<2, 1>)
+                          : (order == 2 ? k_adv_table<3, 2> : k_adv_table<3, 1>);
+    hipLaunchKernelGGL(kt, g, b, 0, st, k, t, u_face, v_face, w_face);
+    if (int rc = check_launch("k_adv_table")) return rc;
+    const int MF = m->max_cell_faces;
+    auto ks = m->dim == 2 ? (MF <= 3 ? (order == 2 ? k_adv_run<2, 2, 3> : k_adv_run<2, 1, 3>)
+                                     : (order == 2 ? k_adv_run<2, 2, 4> : k_adv_run<2, 1, 4>))
+                          : (MF <= 4 ? (order == 2 ? k_adv_run<3, 2, 4> : k_adv_run<3, 1, 4>)
+                                     : (order == 2 ? k_adv_run<3, 2, 8> : k_adv_run<3, 1, 8>));
+    double *in = w_a, *out = w_b;
+    for (int s = 0; s < nsteps; s++) {
+        if (order == 2) {
+            const GradArgs<1> a{{in}, {nullptr}, {t.rec}, {nullptr}, {nullptr}, {nullptr}};
+            if (int rc = gradient_limited<1, true, true>(m, a, st)) return rc;
+        }
+        hipLaunchKernelGGL(ks, g, b, 0, st, k, t, in, out, dt_ring(dt_ring_p, s), (double)(order - 1));
+        if (int rc = check_launch("k_adv_run")) return rc;
+        double *x = in;
+        in = out;
+        out = x;
+    }
+    return MFV_OK;
 }

@@ -103,21 +103,20 @@ class AdvectionSolver(object):
                                       "compute_new_val sequence for other boundary conditions")
         m = self._m
         s = stream_ptr()
-        C = int(self.domain.nbcells)
         _lib.call('mfv_time_step', m.ptr, self.u.cell.data_ptr(), self.v.cell.data_ptr(), self.w.cell.data_ptr(),
                   float(self.cfl), self._clock.dt0.data_ptr(), None, s)
         self._clock.start()
+        nsteps = len(range(nsteps))
         a = self.var.cell
         b = torch.empty_like(a)
-        scratch = torch.zeros((int(self.dim) + 1) * C, dtype=torch.float64, device=a.device)
-        for k in range(nsteps):
-            _lib.call('mfv_advection_step', m.ptr, a.data_ptr(), b.data_ptr(), self.u.cell.data_ptr(),
-                      self.v.cell.data_ptr(), self.w.cell.data_ptr(), self.u.face.data_ptr(), self.v.face.data_ptr(),
-                      self.w.face.data_ptr(), float(self.cfl), int(self.order), self._clock.ring.data_ptr(), k,
-                      scratch.data_ptr(), s)
-            a, b = b, a
+        n = ctypes.c_size_t(0)
+        _lib.call('mfv_advection_run_size', m.ptr, int(self.order), ctypes.byref(n))
+        ws = torch.empty(n.value, dtype=torch.float64, device=a.device)
+        _lib.call('mfv_advection_run', m.ptr, a.data_ptr(), b.data_ptr(), self.u.face.data_ptr(),
+                  self.v.face.data_ptr(), self.w.face.data_ptr(), int(self.order), self._clock.ring.data_ptr(),
+                  nsteps, ws.data_ptr(), s)
         if nsteps % 2 == 1:
-            self.var.cell.copy_(a)
+            a.copy_(b)
         self._clock.step = nsteps
         self.dt = float(self._clock.ring[(nsteps - 1) % 3]) if nsteps else self.dt
         return self._clock.time
