@@ -179,6 +179,9 @@ int mfv_sw_residuals(const mfv_mesh *m, const double *h, const double *hu, const
 /* update_SW (solvers/shallowater/fvm_utils.py:3-14) for h, hu, hv; dt from dt_dev[0]. */
 int mfv_update_sw(const mfv_mesh *m, double *h, double *hu, double *hv, const double *rez,
                   const double *src, const double *dt_dev, void *stream);
+/* The same with dt by value. */
+int mfv_update_sw_by(const mfv_mesh *m, double *h, double *hu, double *hv, const double *rez,
+                     const double *src, double dt, void *stream);
 
 /* The reference's own shallow-water scheme on five fields (h, hu, hv, hc, Z).
  *
@@ -463,6 +466,9 @@ int mfv_euler3d_rusanov(const mfv_mesh *m, const double *U, const double *G, dou
 /* update_euler_3d_fvc (fvm_utils3d.py:1316-1327); dt from dt_dev[0]. */
 int mfv_euler3d_update(const mfv_mesh *m, double *U, const double *rez, double gamma,
                        const double *dt_dev, void *stream);
+/* The same with dt by value. */
+int mfv_euler3d_update_by(const mfv_mesh *m, double *U, const double *rez, double gamma, double dt,
+                          void *stream);
 
 /* The reference's own argument form of the four Euler kernels: the state as six separate
  * device arrays (cells [C], ghosts [F]) and the residual as five, so a caller that holds the

@@ -225,6 +225,7 @@ _SIGNATURES = {
     'mfv_sw_gradients': [MESH_P, P, P, P, P, P, P],
     'mfv_sw_residuals': [MESH_P, P, P, P, P, P, P, c_double, c_int, P, P, P],
     'mfv_update_sw': [MESH_P, P, P, P, P, P, P, P],
+    'mfv_update_sw_by': [MESH_P, P, P, P, P, P, c_double, P],
     'mfv_explicitscheme_convective_sw': [MESH_P] + [P] * 20 + [c_double, c_int, P],
     'mfv_term_source_srnh_sw': [MESH_P, P, P, P, P, P, P, P, P, P, P, c_int, P, c_int, P, P, c_double, c_int, P],
     'mfv_update_sw5': [MESH_P] + [P] * 18 + [c_double, c_double, c_double, P, P],
@@ -249,6 +250,7 @@ _SIGNATURES = {
     'mfv_euler3d_time_step': [MESH_P, P, c_double, c_double, P, DP, P],
     'mfv_euler3d_rusanov': [MESH_P, P, P, c_double, c_int, P, P],
     'mfv_euler3d_update': [MESH_P, P, P, c_double, P, P],
+    'mfv_euler3d_update_by': [MESH_P, P, P, c_double, c_double, P],
     'mfv_ghost_value_tubeschok3d': [MESH_P, ctypes.POINTER(MfvEulerArrays), P, P, P, ctypes.POINTER(MfvEulerArrays),
                                     c_int, P],
     'mfv_time_step_euler_3d': [MESH_P, ctypes.POINTER(MfvEulerArrays), c_double, c_double, P, P],

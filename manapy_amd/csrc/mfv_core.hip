@@ -627,7 +627,7 @@ double *dt_scratch(size_t nwaves, hipStream_t st)
     return e->ptr;
 }
 
-__global__ void __launch_bounds__(1024) k_dt_finish(const double *__restrict__ part, size_t n, double *__restrict__ out)
+__device__ __forceinline__ double dt_block_min(const double *__restrict__ part, size_t n)
 {
     __shared__ double sh[1024];
     // four partials in flight per thread (the minimum of a set does not depend on the order)
@@ -656,9 +656,25 @@ __global__ void __launch_bounds__(1024) k_dt_finish(const double *__restrict__ p
         }
         __syncthreads();
     }
+    return sh[0];
+}
+
+__global__ void __launch_bounds__(1024) k_dt_finish(const double *__restrict__ part, size_t n, double *__restrict__ out)
+{
+    const double r = dt_block_min(part, n);
+    if (threadIdx.x == 0 && r < out[0]) out[0] = r;
+}
+
+// out[0] = min(1e6, min part), and the same to host memory if given (k_dt_total's own start value:
+// no launch to reset out[0] first).
+__global__ void __launch_bounds__(1024) k_dt_total(const double *__restrict__ part, size_t n,
+                                                   double *__restrict__ out, double *host)
+{
+    const double r = dt_block_min(part, n);
     if (threadIdx.x == 0) {
-        const double r = sh[0];
-        if (r < out[0]) out[0] = r;
+        const double dt = (r < 1e6) ? r : 1e6;
+        out[0] = dt;
+        if (host) __hip_atomic_store(host, dt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -671,18 +687,80 @@ int dt_finish(const double *part, size_t n, double *out, hipStream_t st)
 
 }  // namespace mfv
 
-int mfv::finish_dt(double *dt_dev, double *dt_host, void *stream)
+namespace {
+
+// One double of pinned host memory for a dt on its way to the host. A call takes a slot for as long
+// as it waits; as many slots exist as calls have waited at once (threads).
+std::mutex g_dt_slot_mu;
+std::vector<double *> g_dt_slots;
+
+double *take_dt_slot()
 {
-    if (int rc = check_launch("dt kernel")) return rc;
-    if (dt_host) {
-        hipError_t e = hipMemcpyAsync(dt_host, dt_dev, sizeof(double), hipMemcpyDeviceToHost, as_stream(stream));
-        if (e == hipSuccess) e = hipStreamSynchronize(as_stream(stream));
-        if (e != hipSuccess) {
-            set_error("dt readback: %s", hipGetErrorString(e));
-            return MFV_EHIP;
+    {
+        std::lock_guard<std::mutex> lock(g_dt_slot_mu);
+        if (!g_dt_slots.empty()) {
+            double *p = g_dt_slots.back();
+            g_dt_slots.pop_back();
+            return p;
         }
     }
-    return MFV_OK;
+    void *p = nullptr;
+    const hipError_t e = hipHostMalloc(&p, sizeof(double), hipHostMallocPortable | hipHostMallocMapped);
+    if (e != hipSuccess) {
+        set_error("dt readback: hipHostMalloc: %s", hipGetErrorString(e));
+        return nullptr;
+    }
+    return static_cast<double *>(p);
+}
+
+void give_dt_slot(double *p)
+{
+    std::lock_guard<std::mutex> lock(g_dt_slot_mu);
+    g_dt_slots.push_back(p);
+}
+
+}  // namespace
+
+// A dt that the host waits for is written to pinned memory by the fold itself and looked at there:
+// a copy to the caller's (pageable) double is a launch of its own and a wait for its signal on top.
+// The sequence of four 3D advection steps 577 -> 441 us, four of the SRNH scheme at 1k cells
+// (eight dts) 572 -> 354 us.
+int mfv::dt_total(const double *part, size_t n, double *dt_dev, double *dt_host, hipStream_t st)
+{
+    double *slot = nullptr;
+    volatile long long *word = nullptr;
+    const long long kWaiting = 0x7ff8000000000001LL;  // a NaN: no dt has these bits
+    if (dt_host) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+            set_error("dt readback: the stream is being captured; the dt cannot be read on the host");
+            return MFV_EHIP;
+        }
+        slot = take_dt_slot();
+        if (!slot) return MFV_ENOMEM;
+        word = reinterpret_cast<volatile long long *>(slot);
+        *word = kWaiting;
+    }
+    hipLaunchKernelGGL(k_dt_total, dim3(1), dim3(1024), 0, st, part, n, dt_dev, slot);
+    int rc = check_launch("dt kernel");
+    if (slot) {
+        if (rc == MFV_OK) {
+            for (int k = 0; k < 200000 && *word == kWaiting; k++) __builtin_ia32_pause();
+            if (*word == kWaiting) {  // a long queue ahead, or an error: wait as for any other work
+                const hipError_t e = hipStreamSynchronize(st);
+                if (e != hipSuccess) {
+                    set_error("dt readback: %s", hipGetErrorString(e));
+                    return MFV_EHIP;  // the slot may still be written: it is not given back
+                }
+            }
+            const long long w = *word;
+            memcpy(dt_host, &w, sizeof(double));
+        } else {
+            (void)hipStreamSynchronize(st);
+        }
+        give_dt_slot(slot);
+    }
+    return rc;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -715,16 +793,15 @@ extern "C" int mfv_time_step(const mfv_mesh *m, const double *u, const double *v
 {
     if (int rc = validate_mesh(m, 0, 0, 0)) return rc;
     MFV_REQUIRE(u && v && w && dt_dev, "NULL array");
-    if (int rc = mfv_dt_reset(dt_dev, stream)) return rc;
-    if (m->nb_cells) {
-        const size_t nw = waves_for(m->nb_cells);
-        double *part = dt_scratch(nw, as_stream(stream));
+    const size_t nw = m->nb_cells ? waves_for(m->nb_cells) : 0;
+    double *part = nullptr;
+    if (nw) {
+        part = dt_scratch(nw, as_stream(stream));
         if (!part) return MFV_ENOMEM;
         hipLaunchKernelGGL(k_adv_time_step, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream),
                            to_kernel(m), u, v, w, cfl, part);
-        if (int rc = dt_finish(part, nw, dt_dev, as_stream(stream))) return rc;
     }
-    return finish_dt(dt_dev, dt_host, stream);
+    return dt_total(part, nw, dt_dev, dt_host, as_stream(stream));
 }
 
 // Upwind flux of face f in its own orientation (compute_upwind_flux, fvm_utils.py:5-17) with

@@ -696,14 +696,13 @@ extern "C" int mfv_time_step_diffusion(const mfv_mesh *m, const double *u, const
     if (int rc = validate_mesh(m, 0, 0, 0)) return rc;
     MFV_REQUIRE(dt_dev, "NULL dt_dev");
     MFV_REQUIRE((u && v && w) || (!u && !v && !w), "u, v, w must all be given or all be NULL");
-    if (int rc = mfv_dt_reset(dt_dev, stream)) return rc;
-    if (m->nb_cells) {
-        const size_t nw = waves_for(m->nb_cells);
-        double *part = dt_scratch(nw, as_stream(stream));
+    const size_t nw = m->nb_cells ? waves_for(m->nb_cells) : 0;
+    double *part = nullptr;
+    if (nw) {
+        part = dt_scratch(nw, as_stream(stream));
         if (!part) return MFV_ENOMEM;
         hipLaunchKernelGGL(k_time_step_diff, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream),
                            to_kernel(m), u, v, w, cfl, Dxx, Dyy, Dzz, part);
-        if (int rc = dt_finish(part, nw, dt_dev, as_stream(stream))) return rc;
     }
-    return finish_dt(dt_dev, dt_host, stream);
+    return dt_total(part, nw, dt_dev, dt_host, as_stream(stream));
 }

@@ -1210,25 +1210,15 @@ extern "C" int mfv_euler3d_time_step(const mfv_mesh *m, const double *U, double 
     if (int rc = validate_mesh(m, 0, 0, 0)) return rc;
     MFV_REQUIRE(m->dim == 3 && m->max_cell_faces >= 4, "Euler 3D time step needs tetrahedra");
     MFV_REQUIRE(U && dt_dev, "NULL array");
-    if (int rc = mfv_dt_reset(dt_dev, stream)) return rc;
-    if (m->nb_cells) {
-        const size_t nw = waves_for(m->nb_cells);
-        double *part = dt_scratch(nw, as_stream(stream));
+    const size_t nw = m->nb_cells ? waves_for(m->nb_cells) : 0;
+    double *part = nullptr;
+    if (nw) {
+        part = dt_scratch(nw, as_stream(stream));
         if (!part) return MFV_ENOMEM;
         hipLaunchKernelGGL(k_euler_dt, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream), to_kernel(m),
                            U, cfl, gamma, part);
-        if (int rc = dt_finish(part, nw, dt_dev, as_stream(stream))) return rc;
     }
-    if (int rc = check_launch("k_euler_dt")) return rc;
-    if (dt_host) {
-        hipError_t e = hipMemcpyAsync(dt_host, dt_dev, sizeof(double), hipMemcpyDeviceToHost, as_stream(stream));
-        if (e == hipSuccess) e = hipStreamSynchronize(as_stream(stream));
-        if (e != hipSuccess) {
-            set_error("dt readback: %s", hipGetErrorString(e));
-            return MFV_EHIP;
-        }
-    }
-    return MFV_OK;
+    return dt_total(part, nw, dt_dev, dt_host, as_stream(stream));
 }
 
 extern "C" int mfv_euler3d_rusanov(const mfv_mesh *m, const double *U, const double *G, double gamma, int quirk,
@@ -1244,16 +1234,29 @@ extern "C" int mfv_euler3d_rusanov(const mfv_mesh *m, const double *U, const dou
     return check_launch("k_euler_rusanov");
 }
 
-extern "C" int mfv_euler3d_update(const mfv_mesh *m, double *U, const double *rez, double gamma, const double *dt_dev,
-                                  void *stream)
+static int euler3d_update(const mfv_mesh *m, double *U, const double *rez, double gamma, const double *dt_dev,
+                          double dt, void *stream)
 {
     if (int rc = validate_mesh(m, 0, 0, 0)) return rc;
     if (m->nb_cells == 0) return MFV_OK;
-    MFV_REQUIRE(U && rez && dt_dev, "NULL array");
+    MFV_REQUIRE(U && rez, "NULL array");
     hipLaunchKernelGGL((k_euler_update<Rows, Rows>), dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream),
                        m->nb_cells, Rows{U, (size_t)m->nb_cells}, Rows{const_cast<double *>(rez), (size_t)m->nb_cells},
-                       gamma, dt_dev, 0., m->cell_volume);
+                       gamma, dt_dev, dt, m->cell_volume);
     return check_launch("k_euler_update");
+}
+
+extern "C" int mfv_euler3d_update(const mfv_mesh *m, double *U, const double *rez, double gamma, const double *dt_dev,
+                                  void *stream)
+{
+    MFV_REQUIRE(dt_dev || (m && m->nb_cells == 0), "NULL array");
+    return euler3d_update(m, U, rez, gamma, dt_dev, 0., stream);
+}
+
+extern "C" int mfv_euler3d_update_by(const mfv_mesh *m, double *U, const double *rez, double gamma, double dt,
+                                     void *stream)
+{
+    return euler3d_update(m, U, rez, gamma, nullptr, dt, stream);
 }
 
 extern "C" int mfv_euler3d_step_fused(const mfv_mesh *m, const double *U_in, double *U_out, double gamma, double cfl,

@@ -308,12 +308,12 @@ __global__ void __launch_bounds__(kBlock) k_sw_residuals(Mesh m, const double *_
 __global__ void __launch_bounds__(kBlock) k_update_sw(int C, double *__restrict__ h, double *__restrict__ hu,
                                                        double *__restrict__ hv, const double *__restrict__ rez,
                                                        const double *__restrict__ src,
-                                                       const double *__restrict__ dt_dev,
+                                                       const double *__restrict__ dt_dev, double dt_host,
                                                        const double *__restrict__ vol)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= C) return;
-    const double dt = dt_dev[0];
+    const double dt = dt_dev ? dt_dev[0] : dt_host;
     const size_t n = C;
     h[i] += dt * (rez[i] + src[i]) / vol[i];
     hu[i] += dt * ((rez[n + i] + src[n + i]) / vol[i] + 0. + 0.);
@@ -355,16 +355,15 @@ extern "C" int mfv_time_step_sw(const mfv_mesh *m, const double *h, const double
 {
     if (int rc = validate_mesh(m, 0, 0, 0)) return rc;
     MFV_REQUIRE(h && hu && hv && dt_dev, "NULL array");
-    if (int rc = mfv_dt_reset(dt_dev, stream)) return rc;
-    if (m->nb_cells) {
-        const size_t nw = waves_for(m->nb_cells);
-        double *part = dt_scratch(nw, as_stream(stream));
+    const size_t nw = m->nb_cells ? waves_for(m->nb_cells) : 0;
+    double *part = nullptr;
+    if (nw) {
+        part = dt_scratch(nw, as_stream(stream));
         if (!part) return MFV_ENOMEM;
         hipLaunchKernelGGL(k_sw_time_step, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream),
                            to_kernel(m), h, hu, hv, cfl, grav, Dxx, Dyy, part);
-        if (int rc = dt_finish(part, nw, dt_dev, as_stream(stream))) return rc;
     }
-    return finish_dt(dt_dev, dt_host, stream);
+    return dt_total(part, nw, dt_dev, dt_host, as_stream(stream));
 }
 
 extern "C" int mfv_sw_gradients(const mfv_mesh *m, const double *h, const double *hu, const double *hv,
@@ -393,15 +392,28 @@ extern "C" int mfv_sw_residuals(const mfv_mesh *m, const double *h, const double
     return check_launch("k_sw_residuals");
 }
 
-extern "C" int mfv_update_sw(const mfv_mesh *m, double *h, double *hu, double *hv, const double *rez,
-                             const double *src, const double *dt_dev, void *stream)
+static int update_sw(const mfv_mesh *m, double *h, double *hu, double *hv, const double *rez, const double *src,
+                     const double *dt_dev, double dt, void *stream)
 {
     if (int rc = validate_mesh(m, 0, 0, 0)) return rc;
     if (m->nb_cells == 0) return MFV_OK;
-    MFV_REQUIRE(h && hu && hv && rez && src && dt_dev, "NULL array");
+    MFV_REQUIRE(h && hu && hv && rez && src, "NULL array");
     hipLaunchKernelGGL(k_update_sw, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream),
-                       m->nb_cells, h, hu, hv, rez, src, dt_dev, m->cell_volume);
+                       m->nb_cells, h, hu, hv, rez, src, dt_dev, dt, m->cell_volume);
     return check_launch("k_update_sw");
+}
+
+extern "C" int mfv_update_sw(const mfv_mesh *m, double *h, double *hu, double *hv, const double *rez,
+                             const double *src, const double *dt_dev, void *stream)
+{
+    MFV_REQUIRE(dt_dev || (m && m->nb_cells == 0), "NULL array");
+    return update_sw(m, h, hu, hv, rez, src, dt_dev, 0., stream);
+}
+
+extern "C" int mfv_update_sw_by(const mfv_mesh *m, double *h, double *hu, double *hv, const double *rez,
+                                const double *src, double dt, void *stream)
+{
+    return update_sw(m, h, hu, hv, rez, src, nullptr, dt, stream);
 }
 
 extern "C" int mfv_sw_step_fused(const mfv_mesh *m, const double *state_in, double *state_out, const double *Z,

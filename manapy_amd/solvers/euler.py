@@ -85,9 +85,8 @@ class EulerSolver3D(object):
                   self.rez.data_ptr(), stream_ptr())
 
     def compute_new_val(self):
-        self._dt_dev.fill_(float(self.dt))
-        _lib.call('mfv_euler3d_update', self._m.ptr, self.U.data_ptr(), self.rez.data_ptr(), self.gamma,
-                  self._dt_dev.data_ptr(), stream_ptr())
+        _lib.call('mfv_euler3d_update_by', self._m.ptr, self.U.data_ptr(), self.rez.data_ptr(), self.gamma,
+                  float(self.dt), stream_ptr())
 
     def step(self):
         """ghosts, dt, fluxes, update (the data-flow order of the reference kernels)."""

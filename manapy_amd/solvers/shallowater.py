@@ -236,10 +236,8 @@ class ShallowWaterSolver(object):
         """``system.py:237-242`` -> update_SW."""
         if self.flux == 'srnh':
             return self._srnh_update(None)
-        self._dt_dev.fill_(float(self.dt))
-        _lib.call('mfv_update_sw', self._m.ptr, self.h.cell.data_ptr(), self.hu.cell.data_ptr(),
-                  self.hv.cell.data_ptr(), self._rez.data_ptr(), self._src.data_ptr(), self._dt_dev.data_ptr(),
-                  stream_ptr())
+        _lib.call('mfv_update_sw_by', self._m.ptr, self.h.cell.data_ptr(), self.hu.cell.data_ptr(),
+                  self.hv.cell.data_ptr(), self._rez.data_ptr(), self._src.data_ptr(), float(self.dt), stream_ptr())
 
     def run(self, nsteps):
         """``nsteps`` x (stepper, compute_fluxes, compute_new_val), fused on the packed path with
