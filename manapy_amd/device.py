@@ -94,7 +94,11 @@ def dptr(t):
 
 
 def stream_ptr(stream=None):
+    """The stream's handle, by default that of torch's current stream (read without making the
+    Stream object that torch.cuda.current_stream() returns)."""
     import torch
+    if stream is None and torch.cuda.is_initialized():
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
     s = stream if stream is not None else torch.cuda.current_stream()
     return s.cuda_stream
 
