@@ -764,6 +764,8 @@ typedef struct mfv_ell_batch {
 #define MFV_KS_CORRECT 3
 #define MFV_KS_DONE 4
 #define MFV_KS_FAILED 5
+#define MFV_KS_CHECK 6   /* residual formed (mfv_krylov_fused_tick only, as the next) */
+#define MFV_KS_ADVANCE 7 /* at the start of a time step */
 
 #define MFV_KS_SIGMA 0
 #define MFV_KS_TAU 1
@@ -782,9 +784,8 @@ typedef struct mfv_ell_batch {
 #define MFV_KS_IT 14
 #define MFV_KS_OUTER 15
 #define MFV_KS_ITTOT 16
-#define MFV_KS_RHO_OLD 17 /* this and the next two: mfv_krylov_fused_tick only */
-#define MFV_KS_STOP_V 18
-#define MFV_KS_STOP_T 19
+#define MFV_KS_RHO_OLD 17 /* this and DT: mfv_krylov_fused_tick only */
+#define MFV_KS_DT 20 /* the time step of an instance with steps_left */
 #define MFV_KS_NSCAL 24
 
 typedef struct mfv_krylov_work {
@@ -824,8 +825,14 @@ typedef struct mfv_krylov_fused {
     double *pa, *pb, *pr;    /* [S], [5][S], [3][S] */
     double *scal;            /* [I][MFV_KS_NSCAL] */
     int32_t *status;         /* [I] */
+    int32_t *status_t;       /* [I] (the library's own) */
     const int32_t *chunks;   /* [S][4], 16-byte aligned */
     const int32_t *n_chunks; /* device scalar */
+    int32_t *steps_left;     /* [I] time steps still to be taken, or NULL: no advection */
+    const int32_t *adv_up;   /* [adv_slots][64 S], [..][64 S], [64 S]: mfv_advection_rows */
+    const double *adv_coef, *adv_vol;
+    int32_t adv_slots;       /* a multiple of four */
+    int32_t pad_;
 } mfv_krylov_fused;
 
 /* Slices per chunk of an instance of ns slices: four (one per wave of a block), more where an
@@ -833,13 +840,23 @@ typedef struct mfv_krylov_fused {
 #define MFV_KRYLOV_MAX_CHUNKS 512
 #define MFV_KRYLOV_SPAN(ns) (4 * (((ns) + 4 * MFV_KRYLOV_MAX_CHUNKS - 1) / (4 * MFV_KRYLOV_MAX_CHUNKS)))
 
-/* mfv_krylov_tick and mfv_krylov_graph with two launches per BiCGStab iteration instead of
- * eight; the same states, scalars and stopping tests. grid_chunks: blocks of the per-chunk
- * kernels, grid_inst: of the per-instance kernel. */
+/* n_iter rounds of two launches, each one BiCGStab iteration of an instance in INNER or one change
+ * of state of another one (refinement, convergence test, next time step); the same scalars and
+ * stopping tests as mfv_krylov_tick. An instance set to MFV_KS_START solves its system once; one
+ * set to MFV_KS_ADVANCE takes steps_left time steps, each b = x + dt advection(x), x = b as the
+ * first guess, then the solve, and is DONE after the last. grid_chunks: blocks of the kernels.
+ * Asynchronous; poll status[] (and steps_left[]) between ticks. */
 int mfv_krylov_fused_tick(const mfv_ell_batch *e, const mfv_krylov_fused *w, int n_iter, int grid_chunks,
-                          int grid_inst, void *stream);
+                          void *stream);
 int mfv_krylov_fused_graph(const mfv_ell_batch *e, const mfv_krylov_fused *w, int n_iter, int grid_chunks,
-                           int grid_inst, void **graph_out);
+                           void **graph_out);
+
+/* The rows [row0, row0 + rows) of the advection tables of nb_rows rows, from a mesh and the face
+ * velocities of its instance (rows past the cells get no faces). Order 1, Neumann boundaries: the
+ * step b = x + dt advection(x) gives the bits of mfv_advection_step. */
+int mfv_advection_rows(const mfv_mesh *m, const double *u_face, const double *v_face, const double *w_face,
+                       int row0, int rows, int nb_rows, int slots, int32_t *adv_up, double *adv_coef,
+                       double *adv_vol, void *stream);
 
 /* 16-bit columns for the slices [slice0, slice0 + nslices) of an assembled ELL batch (no
  * counterpart in the reference: a storage form of the matrix of solvers/ls/system.py:154-171).

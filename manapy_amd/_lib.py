@@ -172,8 +172,9 @@ class MfvGradientFields(ctypes.Structure):
 
 class MfvKrylovFused(ctypes.Structure):
     """Mirror of ``struct mfv_krylov_fused`` (include/mfv.h)."""
-    _fields_ = [(k, P) for k in ('x', 'b', 'd', 'rh', 'dinv', 'p', 'u', 'w', 'pa', 'pb', 'pr', 'scal', 'status', 'chunks',
-                                 'n_chunks')]
+    _fields_ = [(k, P) for k in ('x', 'b', 'd', 'rh', 'dinv', 'p', 'u', 'w', 'pa', 'pb', 'pr', 'scal', 'status',
+                                 'status_t', 'chunks', 'n_chunks', 'steps_left', 'adv_up', 'adv_coef', 'adv_vol')] + \
+        [('adv_slots', ctypes.c_int32), ('pad_', ctypes.c_int32)]
 
 
 class MfvSwBatch(ctypes.Structure):
@@ -183,10 +184,10 @@ class MfvSwBatch(ctypes.Structure):
 
 
 # per-instance solver states and scalar slots (MFV_KS_* in include/mfv.h)
-KS_IDLE, KS_START, KS_INNER, KS_CORRECT, KS_DONE, KS_FAILED = 0, 1, 2, 3, 4, 5
+KS_IDLE, KS_START, KS_INNER, KS_CORRECT, KS_DONE, KS_FAILED, KS_CHECK, KS_ADVANCE = 0, 1, 2, 3, 4, 5, 6, 7
 KS_SIGMA, KS_TAU, KS_TOL_OUT, KS_TOL_IN, KS_MAXIT_IN, KS_MAXIT_OUT = 0, 1, 2, 3, 4, 5
 KS_RHO, KS_ALPHA, KS_OMEGA, KS_BETA, KS_R0N2, KS_RN2, KS_BN2, KS_RESN2 = 6, 7, 8, 9, 10, 11, 12, 13
-KS_IT, KS_OUTER, KS_ITTOT, KS_NSCAL = 14, 15, 16, 24
+KS_IT, KS_OUTER, KS_ITTOT, KS_DT, KS_NSCAL = 14, 15, 16, 20, 24
 KRYLOV_MAX_CHUNKS = 512
 
 MESH_P = ctypes.POINTER(MfvMesh)
@@ -306,8 +307,9 @@ _SIGNATURES = {
     'mfv_domain_geometry_3d_free': [ctypes.POINTER(MfvDomainGeometry3d)],
     'mfv_krylov_tick': [ELL_P, KW_P, c_int, c_int, c_int, P],
     'mfv_krylov_graph': [ELL_P, KW_P, c_int, c_int, c_int, ctypes.POINTER(c_void_p)],
-    'mfv_krylov_fused_tick': [ELL_P, KF_P, c_int, c_int, c_int, P],
-    'mfv_krylov_fused_graph': [ELL_P, KF_P, c_int, c_int, c_int, ctypes.POINTER(c_void_p)],
+    'mfv_krylov_fused_tick': [ELL_P, KF_P, c_int, c_int, P],
+    'mfv_krylov_fused_graph': [ELL_P, KF_P, c_int, c_int, ctypes.POINTER(P)],
+    'mfv_advection_rows': [MESH_P, P, P, P, c_int, c_int, c_int, c_int, P, P, P, P],
     'mfv_ell_spmv': [ELL_P, P, P, c_int, P],
     'mfv_ell_narrow_columns': [ELL_P, c_int, c_int, P, P, P],
 }

@@ -482,10 +482,20 @@ __global__ void __launch_bounds__(256) k_ell_spmv(Ell e, const double *__restric
 //   instance's chunk sums, in the same fixed order, so all blocks hold the same bits. A chunk is
 //   four slices (one a wave) and an instance has at most 512, so that this costs two loads a
 //   thread; larger instances take more slices a chunk.
-// * A scalar is never read in the launch that writes it: the v product reads ALPHA, RHO_OLD, IT
-//   and STOP_T and writes OMEGA, BETA, RHO, RN2 and STOP_V; the t product reads RHO and STOP_V
-//   and writes ALPHA, RHO_OLD, IT, ITTOT and STOP_T. A launch for a stopped instance finds the
-//   sums unchanged and comes to the same verdict again. Only the instance's first block writes.
+// * The refinement has no launches of its own either. The product that finds the inner solve ended
+//   adds d to x at once, the t product after it forms the FP64 residual instead of a product, and
+//   the v product after that comes to the verdict on it and takes the first step of the next inner
+//   solve. With a launch each for them (four, and a round of the host's, every n_iter iterations) a
+//   change of state waited for the next tick: 20 implicit steps of eight systems took 154 ticks of
+//   six iterations, 120 so; a system of 12.8k rows 13.0 -> 11.3 ms.
+// * An instance that has time steps left (steps_left) takes the next one where it would be done: the
+//   v product writes b = x + dt advection(x), the t product takes x = b and forms its residual.
+//   Nothing of it waits for the host (serving, eight requests of 20 steps: 33.5 -> 26.5 ms).
+// * A scalar is never read in the launch that writes it: the v product reads ALPHA, RHO_OLD, IT,
+//   OUTER, steps_left and status and writes OMEGA, BETA, RHO, RN2, the scalars that an inner solve
+//   starts from (in state CHECK, which reads none of them) and status_t; the t product reads RHO and
+//   status_t and writes ALPHA, RHO_OLD, IT, ITTOT, OUTER, steps_left and status. Between pairs of
+//   launches status is the instance's whole state. Only the instance's first block writes them.
 struct Fused {
     double *__restrict__ x;
     double *__restrict__ b;
@@ -500,15 +510,26 @@ struct Fused {
     double *__restrict__ pr;
     double *__restrict__ scal;
     int32_t *__restrict__ status;
+    int32_t *__restrict__ status_t;
     const int4 *__restrict__ chunks;
     const int32_t *__restrict__ n_chunks;
+    int32_t *__restrict__ steps_left;
+    const int32_t *__restrict__ adv_up;
+    const double *__restrict__ adv_coef;
+    const double *__restrict__ adv_vol;
+    int adv_slots;
 };
+
+// What a t product does with an instance besides its part of an iteration (status_t; the other
+// values are those of status).
+enum { kResidualStart = 16, kResidual, kResidualOfB };
 
 static Fused to_kernel(const mfv_krylov_fused *w)
 {
     return Fused{w->x,  w->b,  w->d,  w->rh,   w->dinv,   reinterpret_cast<float4 *>(w->u),
                  reinterpret_cast<float2 *>(w->w), w->p, w->pa, w->pb, w->pr, w->scal, w->status,
-                 reinterpret_cast<const int4 *>(w->chunks), w->n_chunks};
+                 w->status_t, reinterpret_cast<const int4 *>(w->chunks), w->n_chunks, w->steps_left, w->adv_up,
+                 w->adv_coef, w->adv_vol, w->adv_slots};
 }
 
 constexpr int kChunkBlock = 256;
@@ -685,103 +706,103 @@ struct SlotGroup {
 };
 constexpr int kFirst = 16, kNext = 8;
 
-// x += d with the last iteration's alpha p + omega s (a stop before its t product has none).
-__global__ void __launch_bounds__(kChunkBlock) k_fused_correct(Fused w)
+// x += d, with the last iteration's alpha p + omega s where they are still to come.
+__device__ __forceinline__ void chunk_correct(const Fused &w, const Chunk &h, bool pending, float alpha, float omega)
 {
-    const int n = *w.n_chunks;
-    for (int k = blockIdx.x; k < n; k += gridDim.x) {
-        const Chunk h = chunk_at(w, k);
-        if (w.status[h.inst] != MFV_KS_CORRECT) continue;
-        const double *sc = w.scal + (size_t)h.inst * MFV_KS_NSCAL;
-        const bool pending = sc[MFV_KS_STOP_T] == 0.;
-        const float alpha = (float)sc[MFV_KS_ALPHA], omega = (float)sc[MFV_KS_OMEGA];
-        for (int row = h.begin * 64 + threadIdx.x; row < h.end * 64; row += kChunkBlock) {
-            float d = w.d[row];
-            if (pending) {
-                const float4 u = w.u[row];
-                d = fmaf(omega, u.x, fmaf(alpha, u.z, d));
-            }
-            w.x[row] += (double)d;
+    for (int row = h.begin * 64 + threadIdx.x; row < h.end * 64; row += kChunkBlock) {
+        float d = w.d[row];
+        if (pending) {
+            const float4 u = w.u[row];
+            d = fmaf(omega, u.x, fmaf(alpha, u.z, d));
         }
+        w.x[row] += (double)d;
     }
 }
 
-// r = b - op(x) in FP64 (states START and CORRECT) and the start of the inner solve.
-__global__ void __launch_bounds__(kChunkBlock) k_fused_residual(Ell e, Fused w)
+// b = x + dt advection(x): the upwind values, their outward face velocities and the order of the
+// sum are laid out per row (mfv_advection_rows).
+__device__ __forceinline__ void chunk_advance(const Ell &e, const Fused &w, const Chunk &h, double dt)
+{
+    const size_t R = (size_t)e.S * 64;
+    for (int row = h.begin * 64 + threadIdx.x; row < h.end * 64; row += kChunkBlock) {
+        double rez = 0.;
+        for (int j = 0; j < w.adv_slots; j += 4) {
+            int up[4];
+            double c[4], v[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                up[k] = w.adv_up[(j + k) * R + row];
+                c[k] = w.adv_coef[(j + k) * R + row];
+            }
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[k] = w.x[up[k] < 0 ? row : up[k]] + 0.;
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                if (up[k] >= 0) rez -= c[k] * v[k];
+        }
+        w.b[row] = w.x[row] + dt * ((rez + 0.) / w.adv_vol[row] + 0.);
+    }
+}
+
+// ell_row64 with its slots in groups of four: the registers of groups of eight would cost the
+// iterations that share the kernel a third of their waves.
+__device__ __forceinline__ double row_product64(const Ell &e, int s, int lane, const double *__restrict__ x)
+{
+    const int wdt = e.slice_w[s], row = s * 64 + lane;
+    const unsigned base = (unsigned)lane;
+    const size_t at = (size_t)s * e.W * 64;
+    const double *__restrict__ vals = e.vals + at;
+    const int16_t *__restrict__ c16 = e.cols16 + at;
+    const int32_t *__restrict__ c32 = e.cols + at;
+    const bool narrow = slice_is_narrow(e, s);
+    double acc = 0.;
+    for (int j = 0; j < wdt; j += 4) {
+        double v[4], xv[4];
+        int c[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const unsigned q = base + (unsigned)min(j + k, wdt - 1) * 64u;
+            v[k] = vals[q];
+            c[k] = narrow ? row + c16[q] : c32[q];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) xv[k] = x[c[k]];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (j + k < wdt) acc = fma(v[k], xv[k], acc);
+    }
+    return acc;
+}
+
+// r = b - op(x) in FP64 and the start of the inner solve.
+__device__ __forceinline__ void chunk_residual(const Ell &e, const Fused &w, const Chunk &h, int how, double sigma,
+                                               double tau)
 {
     const int lane = threadIdx.x & 63;
-    const int n = *w.n_chunks;
-    for (int k = blockIdx.x; k < n; k += gridDim.x) {
-        const Chunk h = chunk_at(w, k);
-        const int st = w.status[h.inst];
-        if (st != MFV_KS_START && st != MFV_KS_CORRECT) continue;
-        const double *sc = w.scal + (size_t)h.inst * MFV_KS_NSCAL;
-        const double sigma = sc[MFV_KS_SIGMA], tau = sc[MFV_KS_TAU];
-        double sum[3] = {0., 0., 0.};
-        for (int s = h.begin + wave_index(); s < h.end; s += kChunkWaves) {
-            const int row = s * 64 + lane;
-            float di;
-            if (st == MFV_KS_START) {
-                const double dg = sigma + tau * e.diag[row];
-                w.dinv[row] = di = (dg != 0.) ? (float)(1. / dg) : 0.f;
-            } else {
-                di = w.dinv[row];
-            }
-            const double ax = ell_row64(e, s, lane, w.x);
-            const double bb = w.b[row];
-            const double res = bb - (sigma * w.x[row] + tau * ax);
-            const float r32 = (float)((double)di * res);
-            w.rh[row] = r32;
-            w.d[row] = 0.f;
-            w.u[row] = make_float4(r32, 0.f, 0.f, 0.f);
-            sum[0] += res * res;
-            sum[1] += bb * bb;
-            sum[2] += (double)r32 * (double)r32;
+    const double *x = how == kResidualOfB ? w.b : w.x;  // x = b then, and no row is read and written
+    double sum[3] = {0., 0., 0.};
+    for (int s = h.begin + wave_index(); s < h.end; s += kChunkWaves) {
+        const int row = s * 64 + lane;
+        float di;
+        if (how == kResidual) {
+            di = w.dinv[row];
+        } else {
+            const double dg = sigma + tau * e.diag[row];
+            w.dinv[row] = di = (dg != 0.) ? (float)(1. / dg) : 0.f;
         }
-        chunk_store<3>(w.pr, e.S, h.s0 + h.c, sum);
+        const double ax = row_product64(e, s, lane, x);
+        const double bb = w.b[row], xx = x[row];
+        if (how == kResidualOfB) w.x[row] = xx;
+        const double res = bb - (sigma * xx + tau * ax);
+        const float r32 = (float)((double)di * res);
+        w.rh[row] = r32;
+        w.d[row] = 0.f;
+        w.u[row] = make_float4(r32, 0.f, 0.f, 0.f);
+        sum[0] += res * res;
+        sum[1] += bb * bb;
+        sum[2] += (double)r32 * (double)r32;
     }
-}
-
-__device__ __forceinline__ int chunks_of(int ns) { return (ns + MFV_KRYLOV_SPAN(ns) - 1) / MFV_KRYLOV_SPAN(ns); }
-
-__global__ void __launch_bounds__(kChunkBlock) k_fused_check(Ell e, Fused w)
-{
-    const int n = *e.n_live_inst;
-    for (int i = blockIdx.x; i < n; i += gridDim.x) {
-        const int inst = e.live_inst[i];
-        const int was = w.status[inst];
-        __syncthreads();  // read by every thread before thread 0 changes it
-        if (was != MFV_KS_START && was != MFV_KS_CORRECT) continue;
-        double sum[3];
-        chunk_totals<3>(w.pr, e.S, e.inst_slice0[inst], chunks_of(e.inst_nslices[inst]), sum);
-        if (threadIdx.x == 0) {
-            double *sc = w.scal + (size_t)inst * MFV_KS_NSCAL;
-            const double resn2 = sum[0], bn2 = sum[1];
-            sc[MFV_KS_RESN2] = resn2;
-            sc[MFV_KS_BN2] = bn2;
-            if (was == MFV_KS_START) sc[MFV_KS_OUTER] = 0.;
-            sc[MFV_KS_OUTER] += 1.;
-            const double tol = sc[MFV_KS_TOL_OUT];
-            int st;
-            if (!isfinite(resn2) || !isfinite(bn2)) st = MFV_KS_FAILED;  // NaN/inf data: refinement cannot help
-            else if (resn2 <= tol * tol * bn2) st = MFV_KS_DONE;
-            else if (sc[MFV_KS_OUTER] > sc[MFV_KS_MAXIT_OUT]) st = MFV_KS_FAILED;
-            else {
-                sc[MFV_KS_RHO] = sum[2];
-                sc[MFV_KS_RHO_OLD] = sum[2];
-                sc[MFV_KS_R0N2] = sum[2];
-                sc[MFV_KS_RN2] = sum[2];
-                sc[MFV_KS_ALPHA] = 0.;
-                sc[MFV_KS_OMEGA] = 0.;
-                sc[MFV_KS_BETA] = 0.;
-                sc[MFV_KS_IT] = 0.;
-                sc[MFV_KS_STOP_V] = 0.;
-                sc[MFV_KS_STOP_T] = 0.;
-                st = MFV_KS_INNER;
-            }
-            w.status[inst] = st;
-        }
-    }
+    chunk_store<3>(w.pr, e.S, h.s0 + h.c, sum);
 }
 
 // omega, the new residual's norm and rho, and whether the inner solve ends, from the t product's
@@ -816,8 +837,9 @@ __global__ void __launch_bounds__(kChunkBlock, 3) k_fused_v(Ell e, Fused w)
     for (int k = blockIdx.x; k < n; k += gridDim.x) {
         if (k != (int)blockIdx.x) h = chunk_at(w, k);
         double *sc = w.scal + (size_t)h.inst * MFV_KS_NSCAL;
+        const bool first = h.c == 0 && threadIdx.x == 0;
         const int status = w.status[h.inst];  // the scalars too, before anything is waited for
-        const double stopped = sc[MFV_KS_STOP_T], rho_old = sc[MFV_KS_RHO_OLD], alpha_old = sc[MFV_KS_ALPHA];
+        const double rho_old = sc[MFV_KS_RHO_OLD], alpha_old = sc[MFV_KS_ALPHA];
         const float sigma = (float)sc[MFV_KS_SIGMA], tau = (float)sc[MFV_KS_TAU];
         const Stop lim = stop_of(sc);
         auto load = [&](int c) { return w.u[c]; };
@@ -839,26 +861,63 @@ __global__ void __launch_bounds__(kChunkBlock, 3) k_fused_v(Ell e, Fused w)
         if (s < h.end) take();
         double q[5];
         chunk_totals<5>(w.pb, e.S, h.s0, h.nch, q);
-        if (status != MFV_KS_INNER || stopped != 0.) continue;
         float alpha = 0.f, om = 0.f, be = 0.f;
-        if (lim.it != 0.) {
+        int next = status;  // status_t
+        if (status == MFV_KS_INNER) {
             const Step st = close_step(q, lim);
             const double beta = (st.rho / rho_old) * (alpha_old / st.omega);
-            if (h.c == 0 && threadIdx.x == 0) {
+            if (first) {
                 sc[MFV_KS_OMEGA] = st.omega;
                 sc[MFV_KS_RN2] = st.rn2;
-                if (st.done) {
-                    sc[MFV_KS_STOP_V] = 1.;
-                } else {
+                if (!st.done) {
                     sc[MFV_KS_BETA] = beta;
                     sc[MFV_KS_RHO] = st.rho;
                 }
             }
-            if (st.done) continue;
             alpha = (float)alpha_old;
             om = (float)st.omega;
             be = (float)beta;
+            if (st.done) {
+                chunk_correct(w, h, true, alpha, om);
+                next = kResidual;
+            }
+        } else if (status == MFV_KS_CORRECT) {  // a breakdown in the t product: d holds all there is
+            chunk_correct(w, h, false, 0.f, 0.f);
+            next = kResidual;
+        } else if (status == MFV_KS_START) {
+            next = kResidualStart;
+        } else if (status == MFV_KS_ADVANCE) {
+            chunk_advance(e, w, h, sc[MFV_KS_DT]);
+            next = kResidualOfB;
+        } else if (status == MFV_KS_CHECK) {
+            double sum[3];
+            chunk_totals<3>(w.pr, e.S, h.s0, h.nch, sum);
+            const double tol = sc[MFV_KS_TOL_OUT];
+            if (!isfinite(sum[0]) || !isfinite(sum[1])) next = MFV_KS_FAILED;  // NaN/inf data: refinement cannot help
+            else if (sum[0] <= tol * tol * sum[1]) next = MFV_KS_DONE;
+            else if (sc[MFV_KS_OUTER] > sc[MFV_KS_MAXIT_OUT]) next = MFV_KS_FAILED;
+            else next = MFV_KS_INNER;
+            if (next == MFV_KS_DONE && w.steps_left && w.steps_left[h.inst] > 0) {
+                chunk_advance(e, w, h, sc[MFV_KS_DT]);
+                next = kResidualOfB;
+            }
+            if (first) {
+                sc[MFV_KS_RESN2] = sum[0];
+                sc[MFV_KS_BN2] = sum[1];
+                if (next == MFV_KS_INNER) {
+                    sc[MFV_KS_RHO] = sum[2];
+                    sc[MFV_KS_RHO_OLD] = sum[2];
+                    sc[MFV_KS_R0N2] = sum[2];
+                    sc[MFV_KS_RN2] = sum[2];
+                    sc[MFV_KS_ALPHA] = 0.;
+                    sc[MFV_KS_OMEGA] = 0.;
+                    sc[MFV_KS_BETA] = 0.;
+                    sc[MFV_KS_IT] = 0.;
+                }
+            }
         }
+        if (first) w.status_t[h.inst] = next;
+        if (next != MFV_KS_INNER) continue;
         auto p_of = [&](const float4 &u) { return fmaf(be, fmaf(-om, u.w, u.z), fmaf(-om, u.y, u.x)); };
         double sum[1] = {0.};
         while (s < h.end) {
@@ -882,7 +941,7 @@ __global__ void __launch_bounds__(kChunkBlock, 3) k_fused_v(Ell e, Fused w)
     }
 }
 
-__global__ void __launch_bounds__(kChunkBlock) k_fused_t(Ell e, Fused w)
+__global__ void __launch_bounds__(kChunkBlock, 3) k_fused_t(Ell e, Fused w)
 {
     const int lane = threadIdx.x & 63;
     Chunk h = chunk_at(w, min((int)blockIdx.x, e.S - 1));
@@ -890,8 +949,9 @@ __global__ void __launch_bounds__(kChunkBlock) k_fused_t(Ell e, Fused w)
     for (int k = blockIdx.x; k < n; k += gridDim.x) {
         if (k != (int)blockIdx.x) h = chunk_at(w, k);
         double *sc = w.scal + (size_t)h.inst * MFV_KS_NSCAL;
-        const int status = w.status[h.inst];
-        const double stopped = sc[MFV_KS_STOP_V], rho = sc[MFV_KS_RHO];
+        const bool first = h.c == 0 && threadIdx.x == 0;
+        const int status = w.status_t[h.inst];
+        const double rho = sc[MFV_KS_RHO];
         const float sigma = (float)sc[MFV_KS_SIGMA], tau = (float)sc[MFV_KS_TAU];
         auto load = [&](int c) { return w.w[c]; };
         int s = h.begin + wave_index();
@@ -910,18 +970,29 @@ __global__ void __launch_bounds__(kChunkBlock) k_fused_t(Ell e, Fused w)
         if (s < h.end) take();
         double rv[1];
         chunk_totals<1>(w.pa, e.S, h.s0, h.nch, rv);
-        if (status != MFV_KS_INNER || stopped != 0.) continue;
+        if (status >= kResidualStart) {
+            if (first) {
+                sc[MFV_KS_OUTER] = (status == kResidual ? sc[MFV_KS_OUTER] : 0.) + 1.;
+                if (status == kResidualOfB) w.steps_left[h.inst] -= 1;
+                w.status[h.inst] = MFV_KS_CHECK;
+            }
+            chunk_residual(e, w, h, status, sc[MFV_KS_SIGMA], sc[MFV_KS_TAU]);
+            continue;
+        }
+        if (status != MFV_KS_INNER) {
+            if (first) w.status[h.inst] = status;
+            continue;
+        }
         const double a = rho / rv[0];
         const bool broken = rv[0] == 0. || !isfinite(a);  // breakdown: refine with what d holds
-        if (h.c == 0 && threadIdx.x == 0) {
-            if (broken) {
-                sc[MFV_KS_STOP_T] = 1.;
-            } else {
+        if (first) {
+            if (!broken) {
                 sc[MFV_KS_ALPHA] = a;
                 sc[MFV_KS_RHO_OLD] = rho;
                 sc[MFV_KS_IT] += 1.;
                 sc[MFV_KS_ITTOT] += 1.;
             }
+            w.status[h.inst] = broken ? MFV_KS_CORRECT : MFV_KS_INNER;
         }
         if (broken) continue;
         const float al = (float)a;
@@ -947,34 +1018,6 @@ __global__ void __launch_bounds__(kChunkBlock) k_fused_t(Ell e, Fused w)
             if (s < h.end) take();
         }
         chunk_store<5>(w.pb, e.S, h.s0 + h.c, sum);
-    }
-}
-
-// The end of a tick: an inner solve that has ended moves to CORRECT, so that the next tick starts
-// with its refinement (its last sums would otherwise be looked at one tick later).
-__global__ void __launch_bounds__(kChunkBlock) k_fused_close(Ell e, Fused w)
-{
-    const int n = *e.n_live_inst;
-    for (int i = blockIdx.x; i < n; i += gridDim.x) {
-        const int inst = e.live_inst[i];
-        double *sc = w.scal + (size_t)inst * MFV_KS_NSCAL;
-        const int was = w.status[inst];
-        const bool stopped = sc[MFV_KS_STOP_V] != 0. || sc[MFV_KS_STOP_T] != 0.;
-        const bool fresh = sc[MFV_KS_IT] == 0.;
-        __syncthreads();  // read by every thread before thread 0 changes them
-        if (was != MFV_KS_INNER || (fresh && !stopped)) continue;
-        if (stopped) {
-            if (threadIdx.x == 0) w.status[inst] = MFV_KS_CORRECT;
-            continue;
-        }
-        double q[5];
-        chunk_totals<5>(w.pb, e.S, e.inst_slice0[inst], chunks_of(e.inst_nslices[inst]), q);
-        const Step st = close_step(q, stop_of(sc));
-        if (st.done && threadIdx.x == 0) {
-            sc[MFV_KS_OMEGA] = st.omega;
-            sc[MFV_KS_RN2] = st.rn2;
-            w.status[inst] = MFV_KS_CORRECT;
-        }
     }
 }
 
@@ -1059,62 +1102,104 @@ extern "C" int mfv_krylov_graph(const mfv_ell_batch *e, const mfv_krylov_work *w
     return MFV_OK;
 }
 
-static int check_fused(const mfv_ell_batch *e, const mfv_krylov_fused *w, int n_iter, int grid_chunks, int grid_inst)
+static int check_fused(const mfv_ell_batch *e, const mfv_krylov_fused *w, int n_iter, int grid_chunks)
 {
     if (int rc = validate_ell(e)) return rc;
     MFV_REQUIRE(w != nullptr, "Krylov work descriptor is NULL");
     MFV_REQUIRE(w->x && w->b && w->d && w->rh && w->dinv && w->u && w->w && w->p && w->pa && w->pb && w->pr && w->scal &&
-                    w->status && w->chunks && w->n_chunks,
+                    w->status && w->status_t && w->chunks && w->n_chunks,
                 "Krylov work descriptor has NULL pointers");
+    MFV_REQUIRE(!w->steps_left || (w->adv_up && w->adv_coef && w->adv_vol && w->adv_slots >= 4 && w->adv_slots % 4 == 0),
+                "steps_left needs the advection tables, in groups of four slots");
     MFV_REQUIRE(((reinterpret_cast<uintptr_t>(w->u) | reinterpret_cast<uintptr_t>(w->w) |
                   reinterpret_cast<uintptr_t>(w->chunks)) &
                  15) == 0,
                 "u, w and chunks must be 16-byte aligned");
-    MFV_REQUIRE(n_iter >= 0 && n_iter <= 4096, "n_iter %d out of [0, 4096]", n_iter);
+    MFV_REQUIRE(n_iter >= 1 && n_iter <= 4096, "n_iter %d out of [1, 4096]", n_iter);
     MFV_REQUIRE(grid_chunks >= 1 && grid_chunks <= 65536, "grid_chunks %d out of [1, 65536]", grid_chunks);
-    MFV_REQUIRE(grid_inst >= 1 && grid_inst <= 65536, "grid_inst %d out of [1, 65536]", grid_inst);
     return MFV_OK;
 }
 
 static int fused_launches(const mfv_ell_batch *e, const mfv_krylov_fused *w, int n_iter, int grid_chunks,
-                          int grid_inst, hipStream_t st)
+                          hipStream_t st)
 {
     const Ell ek = to_kernel(e);
     const Fused wk = to_kernel(w);
-    const dim3 gc(grid_chunks), gi(grid_inst), b(kChunkBlock);
-    hipLaunchKernelGGL(k_fused_correct, gc, b, 0, st, wk);
-    hipLaunchKernelGGL(k_fused_residual, gc, b, 0, st, ek, wk);
-    hipLaunchKernelGGL(k_fused_check, gi, b, 0, st, ek, wk);
+    const dim3 gc(grid_chunks), b(kChunkBlock);
     for (int it = 0; it < n_iter; it++) {
         hipLaunchKernelGGL(k_fused_v, gc, b, 0, st, ek, wk);
         hipLaunchKernelGGL(k_fused_t, gc, b, 0, st, ek, wk);
     }
-    hipLaunchKernelGGL(k_fused_close, gi, b, 0, st, ek, wk);
     return check_launch("krylov tick");
 }
 
 extern "C" int mfv_krylov_fused_tick(const mfv_ell_batch *e, const mfv_krylov_fused *w, int n_iter, int grid_chunks,
-                                     int grid_inst, void *stream)
+                                     void *stream)
 {
-    if (int rc = check_fused(e, w, n_iter, grid_chunks, grid_inst)) return rc;
-    return fused_launches(e, w, n_iter, grid_chunks, grid_inst, as_stream(stream));
+    if (int rc = check_fused(e, w, n_iter, grid_chunks)) return rc;
+    return fused_launches(e, w, n_iter, grid_chunks, as_stream(stream));
 }
 
 extern "C" int mfv_krylov_fused_graph(const mfv_ell_batch *e, const mfv_krylov_fused *w, int n_iter, int grid_chunks,
-                                      int grid_inst, void **graph_out)
+                                      void **graph_out)
 {
-    if (int rc = check_fused(e, w, n_iter, grid_chunks, grid_inst)) return rc;
+    if (int rc = check_fused(e, w, n_iter, grid_chunks)) return rc;
     MFV_REQUIRE(graph_out, "graph_out is NULL");
     *graph_out = nullptr;
     MfvGraph *g = new MfvGraph();
     int rc = graph_begin(g);
-    if (rc == MFV_OK) rc = graph_finish(g, fused_launches(e, w, n_iter, grid_chunks, grid_inst, g->stream));
+    if (rc == MFV_OK) rc = graph_finish(g, fused_launches(e, w, n_iter, grid_chunks, g->stream));
     if (rc != MFV_OK) {
         graph_free(g);
         return rc;
     }
     *graph_out = g;
     return MFV_OK;
+}
+
+// ---------------------------------------------------------------------------------------------
+// The rows of an instance in the advection tables of the fused solve.
+
+__global__ void __launch_bounds__(256) k_advection_rows(Mesh m, const double *__restrict__ uf,
+                                                        const double *__restrict__ vf, const double *__restrict__ wf,
+                                                        int row0, int rows, size_t R, int slots,
+                                                        int32_t *__restrict__ up, double *__restrict__ coef,
+                                                        double *__restrict__ vol)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= rows) return;
+    const size_t row = (size_t)row0 + i;
+    const int nf = i < m.C ? m.cell_nfaces[i] : 0;
+    vol[row] = i < m.C ? m.cell_volume[i] : 1.;
+    for (int r = 0; r < slots; r++) {
+        int u = -1;
+        double c = 0.;
+        if (r < nf) {
+            const int f = m.cell_faces[(size_t)m.order_split[(size_t)r * m.C + i] * m.C + i];
+            const int a = m.face_cells[2 * (size_t)f], b = m.face_cells[2 * (size_t)f + 1];
+            const double *n = m.face_normal + 3 * (size_t)f;
+            const double sign = uf[f] * n[0] + vf[f] * n[1] + wf[f] * n[2];
+            u = row0 + ((sign >= 0 || b < 0) ? a : b);
+            c = (a == i) ? sign : -sign;
+        }
+        up[r * R + row] = u;
+        coef[r * R + row] = c;
+    }
+}
+
+extern "C" int mfv_advection_rows(const mfv_mesh *m, const double *u_face, const double *v_face, const double *w_face,
+                                  int row0, int rows, int nb_rows, int slots, int32_t *adv_up, double *adv_coef,
+                                  double *adv_vol, void *stream)
+{
+    if (int rc = validate_mesh(m, 0, 1, 0)) return rc;
+    MFV_REQUIRE(u_face && v_face && w_face && adv_up && adv_coef && adv_vol, "NULL array");
+    MFV_REQUIRE(m->max_cell_faces <= slots, "%d faces a cell, %d slots", m->max_cell_faces, slots);
+    MFV_REQUIRE(row0 >= 0 && rows >= m->nb_cells && (long long)row0 + rows <= nb_rows, "rows [%d, %lld) of %d", row0,
+                (long long)row0 + rows, nb_rows);
+    if (rows == 0) return MFV_OK;
+    hipLaunchKernelGGL(k_advection_rows, dim3(grid_for(rows)), dim3(256), 0, as_stream(stream), to_kernel(m), u_face,
+                       v_face, w_face, row0, rows, (size_t)nb_rows, slots, adv_up, adv_coef, adv_vol);
+    return check_launch("k_advection_rows");
 }
 
 extern "C" int mfv_ell_narrow_columns(const mfv_ell_batch *e, int slice0, int nslices, int16_t *cols16,

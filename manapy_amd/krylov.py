@@ -12,6 +12,7 @@ The solver replaces the factorisation of ``ScipySolver`` / ``MUMPSSolver``
 (``solvers/ls/system.py:236-379, 624-744``): FP32 BiCGStab with Jacobi scaling
 inside FP64 iterative refinement, stopped at ``||b - A x|| <= tol ||b||``.
 """
+import collections
 import ctypes
 
 import numpy as np
@@ -106,7 +107,10 @@ class EllBatch(object):
         self.chunks = torch.zeros((S, 4), dtype=i32, device=dev)
         self.n_chunks = torch.zeros(1, dtype=i32, device=dev)
         self.scal = torch.zeros(I * _lib.KS_NSCAL, dtype=f64, device=dev)
-        self.status = torch.zeros(I, dtype=i32, device=dev)
+        self._state = torch.zeros((2, I), dtype=i32, device=dev)  # read by the host in one copy
+        self.status, self.steps_left = self._state[0], self._state[1]
+        self.status_t = torch.zeros(I, dtype=i32, device=dev)
+        self._posts, self._spare = collections.deque(), []
 
         e = _lib.MfvEllBatch()
         e.nb_slices, e.width, e.nb_inst = S, W, I
@@ -116,12 +120,24 @@ class EllBatch(object):
         w = _lib.MfvKrylovFused()
         for k, t in dict(self.f32, **self.partial).items():
             setattr(w, k, t.data_ptr())
-        for k in ('x', 'b', 'scal', 'status', 'chunks', 'n_chunks'):
+        for k in ('x', 'b', 'scal', 'status', 'status_t', 'chunks', 'n_chunks'):
             setattr(w, k, getattr(self, k).data_ptr())
         self._e, self._w = e, w
         self._ranges = RangeAllocator(S)
         self._inst = {}                # inst -> (slice0, nslices, nrows)
         self._free_ids = list(range(I - 1, -1, -1))
+
+    def enable_advection(self, slots):
+        """Time steps on the device (mfv_krylov_fused_tick with steps_left): tables of ``slots``
+        (a multiple of four) faces a row. Before the first graph tick."""
+        import torch
+        R = self.S * 64
+        self.adv_up = torch.full((slots, R), -1, dtype=torch.int32, device=self.device)
+        self.adv_coef = torch.zeros((slots, R), dtype=torch.float64, device=self.device)
+        self.adv_vol = torch.ones(R, dtype=torch.float64, device=self.device)
+        for k in ('steps_left', 'adv_up', 'adv_coef', 'adv_vol'):
+            setattr(self._w, k, getattr(self, k).data_ptr())
+        self._w.adv_slots = int(slots)
 
     # -- arena ----------------------------------------------------------------------------------
     @property
@@ -226,10 +242,12 @@ class EllBatch(object):
         else:
             self.slice_narrow[s0:s0 + ns].zero_()
 
-    def configure(self, inst, sigma, tau, tol=1e-10, tol_in=1e-4, maxit_in=400, maxit_out=60):
-        """Operator coefficients and stopping parameters of one instance (counters zeroed)."""
+    def configure(self, inst, sigma, tau, tol=1e-10, tol_in=1e-4, maxit_in=400, maxit_out=60, dt=0.):
+        """Operator coefficients, stopping parameters and time step of one instance (counters
+        zeroed)."""
         import torch
         sc = np.zeros(_lib.KS_NSCAL)
+        sc[_lib.KS_DT] = dt
         sc[_lib.KS_SIGMA], sc[_lib.KS_TAU] = sigma, tau
         sc[_lib.KS_TOL_OUT], sc[_lib.KS_TOL_IN] = tol, tol_in
         sc[_lib.KS_MAXIT_IN], sc[_lib.KS_MAXIT_OUT] = maxit_in, maxit_out
@@ -263,24 +281,48 @@ class EllBatch(object):
         return max(1, min(4096, (nsl + 3) // 4)), max(1, ni)
 
     def tick(self, n_iter=8, grid_slices=None, grid_inst=None, stream=None, graph=False):
-        """One tick of every live instance. With ``graph=True`` the tick's launches are
-        replayed from a HIP graph captured once per (n_iter, grid sizes rounded up to powers of
+        """One tick of every live instance (``grid_inst`` is unused: no kernel runs per instance). With ``graph=True`` the tick's launches are
+        replayed from a HIP graph captured once per (n_iter, grid size rounded up to a power of
         two): the kernels read the live lists from device memory, so a graph stays valid as
         instances come and go, and the result is the same bits as the eager tick."""
-        _, gi = self.grids()
-        nch = max(1, min(16384, getattr(self, '_n_live', (0, 0, 0))[2]))
-        gs, gi = int(grid_slices or nch), int(grid_inst or gi)
+        gs = int(grid_slices or max(1, min(16384, getattr(self, '_n_live', (0, 0, 0))[2])))
+        n_iter = int(n_iter) or 1
         if not graph:
-            _lib.call('mfv_krylov_fused_tick', self.eptr, self.wptr, int(n_iter), gs, gi, stream_ptr(stream))
+            _lib.call('mfv_krylov_fused_tick', self.eptr, self.wptr, n_iter, gs, stream_ptr(stream))
             return
-        key = (int(n_iter), min(16384, _pow2(gs)), min(65536, _pow2(gi)))
+        key = (n_iter, min(16384, _pow2(gs)))
         graphs = self.__dict__.setdefault('_graphs', {})
         g = graphs.get(key)
         if g is None:
             out = ctypes.c_void_p()
-            _lib.call('mfv_krylov_fused_graph', self.eptr, self.wptr, key[0], key[1], key[2], ctypes.byref(out))
+            _lib.call('mfv_krylov_fused_graph', self.eptr, self.wptr, key[0], key[1], ctypes.byref(out))
             g = graphs[key] = out.value
         _lib.call('mfv_graph_launch', g, stream_ptr(stream))
+
+    def post_state(self, tag=None):
+        """Asks for a host copy of (status, steps_left) as they are at this point of the current
+        stream; ``take_state`` returns the copies in the order they were asked for, with ``tag``."""
+        import torch
+        buf, ev = self._spare.pop() if self._spare else \
+            (torch.empty((2, self.I), dtype=torch.int32, pin_memory=True), torch.cuda.Event())
+        buf.copy_(self._state, non_blocking=True)
+        ev.record()
+        self._posts.append((buf, ev, tag))
+
+    def posted(self):
+        return len(self._posts)
+
+    def take_state(self):
+        buf, ev, tag = self._posts.popleft()
+        ev.synchronize()
+        st = buf.numpy().copy()
+        self._spare.append((buf, ev))
+        return st[0], st[1], tag
+
+    def drop_states(self):
+        """Forgets the copies still on their way (waits for them: their buffers are used again)."""
+        while self._posts:
+            self.take_state()
 
     def close_graphs(self):
         """Release the captured ticks (after the device has finished any replay of them)."""
@@ -304,9 +346,17 @@ class EllBatch(object):
     def run(self, insts, n_iter=8, max_ticks=20000, graph=False):
         """Tick until every listed instance is DONE or FAILED; returns their statuses."""
         idx = np.asarray(list(insts), dtype=np.int64)
-        for _ in range(max_ticks):
-            self.tick(n_iter, graph=graph)
-            st = self.status.cpu().numpy()[idx]
-            if np.all((st == _lib.KS_DONE) | (st == _lib.KS_FAILED)):
-                return st
+        # the next tick is on its way while the state after the last one is looked at; a finished
+        # instance stays as it is
+        try:
+            for k in range(max_ticks + 1):
+                if k < max_ticks:
+                    self.tick(n_iter, graph=graph)
+                    self.post_state()
+                if self.posted() > 1 or (k == max_ticks and self.posted()):
+                    st = self.take_state()[0][idx]
+                    if np.all((st == _lib.KS_DONE) | (st == _lib.KS_FAILED)):
+                        return st
+        finally:
+            self.drop_states()
         raise _lib.MfvError("Krylov solve did not finish in %d ticks" % max_ticks)

@@ -26,6 +26,7 @@ import numpy as np
 
 from . import _lib
 from .device import DeviceMesh, require_gpu, stream_ptr
+from .diamond import DeviceDiamond
 from .krylov import EllBatch
 
 PHASE_WAIT, PHASE_ADVECT, PHASE_SOLVE, PHASE_DONE, PHASE_FAILED, PHASE_REJECTED = 0, 1, 2, 3, 4, 5
@@ -117,6 +118,7 @@ class ServingEngine(object):
         self.prep_threads = int(prep_threads)
         self.time_ticks = bool(time_ticks)
         self._tick_events = []
+        self.arena.enable_advection(8)  # the most faces a cell has
 
     # -- admission --------------------------------------------------------------------------------
     def never_fits(self, req):
@@ -142,9 +144,8 @@ class ServingEngine(object):
         if inst is None:
             raise RuntimeError("admit called without room")
         d = req.domain
-        dm = d._device_mesh if getattr(d, '_device_mesh', None) is not None else \
-            DeviceMesh(d, lsq=False, host=req._mesh_host)
-        d._device_mesh = dm
+        own = getattr(d, '_device_mesh', None)
+        dm = own if own is not None else DeviceMesh(d, lsq=False, host=req._mesh_host)
         dev = self.device
         C, F = req.C, int(d.nbfaces)
         s = stream_ptr()
@@ -159,53 +160,41 @@ class ServingEngine(object):
         _lib.call('mfv_time_step', dm.ptr, uc.data_ptr(), vc.data_ptr(), wc.data_ptr(), req.cfl, dt_dev.data_ptr(),
                   ctypes.byref(h), s)
         req.dt = h.value
-        ring = torch.zeros(4, dtype=torch.float64, device=dev)
-        _lib.call('mfv_dt_ring_init', ring.data_ptr(), dt_dev.data_ptr(), s)
         # matrix of the all-Neumann diamond operator, then the geometry tables are dropped
-        dd = d.device_diamond
+        dd = DeviceDiamond(dm, host=getattr(d, '_diamond_host', None))
         N = int(d.nbnodes)
         node_dir = torch.zeros(N, dtype=torch.uint8, device=dev)
         rank = torch.full((F,), -1, dtype=torch.int32, device=dev)
         self.arena.assemble_diamond(inst, dd, node_dir, rank)
-        d._device_diamond = None
         row0, _, ns = self.arena.rows(inst)
         self.arena.x[row0:row0 + 64 * ns].zero_()
         self.arena.b[row0:row0 + 64 * ns].zero_()
         self.arena.x[row0:row0 + C] = torch.from_numpy(req.u0).to(dev)
-        self.arena.configure(inst, 1., -req.dt * req.D, tol=self.tol, tol_in=self.tol_inner)
-        req._dev = {'mesh': dm, 'uf': uf, 'vf': vf, 'wf': wf, 'uc': uc, 'vc': vc, 'wc': wc, 'ring': ring,
-                    'row0': row0}
+        arena = self.arena
+        _lib.call('mfv_advection_rows', dm.ptr, uf.data_ptr(), vf.data_ptr(), wf.data_ptr(), row0, 64 * ns,
+                  64 * arena.S, arena.adv_up.shape[0], arena.adv_up.data_ptr(), arena.adv_coef.data_ptr(),
+                  arena.adv_vol.data_ptr(), s)
+        arena.configure(inst, 1., -req.dt * req.D, tol=self.tol, tol_in=self.tol_inner, dt=req.dt)
+        arena._state[:, inst] = torch.tensor([_lib.KS_ADVANCE, req.nsteps], dtype=torch.int32, device=dev)
+        # the arena's rows hold all that the steps need: the mesh tables go with this call; states
+        # of earlier ticks are an earlier instance's
+        req._dev = {'row0': row0, 'tick': self.ticks}
         req.inst = inst
-        req.phase = PHASE_ADVECT
+        req.phase = PHASE_SOLVE
         req.t_admit = now
         self.in_use += req.footprint(self.arena)
         self.active.append(req)
-
-    def _advect(self, req):
-        """u* = u^n + dt * convective(u^n) into b, initial guess x = u*, status START."""
-        a = self.arena
-        g = req._dev
-        row0, C = g['row0'], req.C
-        xs, bs = a.x[row0:row0 + C], a.b[row0:row0 + C]
-        _lib.call('mfv_advection_step', g['mesh'].ptr, xs.data_ptr(), bs.data_ptr(), g['uc'].data_ptr(),
-                  g['vc'].data_ptr(), g['wc'].data_ptr(), g['uf'].data_ptr(), g['vf'].data_ptr(), g['wf'].data_ptr(),
-                  req.cfl, 1, g['ring'].data_ptr(), req.step, None, stream_ptr())
-        xs.copy_(bs)
-        a.status[req.inst] = _lib.KS_START
-        req.phase = PHASE_SOLVE
 
     def _finish(self, req, now, error=None):
         """Retire ``req``: its result (or ``error`` if its solve failed), then its arena
         instance and device tables are released so that the other requests go on."""
         row0 = req._dev['row0']
         if error is None:
-            req.result = self.arena.x[row0:row0 + req.C].cpu().numpy().copy()
+            req.result = self.arena.x[row0:row0 + req.C].cpu().numpy()
         req.iterations = int(self.arena.scalars(req.inst)[_lib.KS_ITTOT])
         self.arena.release(req.inst)
-        self.arena.publish()
         self.in_use -= req.footprint(self.arena)
         req._dev = None
-        req.domain._device_mesh = None
         req.phase = PHASE_DONE if error is None else PHASE_FAILED
         req.error = error
         req.t_done = now
@@ -281,9 +270,6 @@ class ServingEngine(object):
                     elif wait_s > 0:
                         time.sleep(min(wait_s, 0.05))
                     continue
-                for r in self.active:
-                    if r.phase == PHASE_ADVECT:
-                        self._advect(r)
                 if self.time_ticks:
                     ev = (torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))
                     ev[0].record()
@@ -291,24 +277,30 @@ class ServingEngine(object):
                 if self.time_ticks:
                     ev[1].record()
                     self._tick_events.append(ev)
+                self.arena.post_state(self.ticks)
                 self.ticks += 1
-                st = self.arena.status.cpu().numpy()
+                if self.arena.posted() < 2:  # the next tick is queued before this one's outcome is read
+                    continue
+                st, left, tick = self.arena.take_state()
                 now = clock() - t0
+                finished = False
                 for r in list(self.active):
-                    s = st[r.inst]
-                    if s == _lib.KS_DONE:
-                        r.step += 1
-                        if r.step == r.nsteps:
-                            self._finish(r, now)
-                            done.append(r)
-                        else:
-                            r.phase = PHASE_ADVECT
-                    elif s == _lib.KS_FAILED:
+                    if tick < r._dev['tick'] or st[r.inst] not in (_lib.KS_DONE, _lib.KS_FAILED):
+                        continue
+                    r.step = r.nsteps - int(left[r.inst])
+                    if st[r.inst] == _lib.KS_DONE:
+                        self._finish(r, now)
+                    else:
+                        r.step -= 1  # the step that failed, counted from 0
                         self._finish(r, now, error="implicit solve failed at step %d" % r.step)
-                        done.append(r)
+                    done.append(r)
+                    finished = True
+                if finished:
+                    self.arena.publish()
             else:
                 raise _lib.MfvError("serving loop did not finish in %d ticks" % max_ticks)
         finally:
+            self.arena.drop_states()
             pool.shutdown(wait=True)
         torch.cuda.synchronize()
         return done
