@@ -813,7 +813,7 @@ int mfv_krylov_graph(const mfv_ell_batch *e, const mfv_krylov_work *w, int n_ite
 
 /* Work arrays of the two-launch BiCGStab iteration (mfv_krylov_fused_tick). u holds
  * (s, t, p, v) and w (r, v) of a row as one record each, so that a matrix slot costs one record
- * gather. Partial sums are kept per chunk: pa[S], pb[5][S], pr[3][S], the
+ * gather. Partial sums are kept per chunk: pa[S], pb[5][S] (the residual's in its first three), the
  * chunk c of an instance at its first slice + c. chunks[k] = (instance, the instance's first
  * slice, c | chunk count << 16, the instance's slices): chunk c covers the slices
  * [c span, (c + 1) span) of its instance, span = MFV_KRYLOV_SPAN(slices); n_chunks[0] entries,
@@ -822,7 +822,7 @@ typedef struct mfv_krylov_fused {
     double *x, *b;           /* [64 S] FP64 solution and right-hand side */
     float *d, *rh, *dinv, *p; /* [64 S] FP32 inner-solve vectors */
     float *u, *w;            /* [64 S][4] and [64 S][2], 16-byte aligned */
-    double *pa, *pb, *pr;    /* [S], [5][S], [3][S] */
+    double *pa, *pb;         /* [S], [5][S] */
     double *scal;            /* [I][MFV_KS_NSCAL] */
     int32_t *status;         /* [I] */
     int32_t *status_t;       /* [I] (the library's own) */

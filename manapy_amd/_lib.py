@@ -172,7 +172,7 @@ class MfvGradientFields(ctypes.Structure):
 
 class MfvKrylovFused(ctypes.Structure):
     """Mirror of ``struct mfv_krylov_fused`` (include/mfv.h)."""
-    _fields_ = [(k, P) for k in ('x', 'b', 'd', 'rh', 'dinv', 'p', 'u', 'w', 'pa', 'pb', 'pr', 'scal', 'status',
+    _fields_ = [(k, P) for k in ('x', 'b', 'd', 'rh', 'dinv', 'p', 'u', 'w', 'pa', 'pb', 'scal', 'status',
                                  'status_t', 'chunks', 'n_chunks', 'steps_left', 'adv_up', 'adv_coef', 'adv_vol')] + \
         [('adv_slots', ctypes.c_int32), ('pad_', ctypes.c_int32)]
 

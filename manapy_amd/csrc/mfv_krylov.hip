@@ -472,8 +472,9 @@ __global__ void __launch_bounds__(256) k_ell_spmv(Ell e, const double *__restric
 //   w = (r, v) and p; the t product reads those and writes u, so no row writes what another one
 //   reads. With M on the right the v product gathered 20 bytes and held 195 registers, two waves
 //   a SIMD: 12.0 us at 193k rows in eight systems, 8.5 us so.
-// * Measured, v and t product: 6.3 + 5.3 us at 12 800 rows and 8.5 + 7.2 us at 193k rows, against
-//   28 us and 29 us for the eight kernels. What is left is the chain chunk -> columns -> records
+// * Measured, v and t product with all changes of state in them: 7.0 + 6.1 us at 12 800 rows and 8.3 +
+//   8.4 us at 193k rows in eight systems (6.4 + 5.2 and 7.4 + 6.2 us without, and four launches more
+//   a tick), against 28 us and 29 us for the eight kernels. What is left is the chain chunk -> columns -> records
 //   with a trip to memory each, and the fixed cost of adding up.
 // * |r|^2 and rh.r of the new residual follow from the t product's sums (r = s - omega t), so
 //   omega, rho and beta need no third pass; the refinement's own residual stays FP64 and is
@@ -507,7 +508,6 @@ struct Fused {
     float *__restrict__ p;
     double *__restrict__ pa;
     double *__restrict__ pb;
-    double *__restrict__ pr;
     double *__restrict__ scal;
     int32_t *__restrict__ status;
     int32_t *__restrict__ status_t;
@@ -527,7 +527,7 @@ enum { kResidualStart = 16, kResidual, kResidualOfB };
 static Fused to_kernel(const mfv_krylov_fused *w)
 {
     return Fused{w->x,  w->b,  w->d,  w->rh,   w->dinv,   reinterpret_cast<float4 *>(w->u),
-                 reinterpret_cast<float2 *>(w->w), w->p, w->pa, w->pb, w->pr, w->scal, w->status,
+                 reinterpret_cast<float2 *>(w->w), w->p, w->pa, w->pb, w->scal, w->status,
                  w->status_t, reinterpret_cast<const int4 *>(w->chunks), w->n_chunks, w->steps_left, w->adv_up,
                  w->adv_coef, w->adv_vol, w->adv_slots};
 }
@@ -744,26 +744,39 @@ __device__ __forceinline__ void chunk_advance(const Ell &e, const Fused &w, cons
     }
 }
 
-// ell_row64 with its slots in groups of four: the registers of groups of eight would cost the
-// iterations that share the kernel a third of their waves.
+// ell_row64 as the products of the iteration take their slots: the first sixteen (a triangle's row)
+// at once, the columns asked for without waiting for the width, the rest in groups of four. Whatever
+// state the others are in, a launch takes as long as the one system that forms its residual (t product
+// of eight systems 10.8 us on average, 9.9 us so, and 8.4 us behind the loop, see k_fused_t).
 __device__ __forceinline__ double row_product64(const Ell &e, int s, int lane, const double *__restrict__ x)
 {
-    const int wdt = e.slice_w[s], row = s * 64 + lane;
-    const unsigned base = (unsigned)lane;
-    const size_t at = (size_t)s * e.W * 64;
-    const double *__restrict__ vals = e.vals + at;
-    const int16_t *__restrict__ c16 = e.cols16 + at;
-    const int32_t *__restrict__ c32 = e.cols + at;
+    const int row = s * 64 + lane;
+    const size_t base = (size_t)s * e.W * 64 + lane;
+    const int wdt = e.slice_w[s];
     const bool narrow = slice_is_narrow(e, s);
-    double acc = 0.;
-    for (int j = 0; j < wdt; j += 4) {
-        double v[4], xv[4];
-        int c[4];
+    double v[kFirst], xv[kFirst], acc = 0.;
+    int c[kFirst];
+    if (e.cols16) {
+#pragma unroll
+        for (int k = 0; k < kFirst; k++) c[k] = e.cols16[base + (size_t)min(k, e.W - 1) * 64];
+    }
+#pragma unroll
+    for (int k = 0; k < kFirst; k++) v[k] = e.vals[base + (size_t)min(k, e.W - 1) * 64];
+    if (!narrow) {
+#pragma unroll
+        for (int k = 0; k < kFirst; k++) c[k] = e.cols[base + (size_t)min(k, e.W - 1) * 64] - row;
+    }
+#pragma unroll
+    for (int k = 0; k < kFirst; k++) xv[k] = x[row + (k < wdt ? c[k] : 0)];
+#pragma unroll
+    for (int k = 0; k < kFirst; k++)
+        if (k < wdt) acc = fma(v[k], xv[k], acc);
+    for (int j = kFirst; j < wdt; j += 4) {
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            const unsigned q = base + (unsigned)min(j + k, wdt - 1) * 64u;
-            v[k] = vals[q];
-            c[k] = narrow ? row + c16[q] : c32[q];
+            const size_t q = base + (size_t)min(j + k, wdt - 1) * 64;
+            v[k] = e.vals[q];
+            c[k] = narrow ? row + e.cols16[q] : e.cols[q];
         }
 #pragma unroll
         for (int k = 0; k < 4; k++) xv[k] = x[c[k]];
@@ -783,15 +796,13 @@ __device__ __forceinline__ void chunk_residual(const Ell &e, const Fused &w, con
     double sum[3] = {0., 0., 0.};
     for (int s = h.begin + wave_index(); s < h.end; s += kChunkWaves) {
         const int row = s * 64 + lane;
-        float di;
-        if (how == kResidual) {
-            di = w.dinv[row];
-        } else {
-            const double dg = sigma + tau * e.diag[row];
+        const double bb = w.b[row], xx = x[row], diag = e.diag[row];
+        float di = w.dinv[row];
+        const double ax = row_product64(e, s, lane, x);
+        if (how != kResidual) {
+            const double dg = sigma + tau * diag;
             w.dinv[row] = di = (dg != 0.) ? (float)(1. / dg) : 0.f;
         }
-        const double ax = row_product64(e, s, lane, x);
-        const double bb = w.b[row], xx = x[row];
         if (how == kResidualOfB) w.x[row] = xx;
         const double res = bb - (sigma * xx + tau * ax);
         const float r32 = (float)((double)di * res);
@@ -802,7 +813,7 @@ __device__ __forceinline__ void chunk_residual(const Ell &e, const Fused &w, con
         sum[1] += bb * bb;
         sum[2] += (double)r32 * (double)r32;
     }
-    chunk_store<3>(w.pr, e.S, h.s0 + h.c, sum);
+    chunk_store<3>(w.pb, e.S, h.s0 + h.c, sum);  // pb's iteration has been closed
 }
 
 // omega, the new residual's norm and rho, and whether the inner solve ends, from the t product's
@@ -890,11 +901,9 @@ __global__ void __launch_bounds__(kChunkBlock, 3) k_fused_v(Ell e, Fused w)
             chunk_advance(e, w, h, sc[MFV_KS_DT]);
             next = kResidualOfB;
         } else if (status == MFV_KS_CHECK) {
-            double sum[3];
-            chunk_totals<3>(w.pr, e.S, h.s0, h.nch, sum);
             const double tol = sc[MFV_KS_TOL_OUT];
-            if (!isfinite(sum[0]) || !isfinite(sum[1])) next = MFV_KS_FAILED;  // NaN/inf data: refinement cannot help
-            else if (sum[0] <= tol * tol * sum[1]) next = MFV_KS_DONE;
+            if (!isfinite(q[0]) || !isfinite(q[1])) next = MFV_KS_FAILED;  // NaN/inf data: refinement cannot help
+            else if (q[0] <= tol * tol * q[1]) next = MFV_KS_DONE;
             else if (sc[MFV_KS_OUTER] > sc[MFV_KS_MAXIT_OUT]) next = MFV_KS_FAILED;
             else next = MFV_KS_INNER;
             if (next == MFV_KS_DONE && w.steps_left && w.steps_left[h.inst] > 0) {
@@ -902,13 +911,13 @@ __global__ void __launch_bounds__(kChunkBlock, 3) k_fused_v(Ell e, Fused w)
                 next = kResidualOfB;
             }
             if (first) {
-                sc[MFV_KS_RESN2] = sum[0];
-                sc[MFV_KS_BN2] = sum[1];
+                sc[MFV_KS_RESN2] = q[0];
+                sc[MFV_KS_BN2] = q[1];
                 if (next == MFV_KS_INNER) {
-                    sc[MFV_KS_RHO] = sum[2];
-                    sc[MFV_KS_RHO_OLD] = sum[2];
-                    sc[MFV_KS_R0N2] = sum[2];
-                    sc[MFV_KS_RN2] = sum[2];
+                    sc[MFV_KS_RHO] = q[2];
+                    sc[MFV_KS_RHO_OLD] = q[2];
+                    sc[MFV_KS_R0N2] = q[2];
+                    sc[MFV_KS_RN2] = q[2];
                     sc[MFV_KS_ALPHA] = 0.;
                     sc[MFV_KS_OMEGA] = 0.;
                     sc[MFV_KS_BETA] = 0.;
@@ -970,19 +979,7 @@ __global__ void __launch_bounds__(kChunkBlock, 3) k_fused_t(Ell e, Fused w)
         if (s < h.end) take();
         double rv[1];
         chunk_totals<1>(w.pa, e.S, h.s0, h.nch, rv);
-        if (status >= kResidualStart) {
-            if (first) {
-                sc[MFV_KS_OUTER] = (status == kResidual ? sc[MFV_KS_OUTER] : 0.) + 1.;
-                if (status == kResidualOfB) w.steps_left[h.inst] -= 1;
-                w.status[h.inst] = MFV_KS_CHECK;
-            }
-            chunk_residual(e, w, h, status, sc[MFV_KS_SIGMA], sc[MFV_KS_TAU]);
-            continue;
-        }
-        if (status != MFV_KS_INNER) {
-            if (first) w.status[h.inst] = status;
-            continue;
-        }
+        if (status != MFV_KS_INNER) continue;
         const double a = rho / rv[0];
         const bool broken = rv[0] == 0. || !isfinite(a);  // breakdown: refine with what d holds
         if (first) {
@@ -1018,6 +1015,26 @@ __global__ void __launch_bounds__(kChunkBlock, 3) k_fused_t(Ell e, Fused w)
             if (s < h.end) take();
         }
         chunk_store<5>(w.pb, e.S, h.s0 + h.c, sum);
+    }
+    // The block's chunks in another state, behind the loop: with the residual in it the kernel needs 197
+    // registers or spills, 126 so; solves of 12.8k rows took 7.1 us a launch, 6.1 us now.
+#pragma unroll 1
+    for (int k = blockIdx.x; k < n; k += gridDim.x) {
+        const Chunk c = chunk_at(w, k);
+        const int status = w.status_t[c.inst];
+        if (status == MFV_KS_INNER) continue;
+        double *sc = w.scal + (size_t)c.inst * MFV_KS_NSCAL;
+        const bool first = c.c == 0 && threadIdx.x == 0;
+        if (status < kResidualStart) {
+            if (first) w.status[c.inst] = status;
+            continue;
+        }
+        if (first) {
+            sc[MFV_KS_OUTER] = (status == kResidual ? sc[MFV_KS_OUTER] : 0.) + 1.;
+            if (status == kResidualOfB) w.steps_left[c.inst] -= 1;
+            w.status[c.inst] = MFV_KS_CHECK;
+        }
+        chunk_residual(e, w, c, status, sc[MFV_KS_SIGMA], sc[MFV_KS_TAU]);
     }
 }
 
@@ -1106,7 +1123,7 @@ static int check_fused(const mfv_ell_batch *e, const mfv_krylov_fused *w, int n_
 {
     if (int rc = validate_ell(e)) return rc;
     MFV_REQUIRE(w != nullptr, "Krylov work descriptor is NULL");
-    MFV_REQUIRE(w->x && w->b && w->d && w->rh && w->dinv && w->u && w->w && w->p && w->pa && w->pb && w->pr && w->scal &&
+    MFV_REQUIRE(w->x && w->b && w->d && w->rh && w->dinv && w->u && w->w && w->p && w->pa && w->pb && w->scal &&
                     w->status && w->status_t && w->chunks && w->n_chunks,
                 "Krylov work descriptor has NULL pointers");
     MFV_REQUIRE(!w->steps_left || (w->adv_up && w->adv_coef && w->adv_vol && w->adv_slots >= 4 && w->adv_slots % 4 == 0),

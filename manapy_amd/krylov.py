@@ -103,7 +103,7 @@ class EllBatch(object):
         self.b = torch.zeros(R, dtype=f64, device=dev)
         self.f32 = {k: torch.zeros(R, dtype=f32, device=dev) for k in ('d', 'rh', 'dinv', 'p')}
         self.f32.update({k: torch.zeros((R, n), dtype=f32, device=dev) for k, n in (('u', 4), ('w', 2))})
-        self.partial = {k: torch.zeros(S * n, dtype=f64, device=dev) for k, n in (('pa', 1), ('pb', 5), ('pr', 3))}
+        self.partial = {k: torch.zeros(S * n, dtype=f64, device=dev) for k, n in (('pa', 1), ('pb', 5))}
         self.chunks = torch.zeros((S, 4), dtype=i32, device=dev)
         self.n_chunks = torch.zeros(1, dtype=i32, device=dev)
         self.scal = torch.zeros(I * _lib.KS_NSCAL, dtype=f64, device=dev)
