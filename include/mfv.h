@@ -615,6 +615,16 @@ typedef struct mfv_euler_tet_tiles {
 int mfv_euler3d_step_packed_tiled(const mfv_mesh *m, const mfv_euler_tet *t, const mfv_euler_tet_tiles *tt,
                                   const double *rec_in, double *rec_out, double gamma, double cfl, int quirk,
                                   double *dt_ring, int step, void *stream);
+/* nsteps of that step (ring steps 0 .. nsteps - 1) between rec_a (the start) and rec_b; the result
+ * is in rec_a for even nsteps, else in rec_b. cell_rank: mfv_euler_tet's. Same bits. */
+int mfv_euler3d_run_packed_tiled(const mfv_mesh *m, const uint8_t *cell_rank, const mfv_euler_tet_tiles *tt,
+                                 double *rec_a, double *rec_b, double gamma, double cfl, int quirk,
+                                 double *dt_ring, int nsteps, void *stream);
+/* Records in another cell order (record i is cell perm[i] of the mesh and of U) with the state's
+ * time step, and the records' states back to U. */
+int mfv_euler3d_load(const mfv_mesh *m, const double *U, const int64_t *perm, double cfl, double gamma,
+                     double *rec, double *dt_dev, void *stream);
+int mfv_euler3d_store(const mfv_mesh *m, const double *rec, const int64_t *perm, double *U, void *stream);
 /* The same step on the same tiles with one cell phase: after staging the records, each cell
  * evaluates its own four faces' fluxes (an inner face of two tile cells is evaluated by both,
  * from the same arguments), so the LDS holds only the records (48 * max_items bytes <= 64 KiB)

@@ -269,6 +269,9 @@ _SIGNATURES = {
     'mfv_euler3d_unpack': [MESH_P, P, P, P],
     'mfv_euler3d_step_packed': [MESH_P, ET_P, P, P, c_double, c_double, c_int, P, c_int, P],
     'mfv_euler3d_step_packed_tiled': [MESH_P, ET_P, ETT_P, P, P, c_double, c_double, c_int, P, c_int, P],
+    'mfv_euler3d_run_packed_tiled': [MESH_P, P, ETT_P, P, P, c_double, c_double, c_int, P, c_int, P],
+    'mfv_euler3d_load': [MESH_P, P, P, c_double, c_double, P, P, P],
+    'mfv_euler3d_store': [MESH_P, P, P, P, P],
     'mfv_euler3d_step_cells_tiled': [MESH_P, ET_P, ETT_P, P, P, c_double, c_double, c_int, P, c_int, P],
     'mfv_euler32_pack': [MESH_P, P, P, P],
     'mfv_euler32_unpack': [MESH_P, P, P, P],

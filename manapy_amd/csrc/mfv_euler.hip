@@ -504,7 +504,9 @@ template <int T>
 __global__ void __launch_bounds__(T) k_euler_step_packed_tiled(EulerTetK t, EulerTilesK tt,
                                                                 const double *__restrict__ Rin,
                                                                 double *__restrict__ Rout, double gamma, double cfl,
-                                                                int quirk, DtRing ring, double *__restrict__ dtpart)
+                                                                int quirk, DtRing ring,
+                                                                const double *__restrict__ fold, int nfold,
+                                                                double *__restrict__ dtpart)
 {
     extern __shared__ double lds[];
     double2 *sR = reinterpret_cast<double2 *>(lds);  // [T][3]: the tile cells' six values
@@ -513,7 +515,7 @@ __global__ void __launch_bounds__(T) k_euler_step_packed_tiled(EulerTetK t, Eule
     const int c0 = tt.cell0[tile], nc = tt.ncells[tile];
     const int h0 = tt.hptr[tile];
     const int f0 = tt.fptr[tile], nfc = tt.fptr[tile + 1] - f0;
-    ring_advance(ring);
+    const double dt = step_dt(ring, fold, nfold);
     double vol = 0.;  // the thread's cell's volume, kept from its record for the update
     if ((int)threadIdx.x < nc) {
         const double2 *rp = reinterpret_cast<const double2 *>(Rin + 8 * (size_t)(c0 + threadIdx.x));
@@ -582,7 +584,7 @@ __global__ void __launch_bounds__(T) k_euler_step_packed_tiled(EulerTetK t, Eule
         }
         const double2 oa = sR[3 * q], ob = sR[3 * q + 1], oc = sR[3 * q + 2];
         double u[6] = {oa.x, oa.y, ob.x, ob.y, oc.x, oc.y};
-        euler_update_cell(u, r, gamma, ring.cur[0], vol);
+        euler_update_cell(u, r, gamma, dt, vol);
         double2 *wp = reinterpret_cast<double2 *>(Rout + 8 * (size_t)i);
         wp[0] = make_double2(u[0], u[1]);
         wp[1] = make_double2(u[2], u[3]);
@@ -1005,6 +1007,47 @@ __global__ void __launch_bounds__(kBlock) k_euler_unpack(int C, const double *__
     U[3 * n + i] = b.y;
     U[4 * n + i] = e.x;
     U[5 * n + i] = e.y;
+}
+
+// The records in another cell order (record i is cell perm[i]) and the dt of the state, which this
+// pass over U and the faces has in hand (1.6M cells: 99 us, as k_euler_dt and k_euler_pack in the
+// mesh's own order).
+__global__ void __launch_bounds__(kBlock) k_euler_load(Mesh m, const double *__restrict__ U,
+                                                       const int64_t *__restrict__ perm, double cfl, double gamma,
+                                                       double *__restrict__ rec, double *__restrict__ dtpart)
+{
+    const int i = xcd_block() * blockDim.x + threadIdx.x;
+    double d = 1e300;
+    if (i < m.C) {
+        const size_t n = m.C;
+        const int q = (int)perm[i];
+        double u[6];
+#pragma unroll
+        for (int v = 0; v < 6; v++) u[v] = U[v * n + q];
+        double2 *w = reinterpret_cast<double2 *>(rec + 8 * (size_t)i);
+        w[0] = make_double2(u[0], u[1]);
+        w[1] = make_double2(u[2], u[3]);
+        w[2] = make_double2(u[4], u[5]);
+        w[3] = make_double2(m.cell_volume[q], 0.);
+        d = euler_cell_dt(m, q, u[0], u[1], u[2], u[3], u[4], cfl, gamma);
+    }
+    wave_min_part(dtpart, (size_t)i, d);
+}
+
+__global__ void __launch_bounds__(kBlock) k_euler_store(int C, const double *__restrict__ rec,
+                                                        const int64_t *__restrict__ perm, double *__restrict__ U)
+{
+    const int i = xcd_block() * blockDim.x + threadIdx.x;
+    if (i >= C) return;
+    const size_t n = C, q = (size_t)perm[i];
+    const double2 *p = reinterpret_cast<const double2 *>(rec + 8 * (size_t)i);
+    const double2 a = p[0], b = p[1], e = p[2];
+    U[q] = a.x;
+    U[n + q] = a.y;
+    U[2 * n + q] = b.x;
+    U[3 * n + q] = b.y;
+    U[4 * n + q] = e.x;
+    U[5 * n + q] = e.y;
 }
 
 // The fused step on face tiles (mfv_face_tiles): the block stages the states of its cells and
@@ -1445,6 +1488,33 @@ extern "C" int mfv_euler3d_unpack(const mfv_mesh *m, const double *rec, double *
     return check_launch("k_euler_unpack");
 }
 
+extern "C" int mfv_euler3d_load(const mfv_mesh *m, const double *U, const int64_t *perm, double cfl, double gamma,
+                                double *rec, double *dt_dev, void *stream)
+{
+    if (int rc = validate_mesh(m, 0, 0, 0)) return rc;
+    MFV_REQUIRE(m->dim == 3 && m->max_cell_faces >= 4, "Euler 3D needs tetrahedra");
+    MFV_REQUIRE(U && perm && rec && dt_dev && ((uintptr_t)rec & 15) == 0, "NULL or misaligned array");
+    const size_t nw = m->nb_cells ? waves_for(m->nb_cells) : 0;
+    double *part = nullptr;
+    if (nw) {
+        part = dt_scratch(nw, as_stream(stream));
+        if (!part) return MFV_ENOMEM;
+        hipLaunchKernelGGL(k_euler_load, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream), to_kernel(m),
+                           U, perm, cfl, gamma, rec, part);
+    }
+    return dt_total(part, nw, dt_dev, nullptr, as_stream(stream));
+}
+
+extern "C" int mfv_euler3d_store(const mfv_mesh *m, const double *rec, const int64_t *perm, double *U, void *stream)
+{
+    if (int rc = validate_mesh(m, 0, 0, 0)) return rc;
+    if (m->nb_cells == 0) return MFV_OK;
+    MFV_REQUIRE(U && perm && rec && ((uintptr_t)rec & 15) == 0, "NULL or misaligned array");
+    hipLaunchKernelGGL(k_euler_store, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream), m->nb_cells, rec,
+                       perm, U);
+    return check_launch("k_euler_store");
+}
+
 extern "C" int mfv_euler3d_step_packed(const mfv_mesh *m, const mfv_euler_tet *t, const double *rec_in,
                                        double *rec_out, double gamma, double cfl, int quirk, double *dt_ring_p,
                                        int step, void *stream)
@@ -1489,6 +1559,38 @@ static int check_euler_tiles(const mfv_mesh *m, const mfv_euler_tet_tiles *tt, s
     return MFV_OK;
 }
 
+// fold, nfold: see step_dt (the face-phase kernel only).
+static int launch_euler_tiled(bool cells, const uint8_t *rank, const mfv_euler_tet_tiles *tt, size_t lds,
+                              const double *rec_in, double *rec_out, double gamma, double cfl, int quirk, DtRing r,
+                              const double *fold, int nfold, double *part, hipStream_t st)
+{
+    const EulerTetK tk{nullptr, rank, nullptr, 0};  // these kernels take the rest from the tiles
+    const EulerTilesK ek{tt->tile_cell0,
+                         tt->tile_ncells,
+                         tt->halo_ptr,
+                         tt->halo_cells,
+                         tt->face_ptr,
+                         reinterpret_cast<const double2 *>(tt->face_geo),
+                         reinterpret_cast<const int2 *>(tt->face_lr),
+                         reinterpret_cast<const int4 *>(tt->cell_code),
+                         tt->max_items,
+                         tt->max_faces};
+#define MFV_EULER_TILED(TS)                                                                                           \
+    if (cells)                                                                                                        \
+        hipLaunchKernelGGL(k_euler_step_cells_tiled<TS>, dim3(tt->nb_tiles), dim3(TS), lds, st, tk, ek, rec_in,       \
+                           rec_out, gamma, cfl, quirk, r, part);                                                      \
+    else                                                                                                              \
+        hipLaunchKernelGGL(k_euler_step_packed_tiled<TS>, dim3(tt->nb_tiles), dim3(TS), lds, st, tk, ek, rec_in,      \
+                           rec_out, gamma, cfl, quirk, r, fold, nfold, part)
+    switch (tt->tile_size) {
+    case 128: MFV_EULER_TILED(128); break;
+    case 256: MFV_EULER_TILED(256); break;
+    default: MFV_EULER_TILED(512); break;
+    }
+#undef MFV_EULER_TILED
+    return check_launch(cells ? "k_euler_step_cells_tiled" : "k_euler_step_packed_tiled");
+}
+
 static int euler_step_packed_tiled(bool cells, const mfv_mesh *m, const mfv_euler_tet *t,
                                    const mfv_euler_tet_tiles *tt, const double *rec_in, double *rec_out, double gamma,
                                    double cfl, int quirk, double *dt_ring_p, int step, void *stream)
@@ -1510,37 +1612,9 @@ static int euler_step_packed_tiled(bool cells, const mfv_mesh *m, const mfv_eule
     hipStream_t st = as_stream(stream);
     double *part = dt_scratch(nw, st);
     if (!part) return MFV_ENOMEM;
-    const EulerTetK tk{reinterpret_cast<const int4 *>(t->cell_nb), t->cell_rank,
-                       reinterpret_cast<const double2 *>(t->cell_geo), (size_t)m->nb_cells};
-    const EulerTilesK ek{tt->tile_cell0,
-                         tt->tile_ncells,
-                         tt->halo_ptr,
-                         tt->halo_cells,
-                         tt->face_ptr,
-                         reinterpret_cast<const double2 *>(tt->face_geo),
-                         reinterpret_cast<const int2 *>(tt->face_lr),
-                         reinterpret_cast<const int4 *>(tt->cell_code),
-                         tt->max_items,
-                         tt->max_faces};
-#define MFV_EULER_TILED(K, TS)                                                                                        \
-    hipLaunchKernelGGL(K<TS>, dim3(tt->nb_tiles), dim3(TS), lds, st, tk, ek, rec_in, rec_out, gamma, cfl, quirk, r, \
-                       part)
-    switch (tt->tile_size) {
-    case 128:
-        if (cells) MFV_EULER_TILED(k_euler_step_cells_tiled, 128);
-        else MFV_EULER_TILED(k_euler_step_packed_tiled, 128);
-        break;
-    case 256:
-        if (cells) MFV_EULER_TILED(k_euler_step_cells_tiled, 256);
-        else MFV_EULER_TILED(k_euler_step_packed_tiled, 256);
-        break;
-    default:
-        if (cells) MFV_EULER_TILED(k_euler_step_cells_tiled, 512);
-        else MFV_EULER_TILED(k_euler_step_packed_tiled, 512);
-        break;
-    }
-#undef MFV_EULER_TILED
-    if (int rc = check_launch(cells ? "k_euler_step_cells_tiled" : "k_euler_step_packed_tiled")) return rc;
+    if (int rc = launch_euler_tiled(cells, t->cell_rank, tt, lds, rec_in, rec_out, gamma, cfl, quirk, r, nullptr, 0,
+                                    part, st))
+        return rc;
     return dt_finish(part, nw, r.next, st);
 }
 
@@ -1549,6 +1623,37 @@ extern "C" int mfv_euler3d_step_packed_tiled(const mfv_mesh *m, const mfv_euler_
                                              int quirk, double *dt_ring_p, int step, void *stream)
 {
     return euler_step_packed_tiled(false, m, t, tt, rec_in, rec_out, gamma, cfl, quirk, dt_ring_p, step, stream);
+}
+
+// nsteps steps between rec_a and rec_b; up to kFoldMax partials a step folds its predecessor's.
+extern "C" int mfv_euler3d_run_packed_tiled(const mfv_mesh *m, const uint8_t *cell_rank,
+                                            const mfv_euler_tet_tiles *tt, double *rec_a, double *rec_b, double gamma,
+                                            double cfl, int quirk, double *dt_ring_p, int nsteps, void *stream)
+{
+    if (int rc = validate_mesh(m, 0, 0, 0)) return rc;
+    MFV_REQUIRE(m->dim == 3, "the packed Euler step needs a 3D mesh");
+    if (!tt) return check_euler_tiles(m, tt, 0);
+    const size_t lds = 48 * (size_t)tt->tile_size + 40 * (size_t)tt->max_faces;
+    if (int rc = check_euler_tiles(m, tt, lds)) return rc;
+    MFV_REQUIRE(nsteps >= 0, "nsteps < 0");
+    MFV_REQUIRE(cell_rank && rec_a && rec_b && rec_a != rec_b && dt_ring_p, "NULL or aliased array");
+    MFV_REQUIRE((((uintptr_t)rec_a | (uintptr_t)rec_b) & 15) == 0, "misaligned records");
+    if (m->nb_cells == 0 || nsteps == 0) return MFV_OK;
+    const size_t nw = ((size_t)m->nb_cells + 63) / 64;
+    const bool fold = nw <= (size_t)kFoldMax;
+    hipStream_t st = as_stream(stream);
+    double *part = dt_scratch(fold ? 2 * nw : nw, st);
+    if (!part) return MFV_ENOMEM;
+    for (int k = 0; k < nsteps; k++) {
+        const DtRing r = dt_ring(dt_ring_p, k);
+        double *mine = part + (fold && (k & 1) ? nw : 0), *last = part + (fold && !(k & 1) ? nw : 0);
+        if (int rc = launch_euler_tiled(false, cell_rank, tt, lds, k & 1 ? rec_b : rec_a, k & 1 ? rec_a : rec_b, gamma,
+                                        cfl, quirk, r, last, fold && k > 0 ? (int)nw : 0, mine, st))
+            return rc;
+        if (!fold || k == nsteps - 1)
+            if (int rc = dt_finish(mine, nw, r.next, st)) return rc;
+    }
+    return MFV_OK;
 }
 
 extern "C" int mfv_euler3d_step_cells_tiled(const mfv_mesh *m, const mfv_euler_tet *t, const mfv_euler_tet_tiles *tt,

@@ -20,6 +20,7 @@ import ctypes
 import numpy as np
 
 from . import _lib
+from .base import Struct
 
 I32 = np.int32
 
@@ -689,6 +690,43 @@ def euler_tet_tiles_host(H, T):
                               'halo_cells', 'face_ptr')}
     out.update({'face_geo': geo, 'face_lr': lr, 'cell_code': code, 'face_id': ft['face_id'][perm]})
     return out
+
+
+def euler_run_layout(H, perm):
+    """What the tiled Euler step needs of a gpu_layout ``H`` with its cells in ``perm`` order
+    (perm[new] = old), faces as they are."""
+    iperm = np.empty(len(perm), dtype=I32)
+    iperm[perm] = np.arange(len(perm), dtype=I32)
+    fc = H['face_cells']
+    out = {k: np.ascontiguousarray(H[k][:, perm]) for k in ('cell_faces', 'order_sorted')}
+    out['cell_nfaces'] = np.ascontiguousarray(H['cell_nfaces'][perm])
+    out['face_cells'] = np.where(fc >= 0, iperm[np.maximum(fc, 0)], -1).astype(I32)
+    out.update({k: H[k] for k in ('face_name', 'face_normal', 'face_mesure')})
+    return out
+
+
+class EulerRunMesh(object):
+    """A tetrahedral mesh as EulerSolver3D.run takes it: cells in Morton order (a relabelling: same
+    bits), on the largest face tiles whose LDS fits (``tiles`` is None where none does). The curve
+    makes the tiles compact: in a generator's row-major order a tile of 256 cells touches 684 faces
+    and 339 cells outside it, 637 and 223 so; the step of 1.6M cells 149 -> 136 us."""
+
+    def __init__(self, dmesh):
+        import torch
+        from .renumber import morton_order_3d
+        H = dmesh.host
+        perm = morton_order_3d(*H['cell_center'].T)
+        R = Struct(host=euler_run_layout(H, perm), device=dmesh.device, MF=dmesh.MF)
+        order = R.host['order_sorted'].astype(np.uint8)
+        rank = order[0] | (order[1] << 2) | (order[2] << 4) | (order[3] << 6)
+        self.perm = torch.as_tensor(perm.astype(np.int64), device=dmesh.device)
+        self.rank = torch.as_tensor(rank, device=dmesh.device)
+        self.tiles = None
+        for T in (256, 128):
+            cand = EulerTetTiles(R, T)
+            if cand.lds_bytes() <= 64 * 1024:
+                self.tiles = cand
+                break
 
 
 class EulerTetTiles(object):
