@@ -569,6 +569,16 @@ struct BatchK {
     double *__restrict__ rings;
 };
 
+// How a tiled ensemble step comes by an instance's dt: from its ring (part NULL), or as the minimum of
+// the partials that the step before left at part[wave], which saves a launch of k_batch_dt_fold a
+// step; advance: the step also keeps the ring (k_batch_dt_fold does it otherwise). lds: byte offset
+// of the block's T / 64 doubles for it.
+struct BatchFold {
+    const double *part;
+    int advance;
+    unsigned lds;
+};
+
 // Each wave stores its dt minimum at part[global wave] (wave w covers cells 64w..64w+63);
 // k_batch_dt_fold then reduces the waves of each instance.
 template <int MF, int BS>
@@ -800,7 +810,7 @@ struct StagedCells {
 template <int MF, int T, bool BATCH, bool STAGED, int KMAX>
 __global__ void __launch_bounds__(T) k_sw_step32_tiled(Mesh m, mfv_sw_mixed p, TilesK t, double4 *__restrict__ out,
                                                        float g, double cfl, float om, DtRing ring, BatchK b,
-                                                       int kcur, double *__restrict__ part)
+                                                       int kcur, BatchFold fold, double *__restrict__ part)
 {
     extern __shared__ double4 lds4[];
     double4 *s_st = lds4;                                       // [E] when STAGED
@@ -812,6 +822,20 @@ __global__ void __launch_bounds__(T) k_sw_step32_tiled(Mesh m, mfv_sw_mixed p, T
     const size_t r0 = t.iptr[tile];
     const double4 *__restrict__ st = reinterpret_cast<const double4 *>(p.state);
     if (!BATCH) ring_advance(ring);
+    // The instance's dt, folded by the whole block: the loads leave with the staging's, the waves'
+    // minima meet in LDS at the barrier that the staging needs anyway.
+    const int inst = BATCH ? b.wave_inst[c0 >> 6] : 0;
+    double fm = 1e6;
+    if (BATCH && fold.part) {
+        const int w0 = b.inst_cell0[inst] >> 6, w1 = (b.inst_cell0[inst] + b.inst_ncells[inst] + 63) >> 6;
+        for (int w = w0 + (int)threadIdx.x; w < w1; w += 4 * T) {
+            double v[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[k] = fold.part[min(w + k * T, w1 - 1)];
+#pragma unroll
+            for (int k = 0; k < 4; k++) fm = (v[k] < fm) ? v[k] : fm;
+        }
+    }
     if (STAGED) {
         for (int e = threadIdx.x; e < nc + ne; e += 2 * T) {  // two cells per pass: one latency for both
             const int2 c = tile_ext_pair(t.ext, c0, nc, e0, ne, e, T);
@@ -824,7 +848,34 @@ __global__ void __launch_bounds__(T) k_sw_step32_tiled(Mesh m, mfv_sw_mixed p, T
             s_st[eb] = sb;
             s_cc[eb] = pb;
         }
-        __syncthreads();
+    }
+    double *s_dt = reinterpret_cast<double *>(reinterpret_cast<char *>(lds4) + fold.lds);  // [T / 64]
+    if (BATCH && fold.part) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const double o = __shfl_xor(fm, off, 64);
+            fm = (o < fm) ? o : fm;
+        }
+        if ((threadIdx.x & 63) == 0) s_dt[threadIdx.x >> 6] = fm;
+    }
+    if (STAGED || (BATCH && fold.part)) __syncthreads();
+    double dt = 0.;
+    if (BATCH) {
+        double *ring_i = b.rings + 4 * (size_t)inst;
+        if (fold.part) {
+            dt = s_dt[0];
+#pragma unroll
+            for (int k = 1; k < T / 64; k++) dt = (s_dt[k] < dt) ? s_dt[k] : dt;
+        } else {
+            dt = ring_i[kcur];
+        }
+        if (fold.advance && c0 == b.inst_cell0[inst] && threadIdx.x == 0) {  // the instance's first tile
+            if (fold.part) ring_i[kcur] = dt;
+            ring_i[(kcur + 2) % 3] = 1e6;
+            ring_i[3] += dt;
+        }
+    } else {
+        dt = ring.cur[0];
     }
     // A tile cell is reconstructed and updated by the same thread (q = threadIdx.x is in the
     // first pass), which keeps the cell's slot geometry in registers for the flux phase.
@@ -853,7 +904,6 @@ __global__ void __launch_bounds__(T) k_sw_step32_tiled(Mesh m, mfv_sw_mixed p, T
     double dloc = 1e300;
     if (q < nc) {
         const int i = c0 + q;
-        const double dt = BATCH ? b.rings[4 * (size_t)b.wave_inst[i >> 6] + kcur] : ring.cur[0];
         const int32_t *__restrict__ lnbr = t.lnbr;
         const size_t C = m.C;
         // staged: the codes of t.lnbr (the tile cell's lfn row) and the face count kept from the
@@ -904,41 +954,45 @@ TilesK to_tiles(const mfv_sw_tiles *t)
 
 template <int MF, int T, bool BATCH, bool STAGED>
 void launch_tiled(const Mesh &mk, const mfv_sw_mixed &p, const TilesK &tk, size_t lds, double *out, float g,
-                  double cfl, float om, DtRing r, const BatchK &bk, int kcur, double *part, hipStream_t st)
+                  double cfl, float om, DtRing r, const BatchK &bk, int kcur, BatchFold fold, double *part,
+                  hipStream_t st)
 {
     if (kmax_for(mk.K) == 16)
         hipLaunchKernelGGL((k_sw_step32_tiled<MF, T, BATCH, STAGED, 16>), dim3(tk.n), dim3(T), lds, st, mk, p, tk,
-                           reinterpret_cast<double4 *>(out), g, cfl, om, r, bk, kcur, part);
+                           reinterpret_cast<double4 *>(out), g, cfl, om, r, bk, kcur, fold, part);
     else
         hipLaunchKernelGGL((k_sw_step32_tiled<MF, T, BATCH, STAGED, 0>), dim3(tk.n), dim3(T), lds, st, mk, p, tk,
-                           reinterpret_cast<double4 *>(out), g, cfl, om, r, bk, kcur, part);
+                           reinterpret_cast<double4 *>(out), g, cfl, om, r, bk, kcur, fold, part);
 }
 
 template <int MF, bool BATCH, bool STAGED>
 void launch_tiled_t(const Mesh &mk, const mfv_sw_mixed &p, const TilesK &tk, size_t lds, double *out, float g,
-                    double cfl, float om, DtRing r, const BatchK &bk, int kcur, double *part, hipStream_t st)
+                    double cfl, float om, DtRing r, const BatchK &bk, int kcur, BatchFold fold, double *part,
+                    hipStream_t st)
 {
     switch (tk.T) {
-    case 128: launch_tiled<MF, 128, BATCH, STAGED>(mk, p, tk, lds, out, g, cfl, om, r, bk, kcur, part, st); break;
-    case 256: launch_tiled<MF, 256, BATCH, STAGED>(mk, p, tk, lds, out, g, cfl, om, r, bk, kcur, part, st); break;
-    default: launch_tiled<MF, 512, BATCH, STAGED>(mk, p, tk, lds, out, g, cfl, om, r, bk, kcur, part, st); break;
+    case 128: launch_tiled<MF, 128, BATCH, STAGED>(mk, p, tk, lds, out, g, cfl, om, r, bk, kcur, fold, part, st); break;
+    case 256: launch_tiled<MF, 256, BATCH, STAGED>(mk, p, tk, lds, out, g, cfl, om, r, bk, kcur, fold, part, st); break;
+    default: launch_tiled<MF, 512, BATCH, STAGED>(mk, p, tk, lds, out, g, cfl, om, r, bk, kcur, fold, part, st); break;
     }
 }
 
 template <bool BATCH>
 int tiled_step(const mfv_mesh *m, const mfv_sw_mixed *p, const mfv_sw_tiles *t, double *out, float g, double cfl,
-               float om, DtRing r, const BatchK &bk, int kcur, double *part, hipStream_t st)
+               float om, DtRing r, const BatchK &bk, int kcur, BatchFold fold, double *part, hipStream_t st)
 {
     const Mesh mk = to_kernel(m);
     const TilesK tk = to_tiles(t);
-    const size_t lds = tiles_lds_bytes(t, m->max_cell_faces);
+    const size_t own = tiles_lds_bytes(t, m->max_cell_faces);
+    fold.lds = (unsigned)own;
+    const size_t lds = own + (fold.part ? (t->tile_size / 64) * sizeof(double) : 0);
     const bool four = m->max_cell_faces == 4;
     if (t->stage_states) {
-        if (four) launch_tiled_t<4, BATCH, true>(mk, *p, tk, lds, out, g, cfl, om, r, bk, kcur, part, st);
-        else launch_tiled_t<3, BATCH, true>(mk, *p, tk, lds, out, g, cfl, om, r, bk, kcur, part, st);
+        if (four) launch_tiled_t<4, BATCH, true>(mk, *p, tk, lds, out, g, cfl, om, r, bk, kcur, fold, part, st);
+        else launch_tiled_t<3, BATCH, true>(mk, *p, tk, lds, out, g, cfl, om, r, bk, kcur, fold, part, st);
     } else {
-        if (four) launch_tiled_t<4, BATCH, false>(mk, *p, tk, lds, out, g, cfl, om, r, bk, kcur, part, st);
-        else launch_tiled_t<3, BATCH, false>(mk, *p, tk, lds, out, g, cfl, om, r, bk, kcur, part, st);
+        if (four) launch_tiled_t<4, BATCH, false>(mk, *p, tk, lds, out, g, cfl, om, r, bk, kcur, fold, part, st);
+        else launch_tiled_t<3, BATCH, false>(mk, *p, tk, lds, out, g, cfl, om, r, bk, kcur, fold, part, st);
     }
     return check_launch("k_sw_step32_tiled");
 }
@@ -1145,23 +1199,36 @@ extern "C" int mfv_sw_step_mixed_tiled(const mfv_mesh *m, const mfv_sw_mixed *p,
     double *part = dt_scratch(nw, as_stream(stream));
     if (!part) return MFV_ENOMEM;
     const BatchK none{0, 0, nullptr, nullptr, nullptr, nullptr};
-    if (int rc = tiled_step<false>(m, p, t, state_out, (float)grav, cfl, (float)(order - 1), r, none, 0, part,
-                                   as_stream(stream)))
+    if (int rc = tiled_step<false>(m, p, t, state_out, (float)grav, cfl, (float)(order - 1), r, none, 0,
+                                   BatchFold{nullptr, 0, 0}, part, as_stream(stream)))
         return rc;
     return dt_finish(part, nw, r.next, as_stream(stream));
 }
 
+// One step; ``closed``: with the fold of its partials (else the next step's, or the caller's).
 static int batch_tiled_launch(const mfv_mesh *m, const mfv_sw_mixed *p, const mfv_sw_batch *b,
                               const mfv_sw_tiles *t, double *out, float g, double cfl, float om, int step,
-                              double *part, hipStream_t st)
+                              BatchFold fold, bool closed, double *part, hipStream_t st)
 {
     const int k = ((step % 3) + 3) % 3;
     const BatchK bk = to_batch(b);
     const DtRing none{};
-    if (int rc = tiled_step<true>(m, p, t, out, g, cfl, om, none, bk, k, part, st)) return rc;
+    if (int rc = tiled_step<true>(m, p, t, out, g, cfl, om, none, bk, k, fold, part, st)) return rc;
+    if (!closed) return MFV_OK;
     hipLaunchKernelGGL(k_batch_dt_fold, dim3(fold_grid(b->nb_inst)), dim3(256), 0, st, part, bk, k, (k + 1) % 3,
-                       (k + 2) % 3, 1);
+                       (k + 2) % 3, fold.advance ? 0 : 1);
     return check_launch("k_batch_dt_fold");
+}
+
+// Whether the steps of a graph fold the dt themselves: every tile reads its instance's partials, so
+// all tiles together must read little beside the step's own traffic (300 bytes a cell). 30 steps: four
+// instances of 31k cells together 358 -> 309 us, eight of 93k 458 -> 389 us, 24 of 615k (3222 tiles,
+// 10 MB) 1331 -> 1314 us.
+static bool batch_folds(const mfv_mesh *m, const mfv_sw_batch *b, const mfv_sw_tiles *t)
+{
+    const double bytes = 8. * t->nb_tiles * ((double)b->nb_waves / b->nb_inst);
+    return bytes <= 64e6 && bytes <= 30. * m->nb_cells &&
+           tiles_lds_bytes(t, m->max_cell_faces) + (t->tile_size / 64) * sizeof(double) <= 64 * 1024;
 }
 
 extern "C" int mfv_sw_batch_step_tiled(const mfv_mesh *m, const mfv_sw_mixed *p, const mfv_sw_batch *b,
@@ -1176,8 +1243,8 @@ extern "C" int mfv_sw_batch_step_tiled(const mfv_mesh *m, const mfv_sw_mixed *p,
     if (m->nb_cells == 0) return MFV_OK;
     double *part = dt_scratch((size_t)m->nb_cells / 64, as_stream(stream));
     if (!part) return MFV_ENOMEM;
-    return batch_tiled_launch(m, p, b, t, state_out, (float)grav, cfl, (float)(order - 1), step, part,
-                              as_stream(stream));
+    return batch_tiled_launch(m, p, b, t, state_out, (float)grav, cfl, (float)(order - 1), step,
+                              BatchFold{nullptr, 0, 0}, true, part, as_stream(stream));
 }
 
 extern "C" int mfv_sw_batch_graph_tiled(const mfv_mesh *m, const mfv_sw_mixed *p, const mfv_sw_batch *b,
@@ -1194,7 +1261,9 @@ extern "C" int mfv_sw_batch_graph_tiled(const mfv_mesh *m, const mfv_sw_mixed *p
                 nsteps);
     *graph_out = nullptr;
     MfvGraph *g = new MfvGraph();
-    hipError_t e = hipMalloc(reinterpret_cast<void **>(&g->part), ((size_t)m->nb_cells / 64 + 1) * sizeof(double));
+    const bool folds = batch_folds(m, b, t);
+    const size_t nw = (size_t)m->nb_cells / 64 + 1;
+    hipError_t e = hipMalloc(reinterpret_cast<void **>(&g->part), (folds ? 2 : 1) * nw * sizeof(double));
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipStreamBeginCapture(g->stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) {
@@ -1209,7 +1278,10 @@ extern "C" int mfv_sw_batch_graph_tiled(const mfv_mesh *m, const mfv_sw_mixed *p
     for (int k = 0; k < nsteps && rc == MFV_OK; k++) {
         const mfv_sw_mixed &pin = (k % 2 == 0) ? pa : pb;
         double *out = (k % 2 == 0) ? state2 : p->state;
-        rc = batch_tiled_launch(m, &pin, b, t, out, (float)grav, cfl, (float)(order - 1), k, g->part, g->stream);
+        double *mine = g->part + (folds && (k & 1) ? nw : 0), *last = g->part + (k & 1 ? 0 : nw);
+        const BatchFold fold{folds && k > 0 ? last : nullptr, folds, 0};
+        rc = batch_tiled_launch(m, &pin, b, t, out, (float)grav, cfl, (float)(order - 1), k, fold,
+                                !folds || k == nsteps - 1, mine, g->stream);
     }
     e = hipStreamEndCapture(g->stream, &g->graph);
     if (rc != MFV_OK || e != hipSuccess) {
