@@ -217,6 +217,27 @@ int mfv_update_sw5(const mfv_mesh *m, double *h_c, double *hu_c, double *hv_c, d
                    const double *corio_hu, const double *corio_hv, double wind_hu, double wind_hv,
                    double dtime, const double *dt_dev, void *stream);
 
+/* What mfv_srnh_run works on: the five fields (h, hu, hv, hc, Z) and a second set of them, their
+ * ghost values [F] and the segments that fill them (mfv_ghost_values; w of the kinds that read the
+ * cells points into cell), the gradients and limiters of h and hc, the arrays of mfv_update_sw5
+ * and mfv_term_source_srnh_sw, and a face record each for the fluxes. */
+typedef struct mfv_srnh_step {
+    double *cell[5], *cell2[5], *ghost[5];
+    const struct mfv_ghost_seg *segs;
+    double *h_x, *h_y, *h_z, *h_psi, *hc_x, *hc_y, *hc_z, *hc_psi;
+    const double *dissip_hc, *corio_hu, *corio_hv;
+    double *flux; /* [F][4], 32-byte aligned */
+    const int32_t *nodeid, *cellfid;
+    const double *nf, *vertex;
+    int32_t nb_segs, nodeid_width, cellfid_width, quirk;
+} mfv_srnh_step;
+
+/* nsteps (even) steps of ghost values, gradients (order 2), convective flux, source, update_SW and
+ * time_step_SW: step s takes dts[s] (dts[0] is given) and leaves dts[s + 1]; the result is in cell.
+ * The bits of the entry points in that order. */
+int mfv_srnh_run(const mfv_mesh *m, const mfv_srnh_step *p, int order, double grav, double cfl, double *dts,
+                 int nsteps, void *stream);
+
 /* Fused MUSCL/Rusanov step: residuals + update_SW + the next step's time_step_SW.
  * state_in/state_out: [3][C] (h, hu, hv); grad from mfv_sw_gradients(state_in); dt ring as
  * for mfv_advection_step. */

@@ -183,6 +183,14 @@ class MfvSwBatch(ctypes.Structure):
                 ('inst_ncells', P), ('rings', P)]
 
 
+class MfvSrnhStep(ctypes.Structure):
+    """Mirror of ``struct mfv_srnh_step`` (include/mfv.h)."""
+    _fields_ = [('cell', P * 5), ('cell2', P * 5), ('ghost', P * 5), ('segs', P)] + \
+        [(k, P) for k in ('h_x', 'h_y', 'h_z', 'h_psi', 'hc_x', 'hc_y', 'hc_z', 'hc_psi', 'dissip_hc', 'corio_hu',
+                          'corio_hv', 'flux', 'nodeid', 'cellfid', 'nf', 'vertex')] + \
+        [(k, ctypes.c_int32) for k in ('nb_segs', 'nodeid_width', 'cellfid_width', 'quirk')]
+
+
 # per-instance solver states and scalar slots (MFV_KS_* in include/mfv.h)
 KS_IDLE, KS_START, KS_INNER, KS_CORRECT, KS_DONE, KS_FAILED, KS_CHECK, KS_ADVANCE = 0, 1, 2, 3, 4, 5, 6, 7
 KS_SIGMA, KS_TAU, KS_TOL_OUT, KS_TOL_IN, KS_MAXIT_IN, KS_MAXIT_OUT = 0, 1, 2, 3, 4, 5
@@ -230,6 +238,7 @@ _SIGNATURES = {
     'mfv_explicitscheme_convective_sw': [MESH_P] + [P] * 20 + [c_double, c_int, P],
     'mfv_term_source_srnh_sw': [MESH_P, P, P, P, P, P, P, P, P, P, P, c_int, P, c_int, P, P, c_double, c_int, P],
     'mfv_update_sw5': [MESH_P] + [P] * 18 + [c_double, c_double, c_double, P, P],
+    'mfv_srnh_run': [MESH_P, ctypes.POINTER(MfvSrnhStep), c_int, c_double, c_double, P, c_int, P],
     'mfv_sw_step_fused': [MESH_P, P, P, P, P, P, c_double, c_double, c_int, P, c_int, P],
     'mfv_dt_reset': [P, P],
     'mfv_term_friction_sw': [c_int, P, P, P, c_double, c_double, c_double, P],

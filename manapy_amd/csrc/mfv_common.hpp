@@ -178,12 +178,8 @@ __device__ __forceinline__ void ring_advance(const DtRing &r)
 // first wave of the grid then writes the slot and the ring's other entries. A wave reads n / 64
 // values a lane: against the 5 us of a launch of its own this pays up to kFoldMax partials.
 constexpr int kFoldMax = 1024;
-__device__ __forceinline__ double step_dt(const DtRing &r, const double *__restrict__ part, int n)
+__device__ __forceinline__ double fold_min(const double *__restrict__ part, int n)
 {
-    if (n == 0) {
-        ring_advance(r);
-        return r.cur[0];
-    }
     double m = 1e6;
     for (int j = threadIdx.x & 63; j < n; j += 256) {
         double v[4];
@@ -197,6 +193,15 @@ __device__ __forceinline__ double step_dt(const DtRing &r, const double *__restr
         const double o = __shfl_xor(m, off, 64);
         m = (o < m) ? o : m;
     }
+    return m;
+}
+__device__ __forceinline__ double step_dt(const DtRing &r, const double *__restrict__ part, int n)
+{
+    if (n == 0) {
+        ring_advance(r);
+        return r.cur[0];
+    }
+    const double m = fold_min(part, n);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         const_cast<double *>(r.cur)[0] = m;
         r.spare[0] = 1e6;
@@ -251,6 +256,28 @@ inline Mesh to_kernel(const mfv_mesh *m)
     k.lsq_ghosts = m->lsq_ghosts;
     k.lsq_nghosts = m->lsq_nghosts;
     return k;
+}
+
+// time_step_SW (shallowater/fvm_utils.py:16-42): per-cell candidate, faces in faceid order.
+__device__ __forceinline__ double sw_cell_dt(const Mesh &m, int i, double h, double hu, double hv, double cfl,
+                                             double grav, double Dxx, double Dyy)
+{
+    const double vol = m.cell_volume[i];
+    const double velson = sqrt(grav * h);
+    const int nf = m.cell_nfaces[i];
+    double lam = 0.;
+    for (int j = 0; j < nf; j++) {
+        int f = m.cell_faces[(size_t)j * m.C + i];
+        const double *n = m.face_normal + 3 * (size_t)f;
+        double mesu = m.face_mesure[f];
+        double u_n = fabs(hu / h * n[0] + hv / h * n[1]);
+        double lam_convect = u_n / mesu + velson;
+        lam += lam_convect * mesu;
+        double mes = sqrt(n[0] * n[0] + n[1] * n[1]);
+        double lam_diff = Dxx * (mes * mes) + Dyy * (mes * mes);
+        lam += lam_diff / vol;
+    }
+    return cfl * vol / lam;
 }
 
 int validate_mesh(const mfv_mesh *m, int need_lsq, int need_order_split, int need_order_sorted);

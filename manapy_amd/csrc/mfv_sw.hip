@@ -75,28 +75,6 @@ __device__ __forceinline__ void sw_face(double etaL, double huL, double hvL, dou
                       bR);
 }
 
-// time_step_SW (shallowater/fvm_utils.py:16-42): per-cell candidate, faces in faceid order.
-__device__ __forceinline__ double sw_cell_dt(const Mesh &m, int i, double h, double hu, double hv, double cfl,
-                                             double grav, double Dxx, double Dyy)
-{
-    const double vol = m.cell_volume[i];
-    const double velson = sqrt(grav * h);
-    const int nf = m.cell_nfaces[i];
-    double lam = 0.;
-    for (int j = 0; j < nf; j++) {
-        int f = m.cell_faces[(size_t)j * m.C + i];
-        const double *n = m.face_normal + 3 * (size_t)f;
-        double mesu = m.face_mesure[f];
-        double u_n = fabs(hu / h * n[0] + hv / h * n[1]);
-        double lam_convect = u_n / mesu + velson;
-        lam += lam_convect * mesu;
-        double mes = sqrt(n[0] * n[0] + n[1] * n[1]);
-        double lam_diff = Dxx * (mes * mes) + Dyy * (mes * mes);
-        lam += lam_diff / vol;
-    }
-    return cfl * vol / lam;
-}
-
 __global__ void __launch_bounds__(kBlock) k_sw_time_step(Mesh m, const double *__restrict__ h,
                                                           const double *__restrict__ hu,
                                                           const double *__restrict__ hv, double cfl, double grav,

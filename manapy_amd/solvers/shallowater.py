@@ -275,9 +275,37 @@ class ShallowWaterSolver(object):
             self.dt = float(self._clock.ring[(nsteps - 1) % 3])
         return self._clock.time
 
+    def _srnh_fused(self, dts, nsteps):
+        import torch
+        m = self._m
+        v = (self.h, self.hu, self.hv, self.hc, self.Z)
+        dev = dict(dtype=torch.float64, device=m.device)
+        other = torch.empty((5, int(m.C)), **dev)
+        flux = torch.empty((int(m.F), 4), **dev)
+        if self.order == 2:
+            m.ensure_lsq()
+        p = _lib.MfvSrnhStep()
+        for k, x in enumerate(v):
+            p.cell[k], p.cell2[k], p.ghost[k] = x.cell.data_ptr(), other[k].data_ptr(), x.ghost.data_ptr()
+        segs = [b.ghost_segment(x) for x in v for b in x.BCs.values() if len(b.BCfaces)]
+        segs = (_lib.MfvGhostSeg * len(segs))(*segs)
+        p.segs, p.nb_segs = ctypes.cast(segs, ctypes.c_void_p), len(segs)
+        for name, x in (('h', self.h), ('hc', self.hc)):
+            for part, a in (('x', x.gradcellx), ('y', x.gradcelly), ('z', x.gradcellz), ('psi', x.psi)):
+                setattr(p, name + '_' + part, a.data_ptr())
+        p.dissip_hc, p.corio_hu, p.corio_hv = (a.data_ptr() for a in (self.hc.dissipation, self.hu.coriolis,
+                                                                       self.hv.coriolis))
+        p.flux = flux.data_ptr()
+        p.nodeid, p.nodeid_width = self._nodeid.data_ptr(), int(self._nodeid.shape[1])
+        p.cellfid, p.cellfid_width = self._cellfid.data_ptr(), int(self._cellfid.shape[1])
+        p.nf, p.vertex, p.quirk = self._nf.data_ptr(), self._vertex.data_ptr(), self.quirk
+        _lib.call('mfv_srnh_run', m.ptr, ctypes.byref(p), self.order, self.grav, self.cfl, dts.data_ptr(), nsteps,
+                  stream_ptr())
+
     def _srnh_run(self, nsteps):
         """The reference sequence per step with every dt kept on the device (one slot per
-        step, read back once at the end)."""
+        step, read back once at the end). The last one or two steps run the sequence itself, which
+        leaves every array that it fills; the even number before them runs fused (mfv_srnh_run)."""
         import torch
         if nsteps <= 0:
             return 0.
@@ -290,9 +318,16 @@ class ShallowWaterSolver(object):
                 t += float(self.dt)
             return t
         dts = torch.zeros(nsteps, dtype=torch.float64, device=self._m.device)
-        for k in range(nsteps):
+        fused = (nsteps - 1) // 2 * 2
+        if len({x.cell.data_ptr() for x in self.varbs.values()}) < 5:  # a field in two roles is updated twice
+            fused = 0
+        if fused:
+            self._srnh_dt(dts[:1], False)
+            self._srnh_fused(dts, fused)
+        for k in range(fused, nsteps):
             dk = dts[k:k + 1]
-            self._srnh_dt(dk, False)
+            if k != fused or k == 0:  # the fused steps leave the dt of the step after them
+                self._srnh_dt(dk, False)
             self.update_ghost_values()
             self._srnh_convective()
             self.update_term_source()
