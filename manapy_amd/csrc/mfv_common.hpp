@@ -258,22 +258,57 @@ inline Mesh to_kernel(const mfv_mesh *m)
     return k;
 }
 
+// The faces of a cell by slot, all asked for at once; a slot past the cell's count repeats the first.
+// A loop over the count waits for every face's id, then its data, before the next one's id: three or
+// four trips to memory a face, where the loads of all faces together take that many for the cell.
+template <int MF>
+__device__ __forceinline__ void cell_face_ids(const Mesh &m, int i, int nf, int (&f)[MF])
+{
+#pragma unroll
+    for (int s = 0; s < MF; s++) f[s] = m.cell_faces[(size_t)min(s, m.MF - 1) * m.C + i];
+#pragma unroll
+    for (int s = 0; s < MF; s++) f[s] = (s < nf) ? f[s] : s > 0 ? f[0] : 0;
+}
+
+// The same in the order of a residual (order_split or order_sorted).
+template <int MF>
+__device__ __forceinline__ void ordered_face_ids(const Mesh &m, const uint8_t *__restrict__ order, int i, int nf,
+                                                 int (&f)[MF])
+{
+    int s[MF];
+#pragma unroll
+    for (int r = 0; r < MF; r++) s[r] = order[(size_t)min(r, m.MF - 1) * m.C + i];
+#pragma unroll
+    for (int r = 0; r < MF; r++) f[r] = m.cell_faces[(size_t)s[r] * m.C + i];
+#pragma unroll
+    for (int r = 0; r < MF; r++) f[r] = (r < nf) ? f[r] : r > 0 ? f[0] : 0;
+}
+
 // time_step_SW (shallowater/fvm_utils.py:16-42): per-cell candidate, faces in faceid order.
+template <int MF>
 __device__ __forceinline__ double sw_cell_dt(const Mesh &m, int i, double h, double hu, double hv, double cfl,
                                              double grav, double Dxx, double Dyy)
 {
     const double vol = m.cell_volume[i];
     const double velson = sqrt(grav * h);
     const int nf = m.cell_nfaces[i];
+    int f[MF];
+    double n[MF][2], mesu[MF];
+    cell_face_ids<MF>(m, i, nf, f);
+#pragma unroll
+    for (int j = 0; j < MF; j++) {
+        n[j][0] = m.face_normal[3 * (size_t)f[j]];
+        n[j][1] = m.face_normal[3 * (size_t)f[j] + 1];
+        mesu[j] = m.face_mesure[f[j]];
+    }
     double lam = 0.;
-    for (int j = 0; j < nf; j++) {
-        int f = m.cell_faces[(size_t)j * m.C + i];
-        const double *n = m.face_normal + 3 * (size_t)f;
-        double mesu = m.face_mesure[f];
-        double u_n = fabs(hu / h * n[0] + hv / h * n[1]);
-        double lam_convect = u_n / mesu + velson;
-        lam += lam_convect * mesu;
-        double mes = sqrt(n[0] * n[0] + n[1] * n[1]);
+#pragma unroll
+    for (int j = 0; j < MF; j++) {
+        if (j >= nf) continue;
+        double u_n = fabs(hu / h * n[j][0] + hv / h * n[j][1]);
+        double lam_convect = u_n / mesu[j] + velson;
+        lam += lam_convect * mesu[j];
+        double mes = sqrt(n[j][0] * n[j][0] + n[j][1] * n[j][1]);
         double lam_diff = Dxx * (mes * mes) + Dyy * (mes * mes);
         lam += lam_diff / vol;
     }

@@ -530,6 +530,7 @@ __global__ void __launch_bounds__(kBlock) k_face_gradient3(Diamond d, int kind, 
 // dissipative residual (explicitscheme_dissipative, solvers/diffusion/fvm_utils.py:5-26):
 // all faces in id order, +q to cellid[0], -q to cellid[1] on inner faces.
 
+template <int MF>
 __global__ void __launch_bounds__(kBlock) k_dissipative(Mesh m, const double *__restrict__ wx,
                                                          const double *__restrict__ wy,
                                                          const double *__restrict__ wz, double Dxx, double Dyy,
@@ -538,15 +539,23 @@ __global__ void __launch_bounds__(kBlock) k_dissipative(Mesh m, const double *__
     const int K = blockIdx.x * blockDim.x + threadIdx.x;
     if (K >= m.C) return;
     const int nf = m.cell_nfaces[K];
+    int f[MF];
+    double q[MF];
+    bool right[MF];
+    ordered_face_ids<MF>(m, m.order_sorted, K, nf, f);
+#pragma unroll
+    for (int j = 0; j < MF; j++) {
+        const double *n = m.face_normal + 3 * (size_t)f[j];
+        const double z = wz ? wz[f[j]] : 0.;
+        q[j] = Dxx * wx[f[j]] * n[0] + Dyy * wy[f[j]] * n[1] + Dzz * z * n[2];
+        right[j] = m.face_name[f[j]] == 0 && m.face_cells[2 * (size_t)f[j] + 1] == K;
+    }
     double s = 0.;
-    for (int jj = 0; jj < nf; jj++) {
-        const int slot = m.order_sorted[(size_t)jj * m.C + K];
-        const int f = m.cell_faces[(size_t)slot * m.C + K];
-        const double *n = m.face_normal + 3 * f;
-        const double z = wz ? wz[f] : 0.;
-        const double q = Dxx * wx[f] * n[0] + Dyy * wy[f] * n[1] + Dzz * z * n[2];
-        if (m.face_name[f] == 0 && m.face_cells[2 * f + 1] == K) s -= q;
-        else s += q;
+#pragma unroll
+    for (int j = 0; j < MF; j++) {
+        if (j >= nf) continue;
+        if (right[j]) s -= q[j];
+        else s += q[j];
     }
     dis[K] = s;
 }
@@ -555,6 +564,7 @@ __global__ void __launch_bounds__(kBlock) k_dissipative(Mesh m, const double *__
 // time steps with diffusion: solvers/diffusion/fvm_utils.py:30-49 (u == NULL) and
 // solvers/advecdiff/fvm_utils.py:317-340 (u, v, w cell velocities; cells with lam == 0 skipped)
 
+template <int MF>
 __global__ void __launch_bounds__(kBlock) k_time_step_diff(Mesh m, const double *__restrict__ u,
                                                             const double *__restrict__ v,
                                                             const double *__restrict__ w, double cfl,
@@ -566,10 +576,20 @@ __global__ void __launch_bounds__(kBlock) k_time_step_diff(Mesh m, const double 
     if (i < m.C) {
         const double vol = m.cell_volume[i];
         const int nf = m.cell_nfaces[i];
+        int f[MF];
+        double nrm[MF][3];
+        cell_face_ids<MF>(m, i, nf, f);
+#pragma unroll
+        for (int j = 0; j < MF; j++)
+#pragma unroll
+            for (int d = 0; d < 3; d++) nrm[j][d] = m.face_normal[3 * (size_t)f[j] + d];
+        const double ui = u ? u[i] : 0., vi = u ? v[i] : 0., wi = u ? w[i] : 0.;
         double lam = 0.;
-        for (int j = 0; j < nf; j++) {
-            const double *n = m.face_normal + 3 * (size_t)m.cell_faces[(size_t)j * m.C + i];
-            if (u) lam += fabs(u[i] * n[0] + v[i] * n[1] + w[i] * n[2]);
+#pragma unroll
+        for (int j = 0; j < MF; j++) {
+            if (j >= nf) continue;
+            const double *n = nrm[j];
+            if (u) lam += fabs(ui * n[0] + vi * n[1] + wi * n[2]);
             const double mes = sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
             const double lam_diff = Dxx * (mes * mes) + Dyy * (mes * mes) + Dzz * (mes * mes);
             lam += lam_diff / vol;
@@ -684,8 +704,9 @@ extern "C" int mfv_explicitscheme_dissipative(const mfv_mesh *m, const double *w
     if (int rc = validate_mesh(m, 0, 0, 1)) return rc;
     if (m->nb_cells == 0) return MFV_OK;
     MFV_REQUIRE(wx && wy && dissip, "NULL array");
-    hipLaunchKernelGGL(k_dissipative, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream),
-                       to_kernel(m), wx, wy, wz, Dxx, Dyy, Dzz, dissip);
+    auto k = m->max_cell_faces <= 3 ? k_dissipative<3> : m->max_cell_faces <= 4 ? k_dissipative<4> : k_dissipative<8>;
+    hipLaunchKernelGGL(k, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream), to_kernel(m), wx, wy, wz,
+                       Dxx, Dyy, Dzz, dissip);
     return check_launch("k_dissipative");
 }
 
@@ -701,8 +722,11 @@ extern "C" int mfv_time_step_diffusion(const mfv_mesh *m, const double *u, const
     if (nw) {
         part = dt_scratch(nw, as_stream(stream));
         if (!part) return MFV_ENOMEM;
-        hipLaunchKernelGGL(k_time_step_diff, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream),
-                           to_kernel(m), u, v, w, cfl, Dxx, Dyy, Dzz, part);
+        auto k = m->max_cell_faces <= 3   ? k_time_step_diff<3>
+                 : m->max_cell_faces <= 4 ? k_time_step_diff<4>
+                                          : k_time_step_diff<8>;
+        hipLaunchKernelGGL(k, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream), to_kernel(m), u, v, w,
+                           cfl, Dxx, Dyy, Dzz, part);
     }
     return dt_total(part, nw, dt_dev, dt_host, as_stream(stream));
 }

@@ -212,13 +212,60 @@ __device__ __forceinline__ void euler_cell_residual(const Mesh &m, int i, const 
     }
 }
 
-template <class A, class R>
+// The same with the loads of NB faces together (cells of at most four faces, ghosts from G): ids, then
+// geometry, then the other side's state, where the loop above waits for them face by face. All four at
+// once where the mesh leaves the chip idle anyway, two where registers cost waves.
+template <int NB, class A>
+__device__ __forceinline__ void euler_cell_residual4(const Mesh &m, int i, const A &U, const A &G, double gamma,
+                                                     int quirk, double (&rez)[5])
+{
+    const int nf = m.cell_nfaces[i];
+    int ids[4];
+    ordered_face_ids<4>(m, m.order_sorted, i, nf, ids);
+    const Prim6 own = load6(U, i);
+#pragma unroll
+    for (int v = 0; v < 5; v++) rez[v] = 0.;
+#pragma unroll
+    for (int k0 = 0; k0 < 4; k0 += NB) {
+        int2 ab[NB];
+        int nm[NB];
+        double ms[NB], nrm[NB][3];
+        Prim6 nb[NB];
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+            const size_t f = ids[k0 + k];
+            ab[k] = reinterpret_cast<const int2 *>(m.face_cells)[f];
+            nm[k] = m.face_name[f];
+            ms[k] = m.face_mesure[f];
+#pragma unroll
+            for (int d = 0; d < 3; d++) nrm[k][d] = m.face_normal[3 * f + d];
+        }
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+            if (nm[k] == 0) nb[k] = load6(U, ab[k].x == i ? ab[k].y : ab[k].x);
+            else nb[k] = load6(G, ids[k0 + k]);
+        }
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+            if (k0 + k >= nf) continue;
+            const bool left = ab[k].x == i;
+            const double n[3] = {nrm[k][0] / ms[k], nrm[k][1] / ms[k], nrm[k][2] / ms[k]};
+            double fl[5];
+            euler_flux(left ? own : nb[k], left ? nb[k] : own, n, ms[k], gamma, quirk, fl);
+#pragma unroll
+            for (int v = 0; v < 5; v++) rez[v] += left ? -fl[v] : fl[v];
+        }
+    }
+}
+
+template <int NB, class A, class R>
 __global__ void __launch_bounds__(kBlock) k_euler_rusanov(Mesh m, A U, A G, double gamma, int quirk, R rez)
 {
     int i = xcd_block() * blockDim.x + threadIdx.x;
     if (i >= m.C) return;
     double r[5];
-    euler_cell_residual<true>(m, i, U, G, gamma, quirk, r);
+    if (NB > 0) euler_cell_residual4<NB == 0 ? 1 : NB>(m, i, U, G, gamma, quirk, r);
+    else euler_cell_residual<true>(m, i, U, G, gamma, quirk, r);
     for (int v = 0; v < 5; v++) rez.f(v)[i] = r[v];
 }
 
@@ -1229,8 +1276,9 @@ extern "C" int mfv_explicitscheme_euler_3d_rusanov(const mfv_mesh *m, const mfv_
     MFV_REQUIRE(complete(cells) && complete(ghosts), "NULL Euler array");
     if (m->nb_cells == 0) return MFV_OK;
     const Arrays<5> r{{rez->rho, rez->rhou, rez->rhov, rez->rhow, rez->rhoE}};
-    hipLaunchKernelGGL((k_euler_rusanov<Arrays<6>, Arrays<5>>), dim3(grid_for(m->nb_cells)), dim3(kBlock), 0,
-                       as_stream(stream), to_kernel(m), arrays6(cells), arrays6(ghosts), gamma, quirk, r);
+    auto k = m->max_cell_faces <= 4 ? k_euler_rusanov<2, Arrays<6>, Arrays<5>> : k_euler_rusanov<0, Arrays<6>, Arrays<5>>;
+    hipLaunchKernelGGL(k, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream), to_kernel(m), arrays6(cells),
+                       arrays6(ghosts), gamma, quirk, r);
     return check_launch("k_euler_rusanov");
 }
 
@@ -1272,8 +1320,12 @@ extern "C" int mfv_euler3d_rusanov(const mfv_mesh *m, const double *U, const dou
     if (m->nb_cells == 0) return MFV_OK;
     MFV_REQUIRE(U && G && rez, "NULL array");
     const Rows u{const_cast<double *>(U), (size_t)m->nb_cells}, g{const_cast<double *>(G), (size_t)m->nb_faces};
-    hipLaunchKernelGGL((k_euler_rusanov<Rows, Rows>), dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream),
-                       to_kernel(m), u, g, gamma, quirk, Rows{rez, (size_t)m->nb_cells});
+    // 262k cells are four waves a SIMD: below, more registers a wave cost nothing
+    auto k = m->max_cell_faces > 4   ? k_euler_rusanov<0, Rows, Rows>
+             : m->nb_cells <= 131072 ? k_euler_rusanov<4, Rows, Rows>
+                                     : k_euler_rusanov<2, Rows, Rows>;
+    hipLaunchKernelGGL(k, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream), to_kernel(m), u, g, gamma,
+                       quirk, Rows{rez, (size_t)m->nb_cells});
     return check_launch("k_euler_rusanov");
 }
 

@@ -353,7 +353,7 @@ __global__ void __launch_bounds__(kBlock) k_srnh_cell(Mesh m, SrnhSource t, Fiel
         u[4] += dt * (acc[4] + 0.) / vol;
 #pragma unroll
         for (int k = 0; k < 5; k++) out.f[k][i] = u[k];
-        d = sw_cell_dt(m, i, u[0], u[1], u[2], cfl, grav, 0., 0.);
+        d = sw_cell_dt<3>(m, i, u[0], u[1], u[2], cfl, grav, 0., 0.);
     }
     wave_min_part(dtpart, (size_t)i, d);
 }

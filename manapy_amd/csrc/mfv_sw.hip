@@ -75,13 +75,14 @@ __device__ __forceinline__ void sw_face(double etaL, double huL, double hvL, dou
                       bR);
 }
 
+template <int MF>
 __global__ void __launch_bounds__(kBlock) k_sw_time_step(Mesh m, const double *__restrict__ h,
                                                           const double *__restrict__ hu,
                                                           const double *__restrict__ hv, double cfl, double grav,
                                                           double Dxx, double Dyy, double *__restrict__ dtpart)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    double d = (i < m.C) ? sw_cell_dt(m, i, h[i], hu[i], hv[i], cfl, grav, Dxx, Dyy) : 1e300;
+    double d = (i < m.C) ? sw_cell_dt<MF>(m, i, h[i], hu[i], hv[i], cfl, grav, Dxx, Dyy) : 1e300;
     wave_min_part(dtpart, (size_t)i, d);
 }
 
@@ -320,7 +321,7 @@ __global__ void __launch_bounds__(kBlock) k_sw_step(Mesh m, const double *__rest
         Sout[i] = hn;
         Sout[C + i] = un;
         Sout[2 * C + i] = vn;
-        dloc = sw_cell_dt(m, i, hn, un, vn, cfl, g, 0., 0.);
+        dloc = sw_cell_dt<8>(m, i, hn, un, vn, cfl, g, 0., 0.);
     }
     wave_min_part(dtpart, (size_t)i, dloc);
 }
@@ -338,8 +339,11 @@ extern "C" int mfv_time_step_sw(const mfv_mesh *m, const double *h, const double
     if (nw) {
         part = dt_scratch(nw, as_stream(stream));
         if (!part) return MFV_ENOMEM;
-        hipLaunchKernelGGL(k_sw_time_step, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream),
-                           to_kernel(m), h, hu, hv, cfl, grav, Dxx, Dyy, part);
+        auto k = m->max_cell_faces <= 3   ? k_sw_time_step<3>
+                 : m->max_cell_faces <= 4 ? k_sw_time_step<4>
+                                          : k_sw_time_step<8>;
+        hipLaunchKernelGGL(k, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream), to_kernel(m), h, hu, hv,
+                           cfl, grav, Dxx, Dyy, part);
     }
     return dt_total(part, nw, dt_dev, dt_host, as_stream(stream));
 }
