@@ -110,6 +110,30 @@ typedef struct mfv_gradient_fields {
 } mfv_gradient_fields;
 int mfv_cell_gradient_limited(const mfv_mesh *m, int nfields, const mfv_gradient_fields *f, void *stream);
 
+/* The least-squares stencils of a tetrahedral mesh on tiles of 256 cells along a curve: tile t holds
+ * the cells cell[256 t ..] (-1 past the end) and reads the cells ext_cells[ext_ptr[t] .. ext_ptr[t + 1]);
+ * word [j][thread] of pairs holds the positions of its stencil's entries 2j (low 16 bits) and 2j + 1
+ * in that list. LDS: 32 * max_ext bytes (max_ext <= 2048). */
+typedef struct mfv_stencil_tiles {
+    int32_t nb_tiles, tile_size, max_ext, nb_pairs;
+    const int32_t *cell;      /* [nb_tiles * tile_size] */
+    const int32_t *ext_ptr;   /* [nb_tiles + 1] */
+    const int32_t *ext_cells;
+    const uint32_t *pairs;    /* [nb_pairs = (lsq_width + 1) / 2][nb_tiles * tile_size] */
+} mfv_stencil_tiles;
+typedef struct mfv_stencil_tiles_host {
+    int32_t nb_tiles, tile_size, max_ext, nb_pairs, ext_len, pad_;
+    int32_t *cell, *ext_ptr, *ext_cells;
+    uint32_t *pairs;
+} mfv_stencil_tiles_host;
+/* Built on the host from lsq_cells [K][C], lsq_ncells [C] and the cell order perm [C] (new -> old). */
+int mfv_stencil_tiles_build(int C, int K, const int32_t *lsq_cells, const int32_t *lsq_ncells,
+                            const int64_t *perm, int T, mfv_stencil_tiles_host *out);
+void mfv_stencil_tiles_host_free(mfv_stencil_tiles_host *t);
+/* mfv_cell_gradient_limited of one field on stencil tiles; same bits. */
+int mfv_cell_gradient_tiled(const mfv_mesh *m, const mfv_stencil_tiles *t, const mfv_gradient_fields *f,
+                            void *stream);
+
 /* ---------------- advection (solvers/advec) --------------------------------------- */
 
 /* time_step (solvers/advec/fvm_utils.py:293-309): dt = min_K cfl |K| / sum_f |u_K.n_f|.
@@ -148,11 +172,11 @@ int mfv_advection_step(const mfv_mesh *m, const double *w_in, double *w_out, con
 /* nsteps of mfv_advection_step with the velocity and dt of the ring's current slot kept: the face
  * velocities and the upwind cells are laid out once in workspace (mfv_advection_run_size doubles).
  * Alternates between w_a (the start) and w_b; the result is in w_a for even nsteps, else in w_b.
- * The ring is left as by those steps. Same bits. */
+ * The ring is left as by those steps. tiles: the mesh's stencil tiles or NULL. Same bits. */
 int mfv_advection_run_size(const mfv_mesh *m, int order, size_t *doubles);
 int mfv_advection_run(const mfv_mesh *m, double *w_a, double *w_b, const double *u_face,
                       const double *v_face, const double *w_face, int order, double *dt_ring,
-                      int nsteps, double *workspace, void *stream);
+                      int nsteps, double *workspace, const mfv_stencil_tiles *tiles, void *stream);
 
 /* ---------------- shallow water (solvers/shallowater) ----------------------------- */
 

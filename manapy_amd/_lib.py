@@ -65,6 +65,18 @@ class MfvFaceTilesHost(ctypes.Structure):
                           'face_r', 'lface')]
 
 
+class MfvStencilTiles(ctypes.Structure):
+    """Mirror of ``struct mfv_stencil_tiles`` (include/mfv.h)."""
+    _fields_ = [(k, ctypes.c_int32) for k in ('nb_tiles', 'tile_size', 'max_ext', 'nb_pairs')] + \
+        [(k, P) for k in ('cell', 'ext_ptr', 'ext_cells', 'pairs')]
+
+
+class MfvStencilTilesHost(ctypes.Structure):
+    """Mirror of ``struct mfv_stencil_tiles_host`` (include/mfv.h)."""
+    _fields_ = [(k, ctypes.c_int32) for k in ('nb_tiles', 'tile_size', 'max_ext', 'nb_pairs', 'ext_len', 'pad_')] + \
+        [(k, P) for k in ('cell', 'ext_ptr', 'ext_cells', 'pairs')]
+
+
 class MfvEulerTet(ctypes.Structure):
     """Mirror of ``struct mfv_euler_tet`` (include/mfv.h)."""
     _fields_ = [('nb_cells', ctypes.c_int32), ('nb_faces', ctypes.c_int32)] + \
@@ -223,13 +235,16 @@ _SIGNATURES = {
     'mfv_cell_gradient': [MESH_P, P, P, P, P, P, P],
     'mfv_barthlimiter': [MESH_P, P, P, P, P, P, P, P],
     'mfv_cell_gradient_limited': [MESH_P, c_int, ctypes.POINTER(MfvGradientFields), P],
+    'mfv_cell_gradient_tiled': [MESH_P, ctypes.POINTER(MfvStencilTiles), ctypes.POINTER(MfvGradientFields), P],
+    'mfv_stencil_tiles_build': [c_int, c_int, P, P, P, c_int, ctypes.POINTER(MfvStencilTilesHost)],
+    'mfv_stencil_tiles_host_free': [ctypes.POINTER(MfvStencilTilesHost)],
     'mfv_time_step': [MESH_P, P, P, P, c_double, P, DP, P],
     'mfv_explicitscheme_convective': [MESH_P, P, P, P, P, P, P, P, P, P, P, c_int, P],
     'mfv_update_new_value': [MESH_P, P, P, P, P, c_double, P, P],
     'mfv_dt_ring_init': [P, P, P],
     'mfv_advection_step': [MESH_P, P, P, P, P, P, P, P, P, c_double, c_int, P, c_int, P, P],
     'mfv_advection_run_size': [MESH_P, c_int, ctypes.POINTER(ctypes.c_size_t)],
-    'mfv_advection_run': [MESH_P, P, P, P, P, P, c_int, P, c_int, P, P],
+    'mfv_advection_run': [MESH_P, P, P, P, P, P, c_int, P, c_int, P, ctypes.POINTER(MfvStencilTiles), P],
     'mfv_time_step_sw': [MESH_P, P, P, P, c_double, c_double, c_double, c_double, P, DP, P],
     'mfv_sw_gradients': [MESH_P, P, P, P, P, P, P],
     'mfv_sw_residuals': [MESH_P, P, P, P, P, P, P, c_double, c_int, P, P, P],
@@ -326,7 +341,7 @@ _SIGNATURES = {
     'mfv_ell_narrow_columns': [ELL_P, c_int, c_int, P, P, P],
 }
 _RESTYPE = {'mfv_version': c_char_p, 'mfv_last_error': c_char_p, 'mfv_sw_tiles_host_free': None,
-            'mfv_face_tiles_host_free': None, 'mfv_euler_tet_host_free': None, 'mfv_domain_topology_free': None,
+            'mfv_face_tiles_host_free': None, 'mfv_stencil_tiles_host_free': None, 'mfv_euler_tet_host_free': None, 'mfv_domain_topology_free': None,
             'mfv_domain_geometry_2d_free': None, 'mfv_domain_geometry_3d_free': None}
 
 _lib = None

@@ -370,3 +370,80 @@ extern "C" int mfv_face_tiles_build(int C, int MF, const int32_t *cell_faces, co
     }
     return MFV_OK;
 }
+
+// ---------------------------------------------------------------------------------------------
+// Stencil tiles (mfv_stencil_tiles): per tile of T cells along perm, the cells that the tile's
+// least-squares stencils read (ascending) and each stencil as positions in that list.
+
+extern "C" void mfv_stencil_tiles_host_free(mfv_stencil_tiles_host *t)
+{
+    if (!t) return;
+    free(t->cell);
+    free(t->ext_ptr);
+    free(t->ext_cells);
+    free(t->pairs);
+    memset(t, 0, sizeof(*t));
+}
+
+extern "C" int mfv_stencil_tiles_build(int C, int K, const int32_t *lsq_cells, const int32_t *lsq_ncells,
+                                       const int64_t *perm, int T, mfv_stencil_tiles_host *out)
+{
+    MFV_REQUIRE(out, "out is NULL");
+    memset(out, 0, sizeof(*out));
+    MFV_REQUIRE(C > 0 && K > 0 && T > 0, "bad sizes C=%d K=%d T=%d", C, K, T);
+    MFV_REQUIRE(lsq_cells && lsq_ncells && perm, "NULL array");
+    const int nt = (C + T - 1) / T, K2 = (K + 1) / 2;
+    const size_t n = (size_t)nt * T;
+    std::vector<int32_t> cell(n, -1), eptr(nt + 1, 0), ext, te, mark(C, -1), pos(C, 0);
+    std::vector<uint32_t> pairs((size_t)K2 * n, 0);
+    int max_ext = 0;
+    for (int t = 0; t < nt; t++) {
+        te.clear();
+        const int n0 = t * T, nc = std::min(T, C - n0);
+        auto add = [&](int c) {
+            if (mark[c] != t) {
+                mark[c] = t;
+                te.push_back(c);
+            }
+        };
+        for (int l = 0; l < nc; l++) {
+            const int64_t c = perm[n0 + l];
+            MFV_REQUIRE(c >= 0 && c < C, "perm[%d] out of range", n0 + l);
+            MFV_REQUIRE(lsq_ncells[c] >= 0 && lsq_ncells[c] <= K, "cell %d: %d neighbours of %d", (int)c,
+                        lsq_ncells[c], K);
+            cell[(size_t)n0 + l] = (int32_t)c;
+            for (int k = 0; k < lsq_ncells[c]; k++) {
+                const int q = lsq_cells[(size_t)k * C + c];
+                MFV_REQUIRE(q >= 0 && q < C, "cell %d: neighbour %d out of range", (int)c, q);
+                add(q);
+            }
+        }
+        if (te.empty()) te.push_back(cell[n0]);
+        std::sort(te.begin(), te.end());
+        MFV_REQUIRE(te.size() <= 65535, "tile %d reads more than 65535 cells", t);
+        for (size_t e = 0; e < te.size(); e++) pos[te[e]] = (int32_t)e;
+        for (int l = 0; l < nc; l++) {
+            const int c = cell[(size_t)n0 + l];
+            for (int k = 0; k < lsq_ncells[c]; k++)
+                pairs[(size_t)(k / 2) * n + n0 + l] |= (uint32_t)pos[lsq_cells[(size_t)k * C + c]] << (16 * (k & 1));
+        }
+        ext.insert(ext.end(), te.begin(), te.end());
+        eptr[t + 1] = (int32_t)ext.size();
+        max_ext = std::max(max_ext, (int)te.size());
+    }
+    out->nb_tiles = nt;
+    out->tile_size = T;
+    out->max_ext = max_ext;
+    out->nb_pairs = K2;
+    out->ext_len = (int32_t)ext.size();
+    out->cell = copy_out(cell);
+    out->ext_ptr = copy_out(eptr);
+    out->ext_cells = copy_out(ext);
+    out->pairs = copy_out(pairs);
+    if (!out->cell || !out->ext_ptr || !out->ext_cells || !out->pairs) {
+        mfv_stencil_tiles_host_free(out);
+        mfv::set_error("stencil tiles: host allocation failed");
+        return MFV_ENOMEM;
+    }
+    return MFV_OK;
+}

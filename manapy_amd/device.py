@@ -138,6 +138,7 @@ class DeviceMesh(object):
         d.nb_bnd = len(host['bnd_faces'])
         self.desc = d
         self.lsq = lsq
+        self._lsq_host = self._stencil_tiles = None
 
     @property
     def ptr(self):
@@ -155,6 +156,22 @@ class DeviceMesh(object):
         self.desc.lsq_width = host['K']
         self.desc.ghost_width = host['G']
         self.lsq = True
+        self._lsq_host = host
+
+    def stencil_tiles(self):
+        """The mesh's StencilTiles, or None where the gradients gather from memory: 2D meshes (a
+        dozen neighbours), cells of more than four faces, tiles that do not fit the LDS."""
+        self.ensure_lsq()
+        if self._stencil_tiles is None:
+            t = None
+            host = self._lsq_host if self._lsq_host is not None else self.host
+            if self.dim == 3 and self.MF <= 4 and self.C and host['K']:
+                from .renumber import morton_order_3d
+                t = StencilTiles(host, morton_order_3d(*host['cell_center'].T), self.device)
+                if t.desc.max_ext > 2048:
+                    t = None
+            self._stencil_tiles, self._lsq_host = t or False, None
+        return self._stencil_tiles or None
 
     @property
     def dist_ortho(self):
@@ -626,6 +643,38 @@ def euler_tet_native(cell_faces, face_cells, face_name, face_normal, face_mesure
     finally:
         _lib.call('mfv_euler_tet_host_free', ctypes.byref(h))
     return out
+
+
+class StencilTiles(object):
+    """Device copy of a tetrahedral mesh's stencil tiles (mfv_stencil_tiles) from its gpu_layout."""
+
+    T = 256
+
+    def __init__(self, H, perm, device):
+        import torch
+        i32 = lambda a: np.ascontiguousarray(a, dtype=np.int32)
+        C, K = int(H['C']), int(H['K'])
+        arrs = i32(H['lsq_cells']), i32(H['lsq_ncells']), np.ascontiguousarray(perm, dtype=np.int64)
+        h = _lib.MfvStencilTilesHost()
+        _lib.call('mfv_stencil_tiles_build', C, K, *[a.ctypes.data_as(ctypes.c_void_p) for a in arrs], self.T,
+                  ctypes.byref(h))
+        try:
+            n = h.nb_tiles * h.tile_size
+            self.t = {}
+            for k, m in (('cell', n), ('ext_ptr', h.nb_tiles + 1), ('ext_cells', h.ext_len), ('pairs', h.nb_pairs * n)):
+                a = np.ctypeslib.as_array(ctypes.cast(getattr(h, k), ctypes.POINTER(ctypes.c_int32)), (m,))
+                self.t[k] = torch.from_numpy(a.copy()).to(device)
+            d = _lib.MfvStencilTiles()
+            d.nb_tiles, d.tile_size, d.max_ext, d.nb_pairs = h.nb_tiles, h.tile_size, h.max_ext, h.nb_pairs
+        finally:
+            _lib.call('mfv_stencil_tiles_host_free', ctypes.byref(h))
+        for k, a in self.t.items():
+            setattr(d, k, a.data_ptr())
+        self.desc = d
+
+    @property
+    def ptr(self):
+        return ctypes.byref(self.desc)
 
 
 class EulerTet(object):

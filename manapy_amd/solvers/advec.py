@@ -111,10 +111,11 @@ class AdvectionSolver(object):
         b = torch.empty_like(a)
         n = ctypes.c_size_t(0)
         _lib.call('mfv_advection_run_size', m.ptr, int(self.order), ctypes.byref(n))
+        tiles = m.stencil_tiles() if self.order == 2 else None
         ws = torch.empty(n.value, dtype=torch.float64, device=a.device)
         _lib.call('mfv_advection_run', m.ptr, a.data_ptr(), b.data_ptr(), self.u.face.data_ptr(),
                   self.v.face.data_ptr(), self.w.face.data_ptr(), int(self.order), self._clock.ring.data_ptr(),
-                  nsteps, ws.data_ptr(), s)
+                  nsteps, ws.data_ptr(), tiles.ptr if tiles is not None else None, s)
         if nsteps % 2 == 1:
             a.copy_(b)
         self._clock.step = nsteps

@@ -44,7 +44,11 @@ def cell_gradients(domain, variables):
     f = (_lib.MfvGradientFields * len(variables))(*[
         (v.cell.data_ptr(), v.ghost.data_ptr(), v.gradcellx.data_ptr(), v.gradcelly.data_ptr(),
          v.gradcellz.data_ptr(), v.psi.data_ptr()) for v in variables])
-    _lib.call('mfv_cell_gradient_limited', dm.ptr, len(variables), f, stream_ptr())
+    tiles = dm.stencil_tiles() if len(variables) == 1 else None
+    if tiles is not None:
+        _lib.call('mfv_cell_gradient_tiled', dm.ptr, tiles.ptr, f, stream_ptr())
+    else:
+        _lib.call('mfv_cell_gradient_limited', dm.ptr, len(variables), f, stream_ptr())
 
 
 class Boundary(object):
