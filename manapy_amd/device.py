@@ -107,7 +107,8 @@ def stream_ptr(stream=None):
 class DeviceMesh(object):
     """Device copy of a Domain's hot-path arrays and its ``mfv_mesh`` descriptor."""
 
-    def __init__(self, domain, lsq=True, device=None, host=None):
+    def __init__(self, domain, lsq=True, device=None, host=None, without=()):
+        """``without``: tables that the caller's kernels do not read; they are allocated, not uploaded."""
         torch = require_gpu()
         self.domain = domain
         self.device = torch.device(device if device is not None else 'cuda')
@@ -120,7 +121,8 @@ class DeviceMesh(object):
         self.t = {}
         for k, v in host.items():
             if isinstance(v, np.ndarray):
-                self.t[k] = torch.from_numpy(np.ascontiguousarray(v)).to(self.device)
+                v = torch.from_numpy(np.ascontiguousarray(v))
+                self.t[k] = torch.empty_like(v, device=self.device) if k in without else v.to(self.device)
         d = _lib.MfvMesh()
         d.dim = self.dim
         d.nb_cells = self.C

@@ -132,14 +132,18 @@ class DeviceDiamond(object):
     """Device copy of the diamond geometry and its ``mfv_diamond`` descriptor; the
     arrays it shares with the DeviceMesh (cell faces, volumes, normals) are not copied."""
 
-    def __init__(self, dmesh, host=None):
+    def __init__(self, dmesh, host=None, without=()):
+        """``without``: tables that the caller's kernels do not read; they are allocated, not uploaded."""
         import torch
         host = host if host is not None else diamond_layout(dmesh.domain)
         self.dmesh = dmesh
         self.N = host['N']
         self.dim = host['dim']
-        self.t = {k: torch.from_numpy(np.ascontiguousarray(v)).to(dmesh.device)
-                  for k, v in host.items() if isinstance(v, np.ndarray)}
+        self.t = {}
+        for k, v in host.items():
+            if isinstance(v, np.ndarray):
+                v = torch.from_numpy(np.ascontiguousarray(v))
+                self.t[k] = torch.empty_like(v, device=dmesh.device) if k in without else v.to(dmesh.device)
         d = _lib.MfvDiamond()
         d.nb_cells = dmesh.C
         d.nb_faces = dmesh.F
