@@ -165,6 +165,9 @@ class DeviceMesh(object):
         dozen neighbours), cells of more than four faces, tiles that do not fit the LDS."""
         self.ensure_lsq()
         if self._stencil_tiles is None:
+            import torch
+            if torch.cuda.is_current_stream_capturing():  # no uploads in a caller's graph
+                return None
             t = None
             host = self._lsq_host if self._lsq_host is not None else self.host
             if self.dim == 3 and self.MF <= 4 and self.C and host['K']:
