@@ -1126,11 +1126,15 @@ extern "C" int mfv_advection_step(const mfv_mesh *m, const double *w_in, double 
 // is one number for all steps. A step is then one launch (two at order 2) that reads 12 (28, 36)
 // coalesced bytes a slot and gathers one value (record) a slot, where the general step gathers both
 // sides of each face, its normal and velocities, and forms and reduces the same dt again. 100 steps
-// at 80k triangles, order 1: 1022 -> 326 us, about what 100 launches in a row take. The sums are the general step's term for term: the
+// at 80k triangles, order 1: 1022 -> 341 us, about what 100 launches in a row take. The sums are the general step's term for term: the
 // outward velocity is the face's with its sign turned for the right-hand cell, which is exact.
 namespace {
 
 constexpr int kAdvNone = (int)0x80000000;  // no face in this position
+// Cells up to which two steps go into one launch (k_adv_run_pair), 100 steps single and in pairs:
+// triangles 1k 361 and 240 us, 20k 341 and 251, 80k 341 and 300, 131k 348 and 308, 200k 410 and 405,
+// 400k 513 and 581; tetrahedra 10k 325 and 289, 48k 335 and 300, 162k 416 and 492.
+constexpr int kAdvPairCells3 = 131072, kAdvPairCells4 = 65536;
 
 struct AdvTable {
     int32_t *__restrict__ up;   // [MF][C] upwind cell; ~cell: its value without reconstruction (a ghost's)
@@ -1234,6 +1238,71 @@ __global__ void __launch_bounds__(kBlock) k_adv_run(Mesh m, AdvTable t, const do
     w_out[i] = wi + dt * ((rez + 0.) / vol + 0.);
 }
 
+// Two first-order steps in one launch: a cell forms the first step's value of each cell that its second
+// step takes (its own for the faces it flows out of), which costs up to four times the loads and no
+// barrier, and is faster where a step is no more than its launch (100 steps at 80k triangles 341 -> 300
+// us, at 1k 361 -> 240). Same expressions, same bits. The ring: as by the first of the two steps, whose spare slot (which the
+// second would reset) is this launch's dt and is left to the single steps that end a run.
+template <int MF>
+__global__ void __launch_bounds__(kBlock) k_adv_run_pair(Mesh m, AdvTable t, const double *__restrict__ w_in,
+                                                         double *__restrict__ w_out, DtRing ring)
+{
+    const int i = xcd_block() * blockDim.x + threadIdx.x;
+    const double dt = ring.cur[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        ring.next[0] = dt;
+        ring.spare[0] = dt;  // the slot of the step after these two
+        ring.time[0] += dt;
+        ring.time[0] += dt;
+    }
+    if (i >= m.C) return;
+    int up[MF];
+    double c[MF];
+    auto slots = [&](int q, int (&u)[MF], double (&k)[MF]) {
+#pragma unroll
+        for (int s = 0; s < MF; s++) {
+            const size_t row = min(s, m.MF - 1);
+            u[s] = (s < m.MF) ? t.up[row * m.C + q] : kAdvNone;
+            k[s] = t.coef[row * m.C + q];
+        }
+    };
+    auto cell = [&](int u, int own) { return u == kAdvNone ? own : u < 0 ? ~u : u; };
+    slots(i, up, c);
+    int u1[MF + 1][MF], at[MF + 1];
+    double c1[MF + 1][MF], w1[MF + 1], v1[MF + 1], g1[MF + 1][MF];
+    at[MF] = i;
+#pragma unroll
+    for (int s = 0; s < MF; s++) at[s] = cell(up[s], i);
+#pragma unroll
+    for (int q = 0; q <= MF; q++) {
+        if (q < MF) slots(at[q], u1[q], c1[q]);
+        w1[q] = w_in[at[q]];
+        v1[q] = m.cell_volume[at[q]];
+    }
+#pragma unroll
+    for (int s = 0; s < MF; s++) {
+        u1[MF][s] = up[s];
+        c1[MF][s] = c[s];
+    }
+#pragma unroll
+    for (int q = 0; q <= MF; q++)
+#pragma unroll
+        for (int s = 0; s < MF; s++) g1[q][s] = w_in[cell(u1[q][s], at[q])] + 0.;
+    auto stepped = [&](double w, double vol, const int (&u)[MF], const double (&k)[MF], const double (&g)[MF]) {
+        double rez = 0.;
+#pragma unroll
+        for (int s = 0; s < MF; s++)
+            if (u[s] != kAdvNone) rez -= k[s] * g[s];
+        return w + dt * ((rez + 0.) / vol + 0.);
+    };
+#pragma unroll
+    for (int q = 0; q <= MF; q++) w1[q] = stepped(w1[q], v1[q], u1[q], c1[q], g1[q]);
+    double g[MF];
+#pragma unroll
+    for (int s = 0; s < MF; s++) g[s] = w1[s] + 0.;
+    w_out[i] = stepped(w1[MF], v1[MF], up, c, g);
+}
+
 }  // namespace
 
 static int check_advection_run(const mfv_mesh *m, int order)
@@ -1280,7 +1349,19 @@ extern "C" int mfv_advection_run(const mfv_mesh *m, double *w_a, double *w_b, co
                           : (MF <= 4 ? (order == 2 ? k_adv_run<3, 2, 4> : k_adv_run<3, 1, 4>)
                                      : (order == 2 ? k_adv_run<3, 2, 8> : k_adv_run<3, 1, 8>));
     double *in = w_a, *out = w_b;
-    for (int s = 0; s < nsteps; s++) {
+    // an even number of pairs, so that the buffers end as after nsteps single ones, and a single last
+    const int pairs = (order == 1 && MF <= 4 && m->nb_cells <= (MF <= 3 ? kAdvPairCells3 : kAdvPairCells4))
+                          ? (nsteps - 1) / 2 / 2 * 2
+                          : 0;
+    auto kp = MF <= 3 ? k_adv_run_pair<3> : k_adv_run_pair<4>;
+    for (int p = 0; p < pairs; p++) {
+        hipLaunchKernelGGL(kp, g, b, 0, st, k, t, in, out, dt_ring(dt_ring_p, 2 * p));
+        if (int rc = check_launch("k_adv_run_pair")) return rc;
+        double *x = in;
+        in = out;
+        out = x;
+    }
+    for (int s = 2 * pairs; s < nsteps; s++) {
         if (order == 2) {
             const GradArgs<1> a{{in}, {nullptr}, {t.rec}, {nullptr}, {nullptr}, {nullptr}};
             const int rc = tiles ? gradient_tiled<true, true>(m, tiles, a, st) : gradient_limited<1, true, true>(m, a, st);

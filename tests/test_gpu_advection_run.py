@@ -21,6 +21,8 @@ def _bits(a, b):
 
 
 @pytest.mark.parametrize("kind,order,nsteps", [((3, 2), 1, 1), ((3, 2), 2, 2), ((17, 9), 1, 5), ((17, 9), 2, 4),
+                                               ((17, 9), 1, 6), ((41, 37), 1, 9), ((41, 37), 1, 12),
+                                               ("mixed", 1, 7), (3, 1, 8),
                                                ("mixed", 1, 3), ("mixed", 2, 3), (2, 1, 3), (2, 2, 2), (4, 2, 3)])
 def test_advection_run_equals_the_steps(kind, order, nsteps):
     import torch
