@@ -55,7 +55,8 @@ typedef struct mfv_mesh {
     const int32_t *cell_faces;   /* [MF][C]  cells.faceid (reference order), -1 padded */
     const int32_t *cell_nfaces;  /* [C]      cells.faceid[:, -1] */
     const uint8_t *order_split;  /* [MF][C]  residual order of inner-then-boundary face loops:
-                                             slot r -> column of cell_faces */
+                                             slot r -> column of cell_faces (rows past the
+                                             cell's count are not used) */
     const uint8_t *order_sorted; /* [MF][C]  residual order of all-faces-in-id-order loops */
     const int32_t *lsq_cells;    /* [K][C]   cells.cellnid */
     const int32_t *lsq_ncells;   /* [C]      cells.cellnid[:, -1] */

@@ -270,14 +270,18 @@ __device__ __forceinline__ void cell_face_ids(const Mesh &m, int i, int nf, int 
     for (int s = 0; s < MF; s++) f[s] = (s < nf) ? f[s] : s > 0 ? f[0] : 0;
 }
 
-// The same in the order of a residual (order_split or order_sorted).
+// The same in the order of a residual (order_split or order_sorted). What the order's rows past the
+// cell's count hold is the caller's affair: it takes part in no address.
 template <int MF>
 __device__ __forceinline__ void ordered_face_ids(const Mesh &m, const uint8_t *__restrict__ order, int i, int nf,
                                                  int (&f)[MF])
 {
     int s[MF];
 #pragma unroll
-    for (int r = 0; r < MF; r++) s[r] = order[(size_t)min(r, m.MF - 1) * m.C + i];
+    for (int r = 0; r < MF; r++) {
+        const int o = order[(size_t)min(r, m.MF - 1) * m.C + i];
+        s[r] = (r < nf) ? o : 0;
+    }
 #pragma unroll
     for (int r = 0; r < MF; r++) f[r] = m.cell_faces[(size_t)s[r] * m.C + i];
 #pragma unroll
