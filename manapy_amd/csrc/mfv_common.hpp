@@ -258,6 +258,15 @@ inline Mesh to_kernel(const mfv_mesh *m)
     return k;
 }
 
+// The cells of a face in one load, wherever a caller's int32 table begins: the hardware asks for no more
+// than 4 bytes of alignment, and a pointer to int2 would claim 8.
+typedef int IntPair __attribute__((ext_vector_type(2), aligned(4)));
+__device__ __forceinline__ int2 face_pair(const Mesh &m, size_t f)
+{
+    const IntPair p = *reinterpret_cast<const IntPair *>(m.face_cells + 2 * f);
+    return make_int2(p.x, p.y);
+}
+
 // The faces of a cell by slot, all asked for at once; a slot past the cell's count repeats the first.
 // A loop over the count waits for every face's id, then its data, before the next one's id: three or
 // four trips to memory a face, where the loads of all faces together take that many for the cell.

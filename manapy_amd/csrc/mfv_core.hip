@@ -423,7 +423,7 @@ __device__ __forceinline__ void gradient_cell(const Mesh &m, const GradArgs<NF> 
 #pragma unroll
     for (int s = 0; s < MF; s++) {
         const size_t f = fid[s] >= 0 ? fid[s] : 0;
-        ab[s] = reinterpret_cast<const int2 *>(m.face_cells)[f];
+        ab[s] = face_pair(m, f);
         nm[s] = m.face_name[f];
         r[s][0] = m.face_center[3 * f] - cx;
         r[s][1] = m.face_center[3 * f + 1] - cy;
@@ -951,7 +951,7 @@ __device__ __forceinline__ double adv_residual(const Mesh &m, int i, const doubl
     ordered_face_ids<MF>(m, m.order_split, i, nf, f);
 #pragma unroll
     for (int k = 0; k < MF; k++) {
-        const int2 ab = reinterpret_cast<const int2 *>(m.face_cells)[f[k]];
+        const int2 ab = face_pair(m, f[k]);
         const double *n = m.face_normal + 3 * (size_t)f[k];
         sign[k] = uf[f[k]] * n[0] + vf[f[k]] * n[1] + wf[f[k]] * n[2];
         if (ORDER == 2) {

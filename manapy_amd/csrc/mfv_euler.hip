@@ -234,7 +234,7 @@ __device__ __forceinline__ void euler_cell_residual4(const Mesh &m, int i, const
 #pragma unroll
         for (int k = 0; k < NB; k++) {
             const size_t f = ids[k0 + k];
-            ab[k] = reinterpret_cast<const int2 *>(m.face_cells)[f];
+            ab[k] = face_pair(m, f);
             nm[k] = m.face_name[f];
             ms[k] = m.face_mesure[f];
 #pragma unroll

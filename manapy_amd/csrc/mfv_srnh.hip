@@ -276,7 +276,7 @@ __global__ void __launch_bounds__(kBlock) k_srnh_face(Mesh m, Fields5 cell, Fiel
     const int f = xcd_block() * blockDim.x + threadIdx.x;
     if (f >= m.F) return;
     const double *h = cell.f[0], *hu = cell.f[1], *hv = cell.f[2], *hc = cell.f[3], *Z = cell.f[4];
-    const int2 lr = reinterpret_cast<const int2 *>(m.face_cells)[f];
+    const int2 lr = face_pair(m, f);
     const int L = lr.x, R = lr.y, r = R >= 0 ? R : L;
     const double *cf = m.face_center + 3 * (size_t)f, *cl = m.cell_center + 3 * (size_t)L,
                  *cr = m.cell_center + 3 * (size_t)r, *nrm = m.face_normal + 3 * (size_t)f;

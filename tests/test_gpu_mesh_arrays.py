@@ -68,3 +68,18 @@ def test_order_rows_past_the_face_count(size, order):
         t[past] = 255
         filled[k] = t
     _equal(_results(m, _descriptor(m, **filled), order), want)
+
+
+@pytest.mark.parametrize("order", [1, 2])
+def test_face_cells_aligned_to_four_bytes(order):
+    """face_cells is an int32 table: its first entry may lie at any multiple of 4."""
+    import torch
+    d = tri_quad_domain(31, 23, 100., 70.)
+    m = d.device_mesh
+    m.ensure_lsq()
+    want = _results(m, m.desc, order)
+    n = 2 * int(m.F)
+    odd = torch.empty(n + 1, dtype=torch.int32, device="cuda")[1:]
+    odd.copy_(m.t["face_cells"].reshape(-1))
+    assert odd.data_ptr() % 8 == 4
+    _equal(_results(m, _descriptor(m, face_cells=odd), order), want)
