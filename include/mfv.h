@@ -10,7 +10,12 @@
  *     message of the last failure on the calling thread is mfv_last_error().
  *   - `stream` is a hipStream_t passed as void* (NULL = the null stream). All
  *     calls are asynchronous on that stream except those with a *_host output,
- *     which synchronise it.
+ *     which synchronise it. Of the time steps with a dt_host there is a second form,
+ *     *_polled, which returns when the dt is there: all work before it on the stream
+ *     and dt_dev[0] are then complete and seen by whatever the caller starts next, on
+ *     any stream, but the stream need not be idle yet (it is not synchronised). With
+ *     dt_host NULL the two forms are the same. Both are refused while the stream is
+ *     being captured and dt_host is given.
  *   - A mesh descriptor (mfv_mesh) holds device pointers owned by the caller; the
  *     library never frees them.
  *
@@ -141,6 +146,8 @@ int mfv_cell_gradient_tiled(const mfv_mesh *m, const mfv_stencil_tiles *t, const
  * Writes the minimum to dt_dev[0] (device) and, if dt_host != NULL, to *dt_host (sync). */
 int mfv_time_step(const mfv_mesh *m, const double *u, const double *v, const double *w, double cfl,
                   double *dt_dev, double *dt_host, void *stream);
+int mfv_time_step_polled(const mfv_mesh *m, const double *u, const double *v, const double *w, double cfl,
+                         double *dt_dev, double *dt_host, void *stream);
 
 /* explicitscheme_convective_2d / _3d (solvers/advec/fvm_utils.py:19-152, :156-290) with the
  * residual formed by a deterministic cell-centric gather in the reference's face order. */
@@ -185,6 +192,9 @@ int mfv_advection_run(const mfv_mesh *m, double *w_a, double *w_b, const double 
 int mfv_time_step_sw(const mfv_mesh *m, const double *h, const double *hu, const double *hv,
                      double cfl, double grav, double Dxx, double Dyy, double *dt_dev,
                      double *dt_host, void *stream);
+int mfv_time_step_sw_polled(const mfv_mesh *m, const double *h, const double *hu, const double *hv,
+                            double cfl, double grav, double Dxx, double Dyy, double *dt_dev,
+                            double *dt_host, void *stream);
 
 /* Limited least-squares gradients of eta = h + Z, hu, hv for the MUSCL shallow-water step:
  * cell_gradient_2d + barthlimiter_2d applied to the three fields with wall ghosts
@@ -503,6 +513,8 @@ int mfv_euler3d_ghost(const mfv_mesh *m, const double *U, double *G, int quirk, 
 /* time_step_euler_3d (fvm_utils3d.py:809-825) min-reduced: dt_dev[0] = min_K dt_c[K]. */
 int mfv_euler3d_time_step(const mfv_mesh *m, const double *U, double cfl, double gamma,
                           double *dt_dev, double *dt_host, void *stream);
+int mfv_euler3d_time_step_polled(const mfv_mesh *m, const double *U, double cfl, double gamma,
+                                 double *dt_dev, double *dt_host, void *stream);
 
 /* explicitscheme_euler_3d_rusanov (fvm_utils3d.py:1083-1170) + compute_flux_euler_3d_rusanov
  * (:838-886), cell-centric gather in face-id order. rez: [5][C]. */
@@ -780,6 +792,9 @@ int mfv_explicitscheme_dissipative(const mfv_mesh *m, const double *wx, const do
 int mfv_time_step_diffusion(const mfv_mesh *m, const double *u, const double *v, const double *w,
                             double cfl, double Dxx, double Dyy, double Dzz, double *dt_dev,
                             double *dt_host, void *stream);
+int mfv_time_step_diffusion_polled(const mfv_mesh *m, const double *u, const double *v,
+                                   const double *w, double cfl, double Dxx, double Dyy, double Dzz,
+                                   double *dt_dev, double *dt_host, void *stream);
 
 /* ---------------- batched sparse solves (replaces solvers/ls/system.py:624-744) ------- */
 

@@ -239,6 +239,7 @@ _SIGNATURES = {
     'mfv_stencil_tiles_build': [c_int, c_int, P, P, P, c_int, ctypes.POINTER(MfvStencilTilesHost)],
     'mfv_stencil_tiles_host_free': [ctypes.POINTER(MfvStencilTilesHost)],
     'mfv_time_step': [MESH_P, P, P, P, c_double, P, DP, P],
+    'mfv_time_step_polled': [MESH_P, P, P, P, c_double, P, DP, P],
     'mfv_explicitscheme_convective': [MESH_P, P, P, P, P, P, P, P, P, P, P, c_int, P],
     'mfv_update_new_value': [MESH_P, P, P, P, P, c_double, P, P],
     'mfv_dt_ring_init': [P, P, P],
@@ -246,6 +247,7 @@ _SIGNATURES = {
     'mfv_advection_run_size': [MESH_P, c_int, ctypes.POINTER(ctypes.c_size_t)],
     'mfv_advection_run': [MESH_P, P, P, P, P, P, c_int, P, c_int, P, ctypes.POINTER(MfvStencilTiles), P],
     'mfv_time_step_sw': [MESH_P, P, P, P, c_double, c_double, c_double, c_double, P, DP, P],
+    'mfv_time_step_sw_polled': [MESH_P, P, P, P, c_double, c_double, c_double, c_double, P, DP, P],
     'mfv_sw_gradients': [MESH_P, P, P, P, P, P, P],
     'mfv_sw_residuals': [MESH_P, P, P, P, P, P, P, c_double, c_int, P, P, P],
     'mfv_update_sw': [MESH_P, P, P, P, P, P, P, P],
@@ -273,6 +275,7 @@ _SIGNATURES = {
     'mfv_sw_conservation': [MESH_P, SWM_P, P, c_int, P, P],
     'mfv_euler3d_ghost': [MESH_P, P, P, c_int, P],
     'mfv_euler3d_time_step': [MESH_P, P, c_double, c_double, P, DP, P],
+    'mfv_euler3d_time_step_polled': [MESH_P, P, c_double, c_double, P, DP, P],
     'mfv_euler3d_rusanov': [MESH_P, P, P, c_double, c_int, P, P],
     'mfv_euler3d_update': [MESH_P, P, P, c_double, P, P],
     'mfv_euler3d_update_by': [MESH_P, P, P, c_double, c_double, P],
@@ -309,6 +312,7 @@ _SIGNATURES = {
     'mfv_face_gradient_3d': [DIA_P, c_int, P, P, P, P, P, P, P, P, P, P, P],
     'mfv_explicitscheme_dissipative': [MESH_P, P, P, P, c_double, c_double, c_double, P, P],
     'mfv_time_step_diffusion': [MESH_P, P, P, P, c_double, c_double, c_double, c_double, P, DP, P],
+    'mfv_time_step_diffusion_polled': [MESH_P, P, P, P, c_double, c_double, c_double, c_double, P, DP, P],
     'mfv_sw_batch_dt_init': [MESH_P, SWM_P, SWB_P, c_double, c_double, P],
     'mfv_sw_batch_step': [MESH_P, SWM_P, SWB_P, c_double, c_double, c_int, c_int, c_int, P],
     'mfv_sw_step_mixed_tiled': [MESH_P, SWM_P, SWT_P, P, c_double, c_double, c_int, P, c_int, P],

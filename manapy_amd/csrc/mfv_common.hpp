@@ -330,8 +330,10 @@ __device__ __forceinline__ double sw_cell_dt(const Mesh &m, int i, double h, dou
 
 int validate_mesh(const mfv_mesh *m, int need_lsq, int need_order_split, int need_order_sorted);
 
-// dt_dev[0] = min(1e6, part[0..n)) on the stream; if dt_host != NULL, waits for it there.
-int dt_total(const double *part, size_t n, double *dt_dev, double *dt_host, hipStream_t st);
+// dt_dev[0] = min(1e6, part[0..n)) on the stream; if dt_host != NULL, also there: kIdle waits for the
+// stream, kDt only for the value (and so for all work before it).
+enum DtWait { kIdle, kDt };
+int dt_total(const double *part, size_t n, double *dt_dev, double *dt_host, DtWait wait, hipStream_t st);
 
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 

@@ -776,8 +776,8 @@ __global__ void __launch_bounds__(1024) k_dt_finish(const double *__restrict__ p
     if (threadIdx.x == 0 && r < out[0]) out[0] = r;
 }
 
-// out[0] = min(1e6, min part), and the same to host memory if given (k_dt_total's own start value:
-// no launch to reset out[0] first).
+// out[0] = min(1e6, min part), and then the same to host memory if given, in release order at system
+// scope (k_dt_total's own start value: no launch to reset out[0] first).
 __global__ void __launch_bounds__(1024) k_dt_total(const double *__restrict__ part, size_t n,
                                                    double *__restrict__ out, double *host)
 {
@@ -785,7 +785,7 @@ __global__ void __launch_bounds__(1024) k_dt_total(const double *__restrict__ pa
     if (threadIdx.x == 0) {
         const double dt = (r < 1e6) ? r : 1e6;
         out[0] = dt;
-        if (host) __hip_atomic_store(host, dt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (host) __hip_atomic_store(host, dt, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -832,11 +832,13 @@ void give_dt_slot(double *p)
 
 }  // namespace
 
-// A dt that the host waits for is written to pinned memory by the fold itself and looked at there:
-// a copy to the caller's (pageable) double is a launch of its own and a wait for its signal on top.
-// The sequence of four 3D advection steps 577 -> 441 us, four of the SRNH scheme at 1k cells
-// (eight dts) 572 -> 354 us.
-int mfv::dt_total(const double *part, size_t n, double *dt_dev, double *dt_host, hipStream_t st)
+// A dt that the host asks for is written to pinned memory by the fold itself: a copy to the caller's
+// (pageable) double is a launch of its own. kIdle then waits for the stream, as any *_host output
+// promises. kDt looks at the pinned word instead, which the fold stores last and with release order:
+// whoever sees it also sees dt_dev and what the stream held before it, but the kernel itself may not have
+// retired. Four 3D advection steps take 328 us with kIdle and 306 us with kDt, four of the SRNH scheme at
+// 1k cells (eight dts) 338 and 278 us, of Euler at 8k 138 and 120, of advection-diffusion 332 and 240.
+int mfv::dt_total(const double *part, size_t n, double *dt_dev, double *dt_host, DtWait wait, hipStream_t st)
 {
     double *slot = nullptr;
     volatile long long *word = nullptr;
@@ -856,8 +858,9 @@ int mfv::dt_total(const double *part, size_t n, double *dt_dev, double *dt_host,
     int rc = check_launch("dt kernel");
     if (slot) {
         if (rc == MFV_OK) {
-            for (int k = 0; k < 200000 && *word == kWaiting; k++) __builtin_ia32_pause();
-            if (*word == kWaiting) {  // a long queue ahead, or an error: wait as for any other work
+            if (wait == kDt)
+                for (int k = 0; k < 200000 && *word == kWaiting; k++) __builtin_ia32_pause();
+            if (*word == kWaiting || wait == kIdle) {  // kDt: a long queue ahead, or an error
                 const hipError_t e = hipStreamSynchronize(st);
                 if (e != hipSuccess) {
                     set_error("dt readback: %s", hipGetErrorString(e));
@@ -907,8 +910,8 @@ __global__ void __launch_bounds__(kBlock) k_adv_time_step(Mesh m, const double *
     wave_min_part(dtpart, (size_t)i, d);
 }
 
-extern "C" int mfv_time_step(const mfv_mesh *m, const double *u, const double *v, const double *w, double cfl,
-                             double *dt_dev, double *dt_host, void *stream)
+static int time_step(const mfv_mesh *m, const double *u, const double *v, const double *w, double cfl, double *dt_dev,
+                     double *dt_host, DtWait wait, void *stream)
 {
     if (int rc = validate_mesh(m, 0, 0, 0)) return rc;
     MFV_REQUIRE(u && v && w && dt_dev, "NULL array");
@@ -921,7 +924,19 @@ extern "C" int mfv_time_step(const mfv_mesh *m, const double *u, const double *v
         hipLaunchKernelGGL(k, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream), to_kernel(m), u, v, w,
                            cfl, part);
     }
-    return dt_total(part, nw, dt_dev, dt_host, as_stream(stream));
+    return dt_total(part, nw, dt_dev, dt_host, wait, as_stream(stream));
+}
+
+extern "C" int mfv_time_step(const mfv_mesh *m, const double *u, const double *v, const double *w, double cfl,
+                             double *dt_dev, double *dt_host, void *stream)
+{
+    return time_step(m, u, v, w, cfl, dt_dev, dt_host, kIdle, stream);
+}
+
+extern "C" int mfv_time_step_polled(const mfv_mesh *m, const double *u, const double *v, const double *w, double cfl,
+                                    double *dt_dev, double *dt_host, void *stream)
+{
+    return time_step(m, u, v, w, cfl, dt_dev, dt_host, kDt, stream);
 }
 
 // Residual of cell i by the upwind flux (compute_upwind_flux, fvm_utils.py:5-17) with the MUSCL

@@ -710,9 +710,9 @@ extern "C" int mfv_explicitscheme_dissipative(const mfv_mesh *m, const double *w
     return check_launch("k_dissipative");
 }
 
-extern "C" int mfv_time_step_diffusion(const mfv_mesh *m, const double *u, const double *v, const double *w,
-                                       double cfl, double Dxx, double Dyy, double Dzz, double *dt_dev,
-                                       double *dt_host, void *stream)
+static int time_step_diffusion(const mfv_mesh *m, const double *u, const double *v, const double *w, double cfl,
+                               double Dxx, double Dyy, double Dzz, double *dt_dev, double *dt_host, DtWait wait,
+                               void *stream)
 {
     if (int rc = validate_mesh(m, 0, 0, 0)) return rc;
     MFV_REQUIRE(dt_dev, "NULL dt_dev");
@@ -728,5 +728,19 @@ extern "C" int mfv_time_step_diffusion(const mfv_mesh *m, const double *u, const
         hipLaunchKernelGGL(k, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream), to_kernel(m), u, v, w,
                            cfl, Dxx, Dyy, Dzz, part);
     }
-    return dt_total(part, nw, dt_dev, dt_host, as_stream(stream));
+    return dt_total(part, nw, dt_dev, dt_host, wait, as_stream(stream));
+}
+
+extern "C" int mfv_time_step_diffusion(const mfv_mesh *m, const double *u, const double *v, const double *w,
+                                       double cfl, double Dxx, double Dyy, double Dzz, double *dt_dev,
+                                       double *dt_host, void *stream)
+{
+    return time_step_diffusion(m, u, v, w, cfl, Dxx, Dyy, Dzz, dt_dev, dt_host, kIdle, stream);
+}
+
+extern "C" int mfv_time_step_diffusion_polled(const mfv_mesh *m, const double *u, const double *v, const double *w,
+                                              double cfl, double Dxx, double Dyy, double Dzz, double *dt_dev,
+                                              double *dt_host, void *stream)
+{
+    return time_step_diffusion(m, u, v, w, cfl, Dxx, Dyy, Dzz, dt_dev, dt_host, kDt, stream);
 }

@@ -1295,8 +1295,8 @@ extern "C" int mfv_update_euler_3d_fvc(const mfv_mesh *m, const mfv_euler_arrays
     return check_launch("k_euler_update");
 }
 
-extern "C" int mfv_euler3d_time_step(const mfv_mesh *m, const double *U, double cfl, double gamma, double *dt_dev,
-                                     double *dt_host, void *stream)
+static int euler3d_time_step(const mfv_mesh *m, const double *U, double cfl, double gamma, double *dt_dev,
+                             double *dt_host, DtWait wait, void *stream)
 {
     if (int rc = validate_mesh(m, 0, 0, 0)) return rc;
     MFV_REQUIRE(m->dim == 3 && m->max_cell_faces >= 4, "Euler 3D time step needs tetrahedra");
@@ -1309,7 +1309,19 @@ extern "C" int mfv_euler3d_time_step(const mfv_mesh *m, const double *U, double 
         hipLaunchKernelGGL(k_euler_dt, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream), to_kernel(m),
                            U, cfl, gamma, part);
     }
-    return dt_total(part, nw, dt_dev, dt_host, as_stream(stream));
+    return dt_total(part, nw, dt_dev, dt_host, wait, as_stream(stream));
+}
+
+extern "C" int mfv_euler3d_time_step(const mfv_mesh *m, const double *U, double cfl, double gamma, double *dt_dev,
+                                     double *dt_host, void *stream)
+{
+    return euler3d_time_step(m, U, cfl, gamma, dt_dev, dt_host, kIdle, stream);
+}
+
+extern "C" int mfv_euler3d_time_step_polled(const mfv_mesh *m, const double *U, double cfl, double gamma,
+                                            double *dt_dev, double *dt_host, void *stream)
+{
+    return euler3d_time_step(m, U, cfl, gamma, dt_dev, dt_host, kDt, stream);
 }
 
 extern "C" int mfv_euler3d_rusanov(const mfv_mesh *m, const double *U, const double *G, double gamma, int quirk,
@@ -1554,7 +1566,7 @@ extern "C" int mfv_euler3d_load(const mfv_mesh *m, const double *U, const int64_
         hipLaunchKernelGGL(k_euler_load, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream), to_kernel(m),
                            U, perm, cfl, gamma, rec, part);
     }
-    return dt_total(part, nw, dt_dev, nullptr, as_stream(stream));
+    return dt_total(part, nw, dt_dev, nullptr, kIdle, as_stream(stream));
 }
 
 extern "C" int mfv_euler3d_store(const mfv_mesh *m, const double *rec, const int64_t *perm, double *U, void *stream)

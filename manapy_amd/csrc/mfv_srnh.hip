@@ -478,7 +478,7 @@ extern "C" int mfv_srnh_run(const mfv_mesh *m, const mfv_srnh_step *p, int order
                            grav, cfl, dts + s, last, fold && s > 0 ? (int)nw : 0, mine);
         if (int rc = check_launch("k_srnh_cell")) return rc;
         if (!fold || s == nsteps - 1)
-            if (int rc = dt_total(mine, nw, dts + s + 1, nullptr, st)) return rc;
+            if (int rc = dt_total(mine, nw, dts + s + 1, nullptr, kIdle, st)) return rc;
     }
     return MFV_OK;
 }

@@ -328,9 +328,9 @@ __global__ void __launch_bounds__(kBlock) k_sw_step(Mesh m, const double *__rest
 
 }  // namespace
 
-extern "C" int mfv_time_step_sw(const mfv_mesh *m, const double *h, const double *hu, const double *hv,
-                                double cfl, double grav, double Dxx, double Dyy, double *dt_dev, double *dt_host,
-                                void *stream)
+static int time_step_sw(const mfv_mesh *m, const double *h, const double *hu, const double *hv, double cfl,
+                        double grav, double Dxx, double Dyy, double *dt_dev, double *dt_host, DtWait wait,
+                        void *stream)
 {
     if (int rc = validate_mesh(m, 0, 0, 0)) return rc;
     MFV_REQUIRE(h && hu && hv && dt_dev, "NULL array");
@@ -345,7 +345,20 @@ extern "C" int mfv_time_step_sw(const mfv_mesh *m, const double *h, const double
         hipLaunchKernelGGL(k, dim3(grid_for(m->nb_cells)), dim3(kBlock), 0, as_stream(stream), to_kernel(m), h, hu, hv,
                            cfl, grav, Dxx, Dyy, part);
     }
-    return dt_total(part, nw, dt_dev, dt_host, as_stream(stream));
+    return dt_total(part, nw, dt_dev, dt_host, wait, as_stream(stream));
+}
+
+extern "C" int mfv_time_step_sw(const mfv_mesh *m, const double *h, const double *hu, const double *hv, double cfl,
+                                double grav, double Dxx, double Dyy, double *dt_dev, double *dt_host, void *stream)
+{
+    return time_step_sw(m, h, hu, hv, cfl, grav, Dxx, Dyy, dt_dev, dt_host, kIdle, stream);
+}
+
+extern "C" int mfv_time_step_sw_polled(const mfv_mesh *m, const double *h, const double *hu, const double *hv,
+                                       double cfl, double grav, double Dxx, double Dyy, double *dt_dev,
+                                       double *dt_host, void *stream)
+{
+    return time_step_sw(m, h, hu, hv, cfl, grav, Dxx, Dyy, dt_dev, dt_host, kDt, stream);
 }
 
 extern "C" int mfv_sw_gradients(const mfv_mesh *m, const double *h, const double *hu, const double *hv,

@@ -162,8 +162,8 @@ class ServingEngine(object):
         _lib.call('mfv_facetocell', dm.ptr, vf.data_ptr(), vc.data_ptr(), s)
         dt_dev = torch.zeros(1, dtype=torch.float64, device=dev)
         h = ctypes.c_double(0.)
-        _lib.call('mfv_time_step', dm.ptr, uc.data_ptr(), vc.data_ptr(), wc.data_ptr(), req.cfl, dt_dev.data_ptr(),
-                  ctypes.byref(h), s)
+        _lib.call('mfv_time_step_polled', dm.ptr, uc.data_ptr(), vc.data_ptr(), wc.data_ptr(), req.cfl,
+                  dt_dev.data_ptr(), ctypes.byref(h), s)
         req.dt = h.value
         # matrix of the all-Neumann diamond operator, then the geometry tables are dropped
         dd = DeviceDiamond(dm, host=getattr(d, '_diamond_host', None), without=_UNREAD)

@@ -77,7 +77,7 @@ class AdvectionSolver(object):
     def stepper(self):
         """``system.py:129-133``: dt = min_K cfl |K| / sum_f |u_K . n_f|."""
         h = ctypes.c_double(0.)
-        _lib.call('mfv_time_step', self._m.ptr, self.u.cell.data_ptr(), self.v.cell.data_ptr(),
+        _lib.call('mfv_time_step_polled', self._m.ptr, self.u.cell.data_ptr(), self.v.cell.data_ptr(),
                   self.w.cell.data_ptr(), float(self.cfl), self._dt_dev.data_ptr(), ctypes.byref(h), stream_ptr())
         self.dt = h.value
         return self.dt

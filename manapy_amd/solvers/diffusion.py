@@ -93,7 +93,7 @@ class DiffusionSolver(object):
         h = ctypes.c_double(0.)
         uvw = (self.u.cell.data_ptr(), self.v.cell.data_ptr(), self.w.cell.data_ptr()) if self._convective \
             else (None, None, None)
-        _lib.call('mfv_time_step_diffusion', self._m.ptr, *uvw, float(self.cfl), float(self.Dxx), float(self.Dyy),
+        _lib.call('mfv_time_step_diffusion_polled', self._m.ptr, *uvw, float(self.cfl), float(self.Dxx), float(self.Dyy),
                   float(self.Dzz), self._dt_dev.data_ptr(), ctypes.byref(h), stream_ptr())
         self.dt = h.value
         return self.dt

@@ -75,7 +75,7 @@ class EulerSolver3D(object):
 
     def stepper(self):
         hd = ctypes.c_double(0.)
-        _lib.call('mfv_euler3d_time_step', self._m.ptr, self.U.data_ptr(), self.cfl, self.gamma,
+        _lib.call('mfv_euler3d_time_step_polled', self._m.ptr, self.U.data_ptr(), self.cfl, self.gamma,
                   self._dt_dev.data_ptr(), ctypes.byref(hd), stream_ptr())
         self.dt = hd.value
         return self.dt

@@ -134,7 +134,7 @@ class ShallowWaterSolver(object):
 
     def _srnh_dt(self, dt_dev, host):
         hd = ctypes.c_double(0.) if host else None
-        _lib.call('mfv_time_step_sw', self._m.ptr, self.h.cell.data_ptr(), self.hu.cell.data_ptr(),
+        _lib.call('mfv_time_step_sw_polled', self._m.ptr, self.h.cell.data_ptr(), self.hu.cell.data_ptr(),
                   self.hv.cell.data_ptr(), self.cfl, self.grav, float(self.Dxx), float(self.Dyy), dt_dev.data_ptr(),
                   ctypes.byref(hd) if host else None, stream_ptr())
         return hd.value if host else None
@@ -184,7 +184,7 @@ class ShallowWaterSolver(object):
             self.dt = self._srnh_dt(self._dt_dev, True)
             return self.dt
         hd = ctypes.c_double(0.)
-        _lib.call('mfv_time_step_sw', self._m.ptr, self.h.cell.data_ptr(), self.hu.cell.data_ptr(),
+        _lib.call('mfv_time_step_sw_polled', self._m.ptr, self.h.cell.data_ptr(), self.hu.cell.data_ptr(),
                   self.hv.cell.data_ptr(), self.cfl, self.grav, float(self.Dxx), float(self.Dyy),
                   self._dt_dev.data_ptr(), ctypes.byref(hd), stream_ptr())
         self.dt = hd.value

@@ -103,3 +103,64 @@ def test_refused_under_capture():
             g.capture_end()
     torch.cuda.synchronize()
     assert _dt(d.device_mesh, u, dev, stream_ptr()) == float(dev)
+
+
+def _time_steps(d, u, dev, form, stream):
+    """(name, call) of the four time steps with a host dt, in one of their two forms."""
+    import torch
+    from manapy_amd import _lib
+    m, P = d.device_mesh, lambda *ts: [t.data_ptr() for t in ts]
+    h = ctypes.c_double(-1.)
+
+    def call(name, *args):
+        _lib.call(name + form, m.ptr, *args, dev.data_ptr(), ctypes.byref(h), stream)
+        return h.value
+
+    out = [("mfv_time_step", lambda: call("mfv_time_step", *P(*u), .4)),
+           ("mfv_time_step_diffusion", lambda: call("mfv_time_step_diffusion", *P(*u), .4, .1, .1, .1))]
+    if m.dim == 2:
+        pos = u[0].abs() + 1.
+        out.append(("mfv_time_step_sw", lambda: call("mfv_time_step_sw", *P(pos, u[1], u[2]), .4, 9.81, 0., 0.)))
+    else:
+        U = torch.stack([u[0].abs() + 1., u[0].abs() + 2., u[0], u[1], u[2], u[0].abs() + 9.])
+        out.append(("mfv_euler3d_time_step", lambda: call("mfv_euler3d_time_step", U.data_ptr(), .4, 1.4)))
+    return out
+
+
+@pytest.mark.parametrize("make,size", [(make_tri_domain, (200, 170)), (make_tet_domain, (6,))])
+def test_the_stream_is_idle_after_a_host_dt(make, size):
+    """include/mfv.h: a call with a *_host output synchronises its stream."""
+    import torch
+    d = make(*size)
+    u, dev = _setup(d, 6)
+    torch.cuda.synchronize()
+    s = torch.cuda.Stream()
+    for name, call in _time_steps(d, u, dev, "", s.cuda_stream):
+        for _ in range(50):
+            call()
+            assert s.query(), name
+
+
+@pytest.mark.parametrize("make,size", [(make_tri_domain, (200, 170)), (make_tet_domain, (6,))])
+def test_the_polled_dt_is_seen_on_any_stream(make, size):
+    """The polled form: dt_dev and what the stream held before it are there for work that the caller
+    starts next on another stream, with no synchronisation between."""
+    import torch
+    d = make(*size)
+    u, dev = _setup(d, 7)
+    torch.cuda.synchronize()
+    s, other = torch.cuda.Stream(), torch.cuda.Stream()
+    for name, call in _time_steps(d, u, dev, "_polled", s.cuda_stream):
+        idle = dict(_time_steps(d, u, dev, "", s.cuda_stream))[name]()
+        before = torch.zeros(1 << 20, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        for k in range(1, 51):
+            with torch.cuda.stream(s):
+                before.fill_(k)
+                dev.fill_(-1.)
+            got = call()
+            with torch.cuda.stream(other):
+                seen, sees = dev.clone(), before.clone()
+            other.synchronize()
+            assert got == idle == float(seen) and bool((sees == k).all()), (name, k)
+        s.synchronize()
