@@ -486,6 +486,11 @@ int mfv_sw_batch_step_tiled(const mfv_mesh *m, const mfv_sw_mixed *p, const mfv_
 int mfv_sw_batch_graph_tiled(const mfv_mesh *m, const mfv_sw_mixed *p, const mfv_sw_batch *b,
                              const mfv_sw_tiles *t, double *state2, double grav, double cfl, int order,
                              int nsteps, void **graph_out);
+/* Whether the steps of mfv_sw_batch_graph_tiled fold the dt themselves (folds_host = 1) or leave it
+ * to a launch a step: by the partials that all tiles read together. Same bits; host arrays. */
+int mfv_sw_batch_fold_rule(int nb_cells, int nb_inst, const int32_t *inst_ncells_host, int nb_waves,
+                           const int32_t *wave_inst_host, int nb_tiles, const int32_t *tile_cell0_host,
+                           int *folds_host);
 int mfv_graph_launch(void *graph, void *stream);
 int mfv_graph_destroy(void *graph);
 

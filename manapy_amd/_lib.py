@@ -324,6 +324,7 @@ _SIGNATURES = {
     'mfv_sw_batch_step_tiled': [MESH_P, SWM_P, SWB_P, SWT_P, P, c_double, c_double, c_int, c_int, P],
     'mfv_sw_batch_graph_tiled': [MESH_P, SWM_P, SWB_P, SWT_P, P, c_double, c_double, c_int, c_int,
                                  ctypes.POINTER(c_void_p)],
+    'mfv_sw_batch_fold_rule': [c_int, c_int, P, c_int, P, c_int, P, ctypes.POINTER(c_int)],
     'mfv_sw_batch_conservation': [MESH_P, SWM_P, SWB_P, P, P],
     'mfv_sw_batch_graph': [MESH_P, SWM_P, SWB_P, c_double, c_double, c_int, c_int, c_int, ctypes.POINTER(c_void_p)],
     'mfv_graph_launch': [c_void_p, P],

@@ -18,6 +18,8 @@
 // dt and the conservation totals are float64.
 #include "mfv_common.hpp"
 
+#include <stdlib.h>
+
 namespace {
 
 using namespace mfv;
@@ -1220,15 +1222,54 @@ static int batch_tiled_launch(const mfv_mesh *m, const mfv_sw_mixed *p, const mf
     return check_launch("k_batch_dt_fold");
 }
 
-// Whether the steps of a graph fold the dt themselves: every tile reads its instance's partials, so
-// all tiles together must read little beside the step's own traffic (300 bytes a cell). 30 steps: four
-// instances of 31k cells together 358 -> 309 us, eight of 93k 458 -> 389 us, 24 of 615k (3222 tiles,
-// 10 MB) 1331 -> 1314 us.
-static bool batch_folds(const mfv_mesh *m, const mfv_sw_batch *b, const mfv_sw_tiles *t)
+// The rule by which the steps of a graph fold the dt themselves (host tables): every tile reads the
+// partials of its instance, tiles_i waves_i of them for instance i, so that an instance much larger than
+// the others weighs by its square. That costs each round of resident tiles a trip to memory and the bytes;
+// the launch that it saves is about 2 us a step. Up to two rounds it pays up to some 100 MB; with more
+// rounds it is even at best and needs the bytes to be little beside the step's own 300 a cell. Steps with
+// the fold against a launch each, tiles of 256 threads, one instance / 24 even ones / one large with 15 of
+// 5k cells: 100k cells in all (about 520 tiles) 446 / 446 / 449 against 520 / 479 / 496 us for 30 steps,
+// 300k (1570 tiles; 58, 2 and 33 MB) 904 / 844 / 882 against 979 / 885 / 942, 400k (2090; 105, 4, 69 MB)
+// 1162 / 1013 / 1084 against 1167 / 1008 / 1143, 600k (3140; 235, 10, 181 MB) 1638 / 1339 / 1552 against
+// 1549 / 1336 / 1542, 800k (4175; 417, 17, 342 MB) 2177 / 1646 / 2065 against 1956 / 1631 / 1937.
+extern "C" int mfv_sw_batch_fold_rule(int nb_cells, int nb_inst, const int32_t *inst_ncells_host, int nb_waves,
+                                      const int32_t *wave_inst_host, int nb_tiles, const int32_t *tile_cell0_host,
+                                      int *folds_host)
 {
-    const double bytes = 8. * t->nb_tiles * ((double)b->nb_waves / b->nb_inst);
-    return bytes <= 64e6 && bytes <= 30. * m->nb_cells &&
-           tiles_lds_bytes(t, m->max_cell_faces) + (t->tile_size / 64) * sizeof(double) <= 64 * 1024;
+    MFV_REQUIRE(nb_cells >= 0 && nb_inst >= 1 && nb_waves >= 0 && nb_tiles >= 0, "bad sizes");
+    MFV_REQUIRE(inst_ncells_host && wave_inst_host && tile_cell0_host && folds_host, "NULL array");
+    double bytes = 0.;
+    for (int k = 0; k < nb_tiles; k++) {
+        const int w = tile_cell0_host[k] >> 6;
+        MFV_REQUIRE(w >= 0 && w < nb_waves, "tile %d starts at cell %d of %d waves", k, tile_cell0_host[k], nb_waves);
+        const int i = wave_inst_host[w];
+        MFV_REQUIRE(i >= 0 && i < nb_inst, "wave %d belongs to instance %d of %d", w, i, nb_inst);
+        bytes += 8. * ((inst_ncells_host[i] + 63) / 64);
+    }
+    *folds_host = nb_tiles <= 2100 ? bytes <= 100e6 : bytes <= 64e6 && bytes <= 30. * nb_cells;
+    return MFV_OK;
+}
+
+// The same for descriptors on the device, whose three small tables are copied once a graph, on a stream
+// of the graph's own. It decides on speed alone: what cannot be read or told takes the launch a step.
+static bool batch_folds(const mfv_mesh *m, const mfv_sw_batch *b, const mfv_sw_tiles *t, hipStream_t st)
+{
+    if (tiles_lds_bytes(t, m->max_cell_faces) + (t->tile_size / 64) * sizeof(double) > 64 * 1024) return false;
+    const size_t n[3] = {(size_t)b->nb_inst, (size_t)b->nb_waves, (size_t)t->nb_tiles};
+    const int32_t *dev[3] = {b->inst_ncells, b->wave_inst, t->tile_cell0};
+    int32_t *host = static_cast<int32_t *>(malloc((n[0] + n[1] + n[2]) * sizeof(int32_t)));
+    if (!host) return false;
+    int32_t *at[3] = {host, host + n[0], host + n[0] + n[1]};
+    hipError_t e = hipSuccess;
+    for (int k = 0; k < 3 && e == hipSuccess; k++)
+        e = hipMemcpyAsync(at[k], dev[k], n[k] * sizeof(int32_t), hipMemcpyDeviceToHost, st);
+    const hipError_t done = hipStreamSynchronize(st);
+    int folds = 0;
+    if (e == hipSuccess && done == hipSuccess)
+        if (mfv_sw_batch_fold_rule(m->nb_cells, b->nb_inst, at[0], b->nb_waves, at[1], t->nb_tiles, at[2], &folds))
+            folds = 0;
+    free(host);
+    return folds != 0;
 }
 
 extern "C" int mfv_sw_batch_step_tiled(const mfv_mesh *m, const mfv_sw_mixed *p, const mfv_sw_batch *b,
@@ -1261,10 +1302,10 @@ extern "C" int mfv_sw_batch_graph_tiled(const mfv_mesh *m, const mfv_sw_mixed *p
                 nsteps);
     *graph_out = nullptr;
     MfvGraph *g = new MfvGraph();
-    const bool folds = batch_folds(m, b, t);
     const size_t nw = (size_t)m->nb_cells / 64 + 1;
-    hipError_t e = hipMalloc(reinterpret_cast<void **>(&g->part), (folds ? 2 : 1) * nw * sizeof(double));
-    if (e == hipSuccess) e = hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking);
+    hipError_t e = hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking);
+    const bool folds = e == hipSuccess && m->nb_cells && batch_folds(m, b, t, g->stream);
+    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&g->part), (folds ? 2 : 1) * nw * sizeof(double));
     if (e == hipSuccess) e = hipStreamBeginCapture(g->stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) {
         set_error("graph capture setup: %s", hipGetErrorString(e));

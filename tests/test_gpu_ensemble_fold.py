@@ -29,3 +29,8 @@ def test_graph_equals_eager(sizes, config):
         assert torch.equal(a.state, b.state)
         assert torch.equal(a.rings, b.rings)
         a.rings[:, 3] += 0.  # eager work of the caller's between replays
+
+
+def test_graph_with_a_fold_launch_a_step():
+    """More than 2100 tiles whose instance is large: the rule (mfv_sw_batch_fold_rule) leaves the dt to a launch."""
+    test_graph_equals_eager([(300, 240), (3, 2)], ("staged", 128, 64))
