@@ -126,6 +126,7 @@ class EllBatch(object):
         self._ranges = RangeAllocator(S)
         self._inst = {}                # inst -> (slice0, nslices, nrows)
         self._free_ids = list(range(I - 1, -1, -1))
+        self._slice_bytes = self._count_slice_bytes()
 
     def enable_advection(self, slots):
         """Time steps on the device (mfv_krylov_fused_tick with steps_left): tables of ``slots``
@@ -138,6 +139,7 @@ class EllBatch(object):
         for k in ('steps_left', 'adv_up', 'adv_coef', 'adv_vol'):
             setattr(self._w, k, getattr(self, k).data_ptr())
         self._w.adv_slots = int(slots)
+        self._slice_bytes = self._count_slice_bytes()
 
     # -- arena ----------------------------------------------------------------------------------
     @property
@@ -149,8 +151,16 @@ class EllBatch(object):
         return ctypes.byref(self._w)
 
     def bytes_per_slice(self):
-        """HBM bytes one slice of an instance occupies (matrix slots, vectors, partials)."""
-        return self.W * 64 * (4 + 2 + 8 + 4) + 64 * (8 + 8 + 8 + 8 * 4) + 4 * 8 + 8 + 1
+        """HBM bytes one slice of an instance occupies: matrix slots, vectors, chunk sums and lists, and the
+        advection tables once they are enabled."""
+        return self._slice_bytes
+
+    def _count_slice_bytes(self):
+        own = [self.slice_inst, self.slice_w, self.slice_narrow, self.cols, self.cols16, self.vals, self.vals32,
+               self.diag, self.live_slices, self.chunks, self.x, self.b]
+        own += list(self.f32.values()) + list(self.partial.values())
+        own += [getattr(self, k) for k in ('adv_up', 'adv_coef', 'adv_vol') if hasattr(self, k)]
+        return sum(t.numel() * t.element_size() for t in own) // max(1, self.S)
 
     def free_slices(self):
         return self._ranges.available()

@@ -11,10 +11,10 @@ of the advection (constant, the velocity is constant). The implicit system is so
 ``||b - M x|| <= tol ||b||`` (default 1e-10) by the arena solver of ``krylov.EllBatch``.
 
 ``ServingEngine.run`` admits requests as they arrive while the arena has room for them
-(HBM footprint: contiguous matrix slices plus the request's mesh tables, under a byte
-budget), keeps every admitted request's state on the device between steps, and advances
-all of them together: each engine tick launches the advection of the requests entering a
-new step and one solver tick for every system in the arena, whatever stage it is at.
+(HBM footprint: contiguous arena slices, under a byte budget), keeps every admitted
+request's state on the device between steps, and advances all of them together: each
+engine tick is one solver tick for every system in the arena, whatever stage it is at,
+the advection that begins a request's next step among them.
 Requests therefore overlap on the device; each request's arithmetic is independent of the
 others (per-request kernels, position-independent batched solver), so a result is the
 same alone and in any mix.
@@ -30,7 +30,7 @@ from .diamond import DeviceDiamond
 from .krylov import EllBatch
 
 # What admission (matrix, face velocities, time step) does not read of the mesh and diamond tables:
-# 190 of 330 bytes a cell, whose copies were most of an admission (eight requests 8.9 -> 6.1 ms).
+# 223 of 402 bytes a triangle, whose copies were most of an admission (eight requests 8.9 -> 6.1 ms).
 _UNREAD = ('face_name', 'face_mesure', 'face_center', 'face_ghost', 'cell_center', 'bnd_faces', 'face_fk', 'face_air',
            'node_ghost_face')
 
@@ -98,12 +98,10 @@ class AdvDiffRequest(object):
         return self._mesh_host is not None
 
     def footprint(self, arena):
-        """Bytes the request holds on the device while admitted."""
-        slices = (self.C + 63) // 64
-        F = int(self.domain.nbfaces)
-        mesh = self.C * (8 * 4 + 4 * 4 + 2) + F * (4 * 3 + 8 * 8)   # mfv_mesh tables (no LSQ)
-        fields = 8 * (3 * F + 3 * self.C) + 64
-        return slices * arena.bytes_per_slice() + mesh + fields
+        """Bytes the request holds on the device while admitted: its slices of the arena. The mesh
+        and diamond tables that its admission reads are on the device during that call alone (one
+        request's at a time, 460 bytes a triangle with the velocities) and not part of it."""
+        return (self.C + 63) // 64 * arena.bytes_per_slice()
 
 
 class ServingEngine(object):
