@@ -162,7 +162,8 @@ class DeviceMesh(object):
 
     def stencil_tiles(self):
         """The mesh's StencilTiles, or None where the gradients gather from memory: 2D meshes (a
-        dozen neighbours), cells of more than four faces, tiles that do not fit the LDS."""
+        dozen neighbours), cells of more than four faces, tiles that do not fit the LDS or their
+        16-bit positions (then the builder refuses them)."""
         self.ensure_lsq()
         if self._stencil_tiles is None:
             import torch
@@ -172,8 +173,11 @@ class DeviceMesh(object):
             host = self._lsq_host if self._lsq_host is not None else self.host
             if self.dim == 3 and self.MF <= 4 and self.C and host['K']:
                 from .renumber import morton_order_3d
-                t = StencilTiles(host, morton_order_3d(*host['cell_center'].T), self.device)
-                if t.desc.max_ext > 2048:
+                try:
+                    t = StencilTiles(host, morton_order_3d(*host['cell_center'].T), self.device)
+                except _lib.MfvError:
+                    t = None
+                if t is not None and t.desc.max_ext > 2048:
                     t = None
             self._stencil_tiles, self._lsq_host = t or False, None
         return self._stencil_tiles or None

@@ -64,3 +64,26 @@ def test_tiled_gradient_equals_the_gathering_one(n):
     _lib.call("mfv_cell_gradient_limited", m.ptr, 1, f, stream_ptr())
     for a, b in zip(got, (v.gradcellx, v.gradcelly, v.gradcellz, v.psi)):
         np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())
+
+
+def test_stencils_too_wide_for_a_tile_are_gathered(monkeypatch):
+    """A tile that reads more cells than its 16-bit positions tell apart: the builder refuses it and the
+    mesh has no tiles, so that its gradients gather from memory as without them."""
+    from types import SimpleNamespace
+    import torch
+    from manapy_amd import _lib
+    from manapy_amd.device import DeviceMesh, StencilTiles
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)  # asks for a device
+    C, K = 66600, 260
+    cells = np.zeros((K, C), dtype=np.int32)
+    cells[:, :256] = np.arange(256 * K, dtype=np.int32).reshape(K, 256)
+    count = np.where(np.arange(C) < 256, K, 0).astype(np.int32)
+    x = np.linspace(0., 1., C)
+    host = {"C": C, "K": K, "lsq_cells": cells, "lsq_ncells": count, "cell_center": np.stack([x, x, x], axis=1)}
+    with pytest.raises(_lib.MfvError, match="65535"):
+        StencilTiles(host, np.arange(C), "cpu")
+    mesh = SimpleNamespace(ensure_lsq=lambda: None, _stencil_tiles=None, _lsq_host=None, host=host, dim=3, MF=4, C=C,
+                           device="cpu")
+    assert DeviceMesh.stencil_tiles(mesh) is None
+    assert DeviceMesh.stencil_tiles(mesh) is None  # and does not build them again
+    assert mesh._stencil_tiles is False
