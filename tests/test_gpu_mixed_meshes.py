@@ -117,3 +117,30 @@ def test_mixed_paths_on_triangles_and_quads(oracle_lib, T, stage):
         dt = model.step(G, 0.8, dt)
     for k in range(3):
         assert np.array_equal(runs[0][0][:, k], model.state[:, k]), k
+
+
+@pytest.mark.parametrize("order", [1, 2])
+def test_unpacked_step_on_triangles_and_quads(oracle_lib, order):
+    """mfv_sw_step_fused takes its time step's faces by the mesh's face count (four slots, three used)."""
+    import torch
+    from manapy_amd import _lib
+    from manapy_amd.device import DeviceMesh, stream_ptr
+    d, Z, h0 = _case(False)
+    C = int(d.nbcells)
+    h, hu, hv = h0.copy(), np.zeros(C), np.zeros(C)
+    zg = oracle_lib.z_gradient(d, Z)
+    dts = [oracle_lib.sw_step(d, h, hu, hv, Z, zg, G, 0.8, order) for _ in range(5)]
+    m = DeviceMesh(d)
+    s = stream_ptr()
+    S = [_dev(np.stack([h0, np.zeros(C), np.zeros(C)])), _dev(np.zeros((3, C)))]
+    tZ, tg, grad, dt0, ring = _dev(Z), _dev(zg), _dev(np.zeros((9, C))), _dev(np.zeros(1)), _dev(np.zeros(4))
+    _lib.call('mfv_time_step_sw', m.ptr, *[S[0][k].data_ptr() for k in range(3)], 0.8, G, 0., 0., dt0.data_ptr(), None, s)
+    _lib.call('mfv_dt_ring_init', ring.data_ptr(), dt0.data_ptr(), s)
+    for k in range(5):
+        a, b = S[k % 2], S[1 - k % 2]
+        _lib.call('mfv_sw_gradients', m.ptr, *[a[j].data_ptr() for j in range(3)], tZ.data_ptr(), grad.data_ptr(), s)
+        _lib.call('mfv_sw_step_fused', m.ptr, a.data_ptr(), b.data_ptr(), tZ.data_ptr(), grad.data_ptr(), tg.data_ptr(), G,
+                  0.8, order, ring.data_ptr(), k, s)
+    for row, ref, name in zip(S[1].cpu().numpy(), (h, hu, hv), ('h', 'hu', 'hv')):
+        assert np.array_equal(row, ref), name
+    assert float(ring[4 % 3]) == dts[-1]
