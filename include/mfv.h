@@ -872,7 +872,9 @@ typedef struct mfv_krylov_work {
     int32_t *status;                                /* [I] */
 } mfv_krylov_work;
 
-/* One tick: refinement step (x += d, r = b - op(x) in FP64, convergence test) for instances in
+/* The general arena tick, eight launches an iteration (the library's own arenas run on
+ * mfv_krylov_fused_tick; this one needs no chunk lists and no aligned records, and its work arrays
+ * are the caller's): refinement step (x += d, r = b - op(x) in FP64, convergence test) for instances in
  * START/CORRECT, then n_iter BiCGStab iterations (FP32, Jacobi) for instances in INNER.
  * grid_slices / grid_inst are the persistent grid sizes (blocks of 256) of the per-slice and
  * per-instance kernels. Asynchronous; poll status[] between ticks. */
@@ -917,8 +919,11 @@ typedef struct mfv_krylov_fused {
 #define MFV_KRYLOV_SPAN(ns) (4 * (((ns) + 4 * MFV_KRYLOV_MAX_CHUNKS - 1) / (4 * MFV_KRYLOV_MAX_CHUNKS)))
 
 /* n_iter rounds of two launches, each one BiCGStab iteration of an instance in INNER or one change
- * of state of another one (refinement, convergence test, next time step); the same scalars and
- * stopping tests as mfv_krylov_tick. An instance set to MFV_KS_START solves its system once; one
+ * of state of another one (refinement, convergence test, next time step). The refinement and its
+ * stop (TOL_OUT on the FP64 residual, MAXIT_OUT) are those of mfv_krylov_tick. The inner solve is
+ * scaled from the left by the inverse diagonal, where mfv_krylov_tick applies it from the right:
+ * R0N2, RN2 and the stop TOL_IN are on the scaled residual, whose norm follows from the sums of the
+ * last product instead of a stored vector. An instance set to MFV_KS_START solves its system once; one
  * set to MFV_KS_ADVANCE takes steps_left time steps, each b = x + dt advection(x), x = b as the
  * first guess, then the solve, and is DONE after the last. grid_chunks: blocks of the kernels.
  * Asynchronous; poll status[] (and steps_left[]) between ticks. */

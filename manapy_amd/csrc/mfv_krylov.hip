@@ -7,10 +7,12 @@
 // Instances advance independently through a per-instance state machine kept in device memory
 // (status + scalars); every kernel runs a fixed persistent grid over the live-slice or
 // live-instance list and acts only on rows whose instance is in the state the kernel serves.
-// A tick (mfv_krylov_tick) is therefore valid for any mix of instances at any stage and can be
-// replayed from a captured graph while instances join and leave.
+// A tick is therefore valid for any mix of instances at any stage and can be replayed from a captured
+// graph while instances join and leave. mfv_krylov_fused_tick, two launches an iteration, is what the
+// package's arenas run on; mfv_krylov_tick, eight launches, is the ABI's general form and the solver
+// that the tests hold the other one against.
 //
-// Per-instance reductions are two-level and deterministic: each wave reduces its slice in a
+// Per-instance reductions of the latter are two-level and deterministic: each wave reduces its slice in a
 // fixed shuffle pattern into partial[slice], then one block per instance adds the partials of
 // its slices in a fixed order relative to its first slice. An instance's arithmetic therefore
 // does not depend on where it sits in the batch or on what else is in it.
@@ -465,7 +467,8 @@ __global__ void __launch_bounds__(256) k_ell_spmv(Ell e, const double *__restric
 //   t:  alpha from the sum of v;  s = r - alpha v;  t = M op(s);
 //                                           sums t.s, t.t, s.s, rh.s, rh.t
 //
-// * M = 1 / diag scales the rows of the product (the system M op(d) = M r), so a slot needs
+// * M = 1 / diag scales the rows of the product (the system M op(d) = M r), and the inner stop is on M r;
+//   so a slot needs
 //   nothing of its column but p (s), which is computed again from the column's record for each
 //   slot: three multiply-adds (one) and one gather of 16 bytes (8) instead of a launch and a
 //   trip of the vector through memory. The v product reads u = (s, t, p, v) and writes

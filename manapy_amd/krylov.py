@@ -1,16 +1,17 @@
-"""Arena of block-diagonal sparse systems solved on the GPU (``mfv_krylov_tick``).
+"""Arena of block-diagonal sparse systems solved on the GPU (``mfv_krylov_fused_tick``).
 
 An ``EllBatch`` owns one ELL matrix of ``max_slices`` 64-row slices and the vectors
 of the mixed-precision solver. Independent systems ``(sigma I + tau A) x = b``
 occupy contiguous slice ranges; ``alloc`` / ``release`` manage those ranges (first
-fit) and ``publish`` uploads the live-slice and live-instance lists that the
-persistent kernels walk. Because every device pointer and grid size stays fixed,
+fit) and ``publish`` uploads the live lists (slices, instances, chunks of slices) that
+the kernels walk. Because every device pointer and grid size stays fixed,
 one tick is valid for any set of instances at any stage of their solve, and each
 instance's arithmetic is independent of the others (see mfv_krylov.hip).
 
 The solver replaces the factorisation of ``ScipySolver`` / ``MUMPSSolver``
 (``solvers/ls/system.py:236-379, 624-744``): FP32 BiCGStab with Jacobi scaling
-inside FP64 iterative refinement, stopped at ``||b - A x|| <= tol ||b||``.
+inside FP64 iterative refinement, stopped at ``||b - A x|| <= tol ||b||``. The inner
+solves stop on the Jacobi-scaled residual (``tol_in``).
 """
 import collections
 import ctypes
@@ -291,7 +292,8 @@ class EllBatch(object):
         return max(1, min(4096, (nsl + 3) // 4)), max(1, ni)
 
     def tick(self, n_iter=8, grid_slices=None, grid_inst=None, stream=None, graph=False):
-        """One tick of every live instance (``grid_inst`` is unused: no kernel runs per instance). With ``graph=True`` the tick's launches are
+        """One tick of every live instance (``grid_slices``: blocks of its kernels; ``grid_inst`` is
+        taken and not used, no kernel runs per instance). With ``graph=True`` the tick's launches are
         replayed from a HIP graph captured once per (n_iter, grid size rounded up to a power of
         two): the kernels read the live lists from device memory, so a graph stays valid as
         instances come and go, and the result is the same bits as the eager tick."""

@@ -88,3 +88,34 @@ def test_solve_reaches_the_residual_in_as_many_iterations(nx, ny, n_iter):
     b.scal[inst * _lib.KS_NSCAL + _lib.KS_ITTOT] = 0.
     ref = _eight_launch_iterations(b, inst)
     assert abs(mine - ref) <= 0.15 * ref + 3, (mine, ref)
+
+
+# triangles between two Dirichlet sides, cells graded so that the diagonal varies by 2, 7e3, 1e2 and 1e4
+@pytest.mark.gpu
+@pytest.mark.skipif(not gpu_available(), reason="needs a ROCm GPU")
+@pytest.mark.parametrize("n,grade", [(12, 1.), (12, 100.), (30, 10.), (30, 100.)])
+def test_graded_system_without_a_shift(n, grade):
+    """sigma = 0 on a graded mesh, where the inner stop on the Jacobi-scaled residual is not the eight-launch
+    solver's: the FP64 residual still meets the outer stop, in no more iterations."""
+    import torch
+    from manapy_amd import Domain, Variable, _lib, jittered_triangles
+    from manapy_amd.solvers.ls import HIPKrylovSolver
+    el, nd = jittered_triangles(n, n, 1., 1., .1, n)
+    nd = nd.copy()
+    if grade > 1.:
+        nd[:, :2] = (grade ** nd[:, :2] - 1.) / (grade - 1.)
+    d = Domain(2, mesh=(el, nd))
+    var = Variable(domain=d, BC={"in": "dirichlet", "out": "dirichlet"}, values={"in": 1., "out": 2.})
+    sol = HIPKrylovSolver(domain=d, var=var)
+    C = int(d.nbcells)
+    sol(rhs=np.random.default_rng(n).standard_normal(C))
+    b, inst = sol._batch, sol._inst
+    row0 = b.rows(inst)[0]
+    y = torch.zeros_like(b.x)
+    b.spmv(b.x, y)
+    res = (b.b - y)[row0:row0 + C]
+    assert float(res.norm()) <= 1.0001e-10 * float(b.b[row0:row0 + C].norm())
+    for k in (_lib.KS_IT, _lib.KS_ITTOT, _lib.KS_OUTER):
+        b.scal[inst * _lib.KS_NSCAL + k] = 0.
+    ref = _eight_launch_iterations(b, inst, 64)  # up to 6000 iterations here
+    assert sol.stats["iterations"] <= 1.15 * ref + 3, (sol.stats, ref)
