@@ -12,6 +12,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <new>
 #include <vector>
 
 #include "mfv_common.hpp"
@@ -385,11 +386,9 @@ extern "C" void mfv_stencil_tiles_host_free(mfv_stencil_tiles_host *t)
     memset(t, 0, sizeof(*t));
 }
 
-extern "C" int mfv_stencil_tiles_build(int C, int K, const int32_t *lsq_cells, const int32_t *lsq_ncells,
-                                       const int64_t *perm, int T, mfv_stencil_tiles_host *out)
+static int stencil_tiles(int C, int K, const int32_t *lsq_cells, const int32_t *lsq_ncells, const int64_t *perm, int T,
+                         mfv_stencil_tiles_host *out)
 {
-    MFV_REQUIRE(out, "out is NULL");
-    memset(out, 0, sizeof(*out));
     MFV_REQUIRE(C > 0 && K > 0 && T > 0, "bad sizes C=%d K=%d T=%d", C, K, T);
     MFV_REQUIRE(lsq_cells && lsq_ncells && perm, "NULL array");
     const int nt = (C + T - 1) / T, K2 = (K + 1) / 2;
@@ -446,4 +445,17 @@ extern "C" int mfv_stencil_tiles_build(int C, int K, const int32_t *lsq_cells, c
         return MFV_ENOMEM;
     }
     return MFV_OK;
+}
+
+extern "C" int mfv_stencil_tiles_build(int C, int K, const int32_t *lsq_cells, const int32_t *lsq_ncells,
+                                       const int64_t *perm, int T, mfv_stencil_tiles_host *out)
+{
+    MFV_REQUIRE(out, "out is NULL");
+    memset(out, 0, sizeof(*out));
+    try {
+        return stencil_tiles(C, K, lsq_cells, lsq_ncells, perm, T, out);
+    } catch (const std::bad_alloc &) {  // no exception crosses the ABI; the gradients then gather
+        mfv::set_error("stencil tiles: host allocation failed");
+        return MFV_ENOMEM;
+    }
 }

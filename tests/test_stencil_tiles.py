@@ -87,3 +87,14 @@ def test_stencils_too_wide_for_a_tile_are_gathered(monkeypatch):
     assert DeviceMesh.stencil_tiles(mesh) is None
     assert DeviceMesh.stencil_tiles(mesh) is None  # and does not build them again
     assert mesh._stencil_tiles is False
+
+
+def test_a_failed_allocation_is_an_error_code():
+    """A table larger than the address space: the entry point answers with a code, no exception leaves it."""
+    from manapy_amd import _lib
+    h = _lib.MfvStencilTilesHost()
+    one, perm = np.zeros(1, dtype=np.int32), np.zeros(1, dtype=np.int64)
+    with pytest.raises(_lib.MfvError, match="allocation failed"):
+        _lib.call("mfv_stencil_tiles_build", 1, 2 ** 31 - 2, one.ctypes.data, one.ctypes.data, perm.ctypes.data, 1 << 20,
+                  ctypes.byref(h))
+    assert not h.pairs and not h.cell
