@@ -837,7 +837,9 @@ void give_dt_slot(double *p)
 // promises. kDt looks at the pinned word instead, which the fold stores last and with release order:
 // whoever sees it also sees dt_dev and what the stream held before it, but the kernel itself may not have
 // retired. Four 3D advection steps take 328 us with kIdle and 306 us with kDt, four of the SRNH scheme at
-// 1k cells (eight dts) 338 and 278 us, of Euler at 8k 138 and 120, of advection-diffusion 332 and 240.
+// 1k cells (eight dts) 338 and 278 us, of Euler at 8k 138 and 120, of advection-diffusion 332 and 240. The
+// release order itself costs 0.35 us a dt (12.3 -> 12.6 us a call at 1k cells); a write-through store and a
+// wait for it in its place the same.
 int mfv::dt_total(const double *part, size_t n, double *dt_dev, double *dt_host, DtWait wait, hipStream_t st)
 {
     double *slot = nullptr;

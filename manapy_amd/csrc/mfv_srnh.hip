@@ -93,8 +93,8 @@ __device__ __forceinline__ void srnh_flux(double hu_l, double hu_r, double hv_l,
 }
 
 // explicitscheme_convective_SW (shallowater/fvm_utils.py:344-496), one cell per thread. 200k
-// cells at order 2: 21.8 us, and 65 us with the cubic's acos, cos and pow; bound by the latency of
-// its face and cell gathers now, by its arithmetic before.
+// cells at order 2: 21.8 us, and 65 us with the cubic's acos, cos and pow; bound by what it gathers
+// now (110 MB past the L2s at 5.2 TB/s, a copy's rate; vector issue 0.42), by its arithmetic before.
 __global__ void __launch_bounds__(kBlock) k_srnh_convective(Mesh m, Out5 rez, Fields5 cell, Fields5 ghost,
                                                             const double *__restrict__ h_x,
                                                             const double *__restrict__ h_y,
@@ -259,9 +259,10 @@ __global__ void __launch_bounds__(kBlock) k_update_sw5(int C, Out5 st, Fields5 r
 }
 
 // ----- steps in a row --------------------------------------------------------------------------
-// What the sequence of entry points does per step in a face pass and a cell pass. The flux is bound by
-// its arithmetic (nine divisions and three roots a face), so every face is evaluated once, where the
-// cell-centric residual evaluates inner faces twice; the cell pass then adds the three fluxes in the
+// What the sequence of entry points does per step in a face pass and a cell pass. Every face is evaluated
+// once (nine divisions and three roots) and gathered for once, where the cell-centric residual does
+// both twice for inner faces: 51 MB past the L2s in the face pass, at the 5.2 TB/s of a copy, for the
+// residual's 110; the cell pass moves 84 MB at 4.8. The cell pass then adds the three fluxes in the
 // residual's order, forms the source term, updates into a second set of fields (its neighbours still
 // read this one) and takes the next time step's candidate, which otherwise are a launch and a trip
 // of ten arrays each. 200k cells, second order: 9.9 + 18.1 us a step for 21.4 + 11.2 + 7.4 + 8.7 us of the four
